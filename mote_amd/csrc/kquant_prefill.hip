@@ -1,0 +1,721 @@
+// K-quant linear over many tokens on the matrix cores, y[M, N] = x[M, K] (f16)
+// . W[N, K]^T with Q4_K or Q6_K weights (layouts in kquant.hip).
+//
+// A workgroup of 4 KG waves computes a 32 TM x 128 tile of y over one part of
+// K.  Wave (kg, wn) owns 32 weight rows (columns 32 wn .. of the tile) for
+// group kg's share of the part's super-blocks, TM tiles of
+// v_mfma_f32_32x32x16_f16 with the activations as the A operand.  Lane (r, c)
+// (r = lane % 32, c = lane / 32) supplies weight row r and, in the slice
+// (h, u) of quarter p of a super-block, its elements
+//   64 p + 32 h + 16 c + 8 u .. + 7,
+// so a lane's quants of a quarter are contiguous bytes: it loads them itself,
+// global memory to registers, and re-uses the registers for the same quarter
+// of the next super-block as soon as they are decoded (about three quarters
+// ahead of their use; no LDS traffic for the weights).
+//
+// Weight operands are exact binary16 integers, as in the few-token tiles of
+// kquant.hip: Q4_K sc q (at most 63 x 15), one packed fma from 1024 + q or 64 +
+// q; Q6_K sc (q - 32) = 8 s (q - 32) + t (q - 32) with s = sc >> 3, t = sc & 7,
+// two operands (q - 32) s and (q - 32) t / 8 into the same accumulator.  Every
+// product with an activation is exact in f32; once per super-block
+//   Q4_K: y += d C - dmin C',  C' = sum_j m_j S_j (two MFMA operands: S_j, the
+//         activations' sum over sub-block j, as binary16 hi + lo, against m_j)
+//   Q6_K: y += 8 d C.
+// So the decode costs 10 (Q4_K) or 20 (Q6_K) vector instructions per 8
+// weights and TM MFMAs (2 TM for Q6_K), and the per-super-block fold 16 TM.
+//
+// Activations: direct-to-LDS 16-byte loads, 64 k of every group per interval,
+// four slots (three intervals in flight while one is multiplied), 128-byte rows
+// with the 16-byte chunks XOR-swizzled by half the row: the 16 rows that an
+// operand read covers per cycle fall on the 64 banks once (swizzled by the row,
+// every read took 8 cycles instead of 4).  One barrier per interval, before its last slice:
+// the slice's MFMAs cover the first LDS reads and decode of the next interval.
+// The groups' partial tiles meet in LDS (fixed order); K parts, used where the
+// tiles are too few for the chip, meet in scratch planes that
+// kq_parts_reduce_kernel adds in part order.
+//
+// A result that is not finite is recomputed element by element with GGML's
+// values, as in the few-token tiles.
+//
+// Measured on MI355X (weights of three calls rotated): 512 x 4096 x 14 336 Q4_K
+// 84 us (716 TFLOP/s), where the four-token passes of the LDS-ring GEMV, which
+// read every weight M / 4 times, took 1723; 256 x 14 336 x 4096 Q6_K 62 us
+// against 1203.  Bound by the interval's instruction stream: MFMAs fill 37 % of
+// the cycles, vector instructions and the LDS (A operands read once per wave)
+// a third each, imperfectly overlapped at two waves per SIMD.  128 x 256 tiles
+// of four waves with 512 registers (half the A reads per MFMA) measured level
+// (84 us); 64-row tiles 20 - 35 % slower per row.
+#include "kquant_blocks.hpp"
+#include "q4_0.hpp"
+
+#include <cmath>
+#include <type_traits>
+
+namespace mote::kquant {
+namespace {
+
+typedef __attribute__((address_space(3))) void* lds_ptr_t;
+// 16-byte vector at a 2-byte-aligned address (one unaligned dwordx4 load).
+typedef uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
+
+constexpr int kTileWaves = 4;                 // waves along N
+
+constexpr int vm_wait(int n) { return (n & 0xF) | ((n >> 4) << 14) | 0x0F70; }
+constexpr int kLgkmWait = 0xC07F;  // lgkmcnt(0) alone; ANDed with vm_wait(n): both
+
+// The builtins behind plain functions (usable from generic lambdas).
+typedef __amdgpu_buffer_rsrc_t Buffer;
+__device__ __forceinline__ Buffer buffer_at(const void* base) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, 0xFFFFFFFFu, 0x00020000);
+}
+__device__ __forceinline__ void load_lds16(Buffer src, uint32_t lane_offset, uint32_t offset, uint8_t* dst) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (lds_ptr_t)dst, 16, lane_offset, offset, 0, 0);
+}
+template <int I>
+__device__ __forceinline__ void wait_counts() { __builtin_amdgcn_s_waitcnt(I); }
+__device__ __forceinline__ void order_fence() { __builtin_amdgcn_sched_barrier(0); }
+// Keeps memory operations on their side of this point, in the compiler's
+// intermediate code and in its schedule: the counted waits below rely on the
+// order in which the loads are issued.
+__device__ __forceinline__ void issue_fence() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+}
+__device__ __forceinline__ void group_barrier() { __builtin_amdgcn_s_barrier(); }
+__device__ __forceinline__ f32x16 mfma32(const f16x8& a, const f16x8& b, const f32x16& c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ uint32_t perm(uint32_t hi, uint32_t lo, uint32_t sel) {
+    return __builtin_amdgcn_perm(hi, lo, sel);
+}
+__device__ __forceinline__ f16x2 both(f16x2 v, bool high) {
+    const uint32_t b = __builtin_bit_cast(uint32_t, v);
+    return as_h2(perm(b, b, high ? 0x03020302u : 0x01000100u));
+}
+__device__ __forceinline__ f16x2 both(_Float16 v) { return f16x2{v, v}; }
+__device__ __forceinline__ f16x8 join(f16x2 a, f16x2 b, f16x2 c, f16x2 d) {
+    return f16x8{a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y};
+}
+
+// Keeps a converted scale in f32: as mixed-precision fmas from the binary16
+// word, two of which in a row need a wait state, the folds took twice as long.
+__device__ __forceinline__ float as_f32(float v) {
+    asm("" : "+v"(v));
+    return v;
+}
+
+// A lane's quants of one super-block and the words its scales come from.
+template <Fmt F>
+struct Raw;
+template <>
+struct Raw<Fmt::Q4K> {
+    u32x4 qs[4];  // bytes 16 c .. 16 c + 15 of quarter p's 32
+    u32x4 head;   // d, dmin, scales
+};
+template <>
+struct Raw<Fmt::Q6K> {
+    u32x4 la[2], lb[2], qh[2];  // per half block: ql bytes 16 c.. of its two 32-byte runs, qh bytes 16 c..
+    u32x4 sc;
+    uint32_t d;
+};
+
+// The scales of the super-block being multiplied.
+template <Fmt F>
+struct Scales;
+template <>
+struct Scales<Fmt::Q4K> {
+    uint32_t sc[2];  // sc_0..3, sc_4..7, a byte each
+    uint32_t m[2];   // m_0..3, m_4..7
+    float d, dmin;
+};
+template <>
+struct Scales<Fmt::Q6K> {
+    uint32_t sc[4];  // quarter p: its scales at bytes 0 (h = 0) and 2 (h = 1)
+    float d;
+};
+
+template <Fmt F, int TM, int TN, int KG, bool SK, typename OutT>
+__global__ __launch_bounds__(64 * kTileWaves * KG) void kq_prefill_kernel(
+    const uint16_t* __restrict__ x, const uint8_t* __restrict__ w, const uint16_t* __restrict__ sums,
+    OutT* __restrict__ y, float* __restrict__ partial, uint32_t M, uint32_t N, uint32_t K, uint32_t m_tiles,
+    uint32_t n_tiles, uint32_t part_blocks, uint32_t total, uint32_t per_xcd) {
+    constexpr int BM = 32 * TM;
+    constexpr uint32_t BN = 32 * TN * kTileWaves;
+    constexpr int kUnit = BM * 128;            // LDS bytes of one group's activations of an interval
+    constexpr int kSlots = 4;                  // interval t, a quarter p = t % 4 of a super-block: slot p
+    constexpr int NA = BM / (8 * kTileWaves);  // activation loads per wave and interval
+    constexpr int NB = F == Fmt::Q6K ? 2 : 1;  // operands per 8 weights
+    constexpr uint32_t BB = block_bytes<F>();
+    static_assert((KG == 1 || KG == 2) && TM % KG == 0, "the groups share the output tiles evenly");
+    constexpr int kRing = kSlots * KG * kUnit;
+    constexpr int kReduce = KG == 1 ? 0 : kTileWaves * KG * (TM / 2) * TN * 4096;
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[kRing > kReduce ? kRing : kReduce];
+
+    const uint32_t logical = (blockIdx.x % 8u) * per_xcd + blockIdx.x / 8u;
+    if (logical >= total) return;
+    const uint32_t tile_m = logical % m_tiles, rest = logical / m_tiles;
+    const uint32_t tile_n = rest % n_tiles, part = rest / n_tiles;
+    const uint32_t m0 = tile_m * BM, n0 = tile_n * BN;
+    const uint32_t nb = K / kSuper;
+    const uint32_t pb0 = part * part_blocks, pb1 = min(pb0 + part_blocks, nb);
+
+    const int lane = static_cast<int>(threadIdx.x) & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+    const int kg = wave / kTileWaves, wn = wave % kTileWaves;
+    const int lr = lane & 31, lc = lane >> 5;
+    // this group's super-blocks: [b0, b0 + ns)
+    const uint32_t per = (pb1 - pb0 + KG - 1) / KG;
+    const uint32_t b0 = min(pb0 + static_cast<uint32_t>(kg) * per, pb1);
+    const uint32_t ns = min(per, pb1 - b0);
+
+    // Activation load i of a wave covers 8 rows; position p of row r holds the
+    // chunk (8 elements) of slice position q = p ^ (r / 2) % 8, chunk 4 h + 2 c
+    // + u for q = 4 c + 2 h + u.
+    const uint8_t* xb = reinterpret_cast<const uint8_t*>(x) + (static_cast<size_t>(m0) * K + b0 * kSuper) * 2;
+    uint32_t aoff[NA];
+#pragma unroll
+    for (int i = 0; i < NA; ++i) {
+        const uint32_t row = (wn * NA + i) * 8 + (lane >> 3);
+        const uint32_t q = (lane & 7) ^ ((row >> 1) & 7);
+        aoff[i] = (min(m0 + row, M - 1) - m0) * (K * 2) + (4 * ((q >> 1) & 1) + 2 * (q >> 2) + (q & 1)) * 16;
+    }
+    const Buffer xsrc = buffer_at(xb);
+    uint8_t* const unit = lds + kg * kUnit;
+    const uint32_t last = ns * 4 - 1;
+    auto load_a = [&](uint32_t t, uint32_t slot) {  // interval t (clamped) of this group
+        const uint32_t o = min(t, last) * 128u;
+#pragma unroll
+        for (int i = 0; i < NA; ++i)
+            load_lds16(xsrc, aoff[i], o, unit + slot * (KG * kUnit) + (wn * NA + i) * 1024);
+    };
+    // Weights: row r of each of this wave's TN column tiles (clamped), from
+    // super-block b0 on.
+    const uint8_t* wrow[TN];
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+        wrow[j] = w + (static_cast<size_t>(min(n0 + (wn * TN + j) * 32 + lr, N - 1)) * nb + b0) * BB;
+    Raw<F> raw[TN];
+    // The quants freed by quarter p, of super-block s (clamped): quarter p's
+    // (Q4_K), half p / 2's after its second quarter (Q6_K).
+    auto load_quants = [&](auto pc, uint32_t s) {
+        constexpr int P = decltype(pc)::value;
+        const size_t at = static_cast<size_t>(min(s, ns - 1)) * BB;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            const uint8_t* blk = wrow[j] + at;
+            if constexpr (F == Fmt::Q4K) {
+                raw[j].qs[P] = *reinterpret_cast<const u32x4*>(blk + 16 + 32 * P + 16 * lc);
+            } else if constexpr (P % 2 == 1) {
+                constexpr int g = P / 2;
+                raw[j].la[g] = *reinterpret_cast<const u32x4_a2*>(blk + 64 * g + 16 * lc);
+                raw[j].lb[g] = *reinterpret_cast<const u32x4_a2*>(blk + 64 * g + 32 + 16 * lc);
+                raw[j].qh[g] = *reinterpret_cast<const u32x4_a2*>(blk + 128 + 32 * g + 16 * lc);
+            }
+        }
+    };
+    auto load_head = [&](uint32_t s) {
+        const size_t at = static_cast<size_t>(min(s, ns - 1)) * BB;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            const uint8_t* blk = wrow[j] + at;
+            if constexpr (F == Fmt::Q4K) {
+                raw[j].head = *reinterpret_cast<const u32x4*>(blk);
+            } else {
+                raw[j].sc = *reinterpret_cast<const u32x4_a2*>(blk + 192);
+                raw[j].d = *reinterpret_cast<const uint16_t*>(blk + 208);
+            }
+        }
+    };
+    Scales<F> sl[TN];
+    float d_fold[TN] = {};  // the scale of the block sums not yet folded
+    auto unpack_head = [&]() {
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            if constexpr (F == Fmt::Q4K) {
+                const u32x4 head = raw[j].head;
+                sl[j].sc[0] = head.y & 0x3F3F3F3Fu;
+                sl[j].sc[1] = (head.w & 0x0F0F0F0Fu) | ((head.y >> 2) & 0x30303030u);
+                sl[j].m[0] = head.z & 0x3F3F3F3Fu;
+                sl[j].m[1] = ((head.w >> 4) & 0x0F0F0F0Fu) | ((head.z >> 2) & 0x30303030u);
+                sl[j].d = as_f32(half_lo_to_float(head.x));
+                sl[j].dmin = as_f32(half_hi_to_float(head.x));
+            } else {
+                const uint32_t s[4] = {raw[j].sc.x, raw[j].sc.y, raw[j].sc.z, raw[j].sc.w};
+#pragma unroll
+                for (int p = 0; p < 4; ++p) sl[j].sc[p] = s[p] >> (8 * lc);
+                sl[j].d = as_f32(8.0f * half_bits_to_float(raw[j].d));
+            }
+        }
+    };
+    // The binary16 factors of a quarter's two sub-blocks (h = 0, 1).
+    f16x2 mul[TN][2][NB], add[TN][2][NB];
+    auto quarter_scales = [&](auto pc) {
+        constexpr int P = decltype(pc)::value;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            if constexpr (F == Fmt::Q4K) {
+                const uint32_t word = sl[j].sc[P / 2];
+                const f16x2 sc = as_h2(perm(0x64646464u, word, P % 2 ? 0x04030402u : 0x04010400u)) +
+                                 both(static_cast<_Float16>(-1024.0f));
+                mul[j][0][0] = both(sc, false);
+                mul[j][1][0] = both(sc, true);
+                add[j][0][0] = mul[j][0][0] * both(static_cast<_Float16>(-1024.0f));
+                add[j][1][0] = mul[j][1][0] * both(static_cast<_Float16>(-64.0f));
+            } else {
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const int sc = static_cast<int8_t>((sl[j].sc[P] >> (16 * h)) & 0xFFu);
+                    const _Float16 s = static_cast<_Float16>(static_cast<short>(sc >> 3));
+                    const _Float16 t =
+                        static_cast<_Float16>(static_cast<short>(sc & 7)) * static_cast<_Float16>(0.125f);
+                    mul[j][h][0] = both(s);
+                    mul[j][h][NB - 1] = both(t);
+                    add[j][h][0] = both(static_cast<_Float16>(s * static_cast<_Float16>(-1056.0f)));
+                    add[j][h][NB - 1] = both(static_cast<_Float16>(t * static_cast<_Float16>(-1056.0f)));
+                }
+            }
+        }
+    };
+    // The operands of slice (h, u) of quarter p.
+    f16x8 b[2][TN][NB];
+    auto decode = [&](auto pc, auto uc, f16x8 (&dst)[TN][NB]) {
+        constexpr int P = decltype(pc)::value, U = decltype(uc)::value, h = U / 2, u = U % 2;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            uint32_t q[2];
+            if constexpr (F == Fmt::Q4K) {
+                constexpr uint32_t mask = h ? 0xF0F0F0F0u : 0x0F0F0F0Fu, e = h ? 0x54545454u : 0x64646464u;
+                q[0] = (u ? raw[j].qs[P].z : raw[j].qs[P].x) & mask;
+                q[1] = (u ? raw[j].qs[P].w : raw[j].qs[P].y) & mask;
+                const f16x2 m = mul[j][h][0], a = add[j][h][0];
+                dst[j][0] = join(__builtin_elementwise_fma(as_h2(perm(e, q[0], 0x04010400u)), m, a),
+                                 __builtin_elementwise_fma(as_h2(perm(e, q[0], 0x04030402u)), m, a),
+                                 __builtin_elementwise_fma(as_h2(perm(e, q[1], 0x04010400u)), m, a),
+                                 __builtin_elementwise_fma(as_h2(perm(e, q[1], 0x04030402u)), m, a));
+            } else {
+                // quarter c4 of half g: nibble c4 / 2 of run c4 % 2
+                constexpr int g = P / 2, c4 = 2 * (P % 2) + h;
+                const u32x4 l = c4 % 2 ? raw[j].lb[g] : raw[j].la[g];
+                const uint32_t lw[2] = {u ? l.z : l.x, u ? l.w : l.y};
+                const uint32_t hw[2] = {u ? raw[j].qh[g].z : raw[j].qh[g].x, u ? raw[j].qh[g].w : raw[j].qh[g].y};
+                f16x2 v[4];
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    const uint32_t low = (c4 < 2 ? lw[i] : lw[i] >> 4) & 0x0F0F0F0Fu;
+                    const uint32_t top = c4 == 0 ? hw[i] << 4 : c4 == 1 ? hw[i] << 2 : c4 == 2 ? hw[i] : hw[i] >> 2;
+                    q[i] = (top & 0x30303030u) | low;
+                    v[2 * i] = as_h2(perm(0x64646464u, q[i], 0x04010400u));
+                    v[2 * i + 1] = as_h2(perm(0x64646464u, q[i], 0x04030402u));
+                }
+#pragma unroll
+                for (int k = 0; k < NB; ++k)
+                    dst[j][k] = join(__builtin_elementwise_fma(v[0], mul[j][h][k], add[j][h][k]),
+                                     __builtin_elementwise_fma(v[1], mul[j][h][k], add[j][h][k]),
+                                     __builtin_elementwise_fma(v[2], mul[j][h][k], add[j][h][k]),
+                                     __builtin_elementwise_fma(v[3], mul[j][h][k], add[j][h][k]));
+            }
+        }
+    };
+
+    f32x16 acc[TM][TN], blk[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = blk[i][j][r] = 0.0f;
+    const f32x16 zero = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    f16x8 a[2][TM];
+    const uint32_t a_row = lr * 128, a_x = (lr >> 1) & 7;
+    auto read_a = [&](uint32_t slot, int u, f16x8 (&dst)[TM]) {
+        const uint8_t* base = unit + slot * (KG * kUnit) + a_row + (((4 * lc + u) ^ a_x) * 16);
+#pragma unroll
+        for (int i = 0; i < TM; ++i) dst[i] = *reinterpret_cast<const f16x8*>(base + i * 4096);
+    };
+    auto multiply = [&](auto cc) {
+        constexpr int C = decltype(cc)::value;
+#pragma unroll
+        for (int k = 0; k < NB; ++k)
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) blk[i][j] = mfma32(a[C][i], b[C][j][k], blk[i][j]);
+    };
+    // The first slice of a super-block: the sums of the one before join the
+    // result, tile by tile ahead of the tile's first product.
+    auto fold = [&](int i, int j) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][j][r] = __builtin_fmaf(d_fold[j], blk[i][j][r], acc[i][j][r]);
+    };
+    auto multiply_first = [&]() {
+#pragma unroll
+        for (int k = 0; k < NB; ++k)
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    if (k == 0) fold(i, j);
+                    blk[i][j] = mfma32(a[0][i], b[0][j][k], k == 0 ? zero : blk[i][j]);
+                }
+    };
+    // Q4_K's minimum term of the super-block, one tile per slice of its second
+    // half: token row r of tile i holds the eight hi (c = 0) or lo (c = 1)
+    // halves of the sub-block sums.
+    f16x8 sx[TM];
+    auto load_sums = [&](uint32_t s) {
+        if constexpr (F == Fmt::Q4K) {
+            const uint16_t* src = sums + static_cast<size_t>(b0 + s) * 16 + 8 * lc;
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+                sx[i] = *reinterpret_cast<const f16x8*>(src + static_cast<size_t>(min(m0 + i * 32 + lr, M - 1)) * nb * 16);
+        }
+    };
+    auto mins = [&](int j) {
+        if constexpr (F == Fmt::Q4K) {
+            const f16x2 b = both(static_cast<_Float16>(-1024.0f));
+            const uint32_t e = 0x64646464u, lo = sl[j].m[0], hi = sl[j].m[1];
+            return join(as_h2(perm(e, lo, 0x04010400u)) + b, as_h2(perm(e, lo, 0x04030402u)) + b,
+                        as_h2(perm(e, hi, 0x04010400u)) + b, as_h2(perm(e, hi, 0x04030402u)) + b);
+        }
+    };
+    auto minimum = [&](auto pc, auto ic, auto slice) {
+        constexpr int I = 4 * (decltype(pc)::value - 2) + decltype(ic)::value;
+        if constexpr (F == Fmt::Q4K) {
+            if constexpr (I >= 0 && I < TM) {
+                f32x16 mn[TN];
+#pragma unroll
+                for (int j = 0; j < TN; ++j) mn[j] = mfma32(sx[I], mins(j), zero);
+                slice();
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) acc[I][j][r] = __builtin_fmaf(-sl[j].dmin, mn[j][r], acc[I][j][r]);
+            } else {
+                slice();
+            }
+        } else {
+            slice();
+        }
+    };
+    // Loads a wave issues behind interval t's activations of four intervals on:
+    // quants, the sums (p = 0), the next header (p = 2).
+    constexpr int kBehind[4] = {F == Fmt::Q4K ? TN + TM : 0, F == Fmt::Q4K ? TN : 3 * TN, F == Fmt::Q4K ? 2 * TN : 2 * TN,
+                                F == Fmt::Q4K ? TN : 3 * TN};
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+    using I2 = std::integral_constant<int, 2>;
+    using I3 = std::integral_constant<int, 3>;
+
+    if (ns > 0) {  // uniform over the wave; groups without work only meet the barriers
+        load_a(0, 0);
+        issue_fence();
+        load_quants(I0{}, 0);
+        issue_fence();
+        load_a(1, 1);
+        issue_fence();
+        load_quants(I1{}, 0);
+        issue_fence();
+        load_a(2, 2);
+        issue_fence();
+        load_quants(I2{}, 0);
+        load_head(0);
+        issue_fence();
+        load_a(3, 3);
+        issue_fence();
+        load_quants(I3{}, 0);
+        issue_fence();
+        wait_counts<vm_wait(3 * NA + (F == Fmt::Q4K ? 5 : 8) * TN)>();  // interval 0's activations
+    }
+    group_barrier();
+    order_fence();
+    if (ns > 0) {
+        read_a(0, 0, a[0]);
+        unpack_head();
+        quarter_scales(I0{});
+        decode(I0{}, I0{}, b[0]);
+        order_fence();
+        // One interval: quarter p of super-block s.
+        auto interval = [&](auto pc, uint32_t s) {
+            constexpr int P = decltype(pc)::value;
+            using PN = std::integral_constant<int, (P + 1) & 3>;
+            read_a(P, 1, a[1]);
+            minimum(pc, I0{}, [&] {
+                if constexpr (P == 0) multiply_first(); else multiply(I0{});
+                decode(pc, I1{}, b[1]);
+            });
+            order_fence();
+            read_a(P, 2, a[0]);
+            minimum(pc, I1{}, [&] {
+                multiply(I1{});
+                decode(pc, I2{}, b[0]);
+            });
+            order_fence();
+            read_a(P, 3, a[1]);
+            minimum(pc, I2{}, [&] {
+                multiply(I0{});
+                decode(pc, I3{}, b[1]);
+            });
+            issue_fence();
+            // The next interval's activations have landed (what may be
+            // outstanding is all younger), and every wave has read this one's.
+            wait_counts<vm_wait(2 * NA + kBehind[(P + 1) & 3] + kBehind[(P + 2) & 3] + kBehind[(P + 3) & 3]) &
+                        kLgkmWait>();
+            group_barrier();
+            order_fence();
+            read_a((P + 1) & 3, 0, a[0]);
+            load_a(4 * s + P + 4, P);
+            issue_fence();
+            load_quants(pc, s + 1);
+            if constexpr (P == 2) load_head(s + 1);
+            if constexpr (P == 0) load_sums(s);
+            issue_fence();
+            minimum(pc, I3{}, [&] {
+                multiply(I1{});
+                if constexpr (P == 3) {
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) d_fold[j] = sl[j].d;
+                    unpack_head();
+                }
+                quarter_scales(PN{});
+                decode(PN{}, I0{}, b[0]);
+            });
+            order_fence();
+        };
+        for (uint32_t s = 0; s < ns; ++s) {
+            interval(I0{}, s);
+            interval(I1{}, s);
+            interval(I2{}, s);
+            interval(I3{}, s);
+        }
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) fold(i, j);
+    }
+    for (uint32_t t = ns * 4; t < per * 4; ++t) group_barrier();
+    wait_counts<vm_wait(0)>();
+    __syncthreads();
+
+    // Two groups: each keeps half of the tiles and hands the other half over.
+    int tile0 = 0;
+    if constexpr (KG == 2) {
+        constexpr int H = TM / 2;
+        float* red = reinterpret_cast<float*>(lds);
+        auto slot = [&](int wv, int i, int j, int r) { return red + (((wv * H + i) * TN + j) * 4 + r) * 256 + lane * 4; };
+        auto give = [&](const f32x16& v, int i, int j) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                *reinterpret_cast<f32x4*>(slot(wave, i, j, r)) = f32x4{v[4 * r], v[4 * r + 1], v[4 * r + 2], v[4 * r + 3]};
+        };
+        if (kg == 0) {
+#pragma unroll
+            for (int i = 0; i < H; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) give(acc[H + i][j], i, j);
+        } else {
+#pragma unroll
+            for (int i = 0; i < H; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    give(acc[i][j], i, j);
+                    acc[i][j] = acc[H + i][j];
+                }
+        }
+        __syncthreads();
+        const int other = wave ^ kTileWaves;
+#pragma unroll
+        for (int i = 0; i < H; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const f32x4 v = *reinterpret_cast<const f32x4*>(slot(other, i, j, r));
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) acc[i][j][4 * r + k] += v[k];
+                }
+        tile0 = kg * H;
+    }
+    // Lane (r, c) holds column r of each tile, rows 8 (k / 4) + 4 c + k % 4.
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+        const uint32_t n = n0 + (wn * TN + j) * 32 + lr;
+        if (n >= N) continue;
+#pragma unroll
+        for (int i = 0; i < TM / KG; ++i) {
+#pragma unroll
+            for (int k = 0; k < 16; ++k) {
+                const uint32_t m = m0 + (tile0 + i) * 32 + 8 * (k / 4) + 4 * lc + k % 4;
+                if (m >= M) continue;
+                float v = acc[i][j][k];
+                if (__builtin_expect(not_finite(v), 0))
+                    v = kq_exact_thread<F>(w + (static_cast<size_t>(n) * nb + pb0) * BB,
+                                           x + static_cast<size_t>(m) * K + static_cast<size_t>(pb0) * kSuper, pb1 - pb0);
+                if constexpr (SK)
+                    partial[(static_cast<size_t>(part) * M + m) * N + n] = v;
+                else
+                    y[static_cast<size_t>(m) * N + n] = to_out<OutT>(v);
+            }
+        }
+    }
+}
+
+// sums[m][b][0..7] and [8..15]: the binary16 hi and lo halves of the sums of
+// token m's activations over the eight sub-blocks of super-block b.  One thread
+// per sub-block.
+__global__ __launch_bounds__(256) void kq_sums_kernel(const uint16_t* __restrict__ x, uint16_t* __restrict__ sums,
+                                                      uint64_t count) {
+    const uint64_t i = static_cast<uint64_t>(blockIdx.x) * 256 + threadIdx.x;
+    if (i >= count) return;
+    const u32x4* src = reinterpret_cast<const u32x4*>(x + i * 32);
+    const uint32_t one = 0x3C003C00u;
+    float s = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const u32x4 v = src[k];
+        s = dot2(v.w, one, dot2(v.z, one, dot2(v.y, one, dot2(v.x, one, s))));
+    }
+    const _Float16 hi = static_cast<_Float16>(s);
+    const _Float16 lo = static_cast<_Float16>(s - static_cast<float>(hi));
+    uint16_t* dst = sums + (i / 8) * 16 + i % 8;
+    dst[0] = __builtin_bit_cast(uint16_t, hi);
+    dst[8] = __builtin_bit_cast(uint16_t, lo);
+}
+
+// y[i] = the sum of the K parts' planes at i, in part order, converted.
+template <typename OutT>
+__global__ __launch_bounds__(256) void kq_parts_reduce_kernel(const float* __restrict__ partial, uint32_t parts,
+                                                              uint64_t count, OutT* __restrict__ y) {
+    const uint64_t i = static_cast<uint64_t>(blockIdx.x) * 256 + threadIdx.x;
+    if (i >= count) return;
+    float v = partial[i];
+    for (uint32_t k = 1; k < parts; ++k) v += partial[k * count + i];
+    y[i] = to_out<OutT>(v);
+}
+
+template <Fmt F, int TM, int TN, int KG, typename OutT>
+hipError_t launch_tile(const uint16_t* x, const uint8_t* w, OutT* y, uint32_t M, uint32_t N, uint32_t K,
+                       uint32_t parts, hipStream_t stream) {
+    const uint32_t nb = K / kSuper;
+    const uint32_t m_tiles = (M + 32 * TM - 1) / (32 * TM), n_tiles = (N + 32 * TN * kTileWaves - 1) / (32 * TN * kTileWaves);
+    const uint32_t part_blocks = (nb + parts - 1) / parts;
+    parts = (nb + part_blocks - 1) / part_blocks;
+    const uint64_t total64 = static_cast<uint64_t>(m_tiles) * n_tiles * parts;
+    if (total64 > 0x7ffffff0ull) return hipErrorInvalidConfiguration;
+    const uint32_t total = static_cast<uint32_t>(total64), per_xcd = (total + 7) / 8;
+    // Scratch: the arrival counters every user of the pool leaves in place, the
+    // parts' planes, the activation sums.
+    const uint64_t count = static_cast<uint64_t>(M) * N;
+    const uint64_t plane_bytes = parts > 1 ? (count * parts * sizeof(float) + 15) / 16 * 16 : 0;
+    const uint64_t sum_bytes = F == Fmt::Q4K ? static_cast<uint64_t>(M) * nb * 32 : 0;
+    q4_0::ScratchPool::Lease lease;
+    float* partial = nullptr;
+    uint16_t* sums = nullptr;
+    if (plane_bytes + sum_bytes > 0) {
+        const hipError_t e = q4_0::acquire_scratch(stream, q4_0::kSplitKCounterBytes + plane_bytes + sum_bytes, &lease);
+        if (e != hipSuccess) return e;
+        auto* base = static_cast<uint8_t*>(lease.ptr());
+        if (lease.fresh()) {
+            const hipError_t z =
+                q4_0::launch_zero_fill(base, q4_0::kSplitKCounterBytes / 4, q4_0::OutType::F32, stream);
+            if (z != hipSuccess) return z;
+        }
+        partial = reinterpret_cast<float*>(base + q4_0::kSplitKCounterBytes);
+        sums = reinterpret_cast<uint16_t*>(base + q4_0::kSplitKCounterBytes + plane_bytes);
+    }
+    if constexpr (F == Fmt::Q4K) {
+        const uint64_t subs = static_cast<uint64_t>(M) * nb * 8;
+        hipLaunchKernelGGL(kq_sums_kernel, dim3(static_cast<uint32_t>((subs + 255) / 256)), dim3(256), 0, stream, x,
+                           sums, subs);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    const dim3 grid(per_xcd * 8), block(64 * kTileWaves * KG);
+    if (parts == 1) {
+        hipLaunchKernelGGL((kq_prefill_kernel<F, TM, TN, KG, false, OutT>), grid, block, 0, stream, x, w, sums, y, partial, M,
+                           N, K, m_tiles, n_tiles, part_blocks, total, per_xcd);
+        return hipGetLastError();
+    }
+    hipLaunchKernelGGL((kq_prefill_kernel<F, TM, TN, KG, true, float>), grid, block, 0, stream, x, w, sums,
+                       static_cast<float*>(nullptr), partial, M, N, K, m_tiles, n_tiles, part_blocks, total, per_xcd);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL((kq_parts_reduce_kernel<OutT>), dim3(static_cast<uint32_t>((count + 255) / 256)), dim3(256), 0,
+                       stream, partial, parts, count, y);
+    return hipGetLastError();
+}
+
+// Which tile and how many K parts: the least of
+//   rounds x (start + blocks x block time) + reduction,
+// rounds of one workgroup per CU, blocks the super-blocks of a part, the
+// reduction 3 us and the planes written and read once at 4 TB/s.  The start, 5
+// us, and the block times in us are fits to MI355X timings, within 10 % at the
+// shapes fitted (measured against predicted, us): Q4_K 512 x 4096 x 14336 89 /
+// 90 (128-row tiles), 118 / 113 (64-row), 132 / 132 (64-row, two parts); 100 x
+// 4096 x 4096 26 / 28, 20.6 / 21, 18.5 / 17 (64-row, one, two, four parts); Q6_K
+// 256 x 14336 x 4096 157 / 184, 88 / 102, 63 / 61 (128-row, one, two, four), 74
+// / 74 (64-row, two).
+struct Plan {
+    int tm;
+    uint32_t parts;
+};
+// The planes of the parts stay inside the scratch a library stream starts with.
+constexpr uint64_t kMaxPlaneBytes = 48ull << 20;
+
+template <Fmt F>
+Plan choose(uint32_t M, uint32_t N, uint32_t K) {
+    const uint32_t nb = K / kSuper;
+    const double cus = device_cus();
+    Plan best{4, 1};
+    double best_cost = 0.0;
+    for (int tm = 4; tm >= 2; tm -= 2) {
+        const double block = F == Fmt::Q4K ? (tm == 4 ? 2.5 : 1.45) : (tm == 4 ? 3.2 : 2.2);
+        const double tiles = static_cast<double>((M + 32u * tm - 1) / (32u * tm)) * ((N + 127u) / 128u);
+        for (uint32_t parts = 1; parts <= 8 && parts * 2 <= nb + 1; ++parts) {
+            const double plane_bytes = 4.0 * M * N * parts;
+            if (parts > 1 && plane_bytes > static_cast<double>(kMaxPlaneBytes)) break;
+            const double rounds = std::ceil(tiles * parts / cus);
+            double cost = rounds * (5.0 + block * ((nb + parts - 1) / parts));
+            if (parts > 1) cost += 3.0 + 2.0 * plane_bytes / 4e6;
+            if (best_cost == 0.0 || cost < best_cost) {
+                best_cost = cost;
+                best = {tm, parts};
+            }
+        }
+    }
+    return best;
+}
+
+template <Fmt F, typename OutT>
+hipError_t launch(const void* x, const void* w, void* y, uint32_t M, uint32_t N, uint32_t K, hipStream_t stream) {
+    const auto* xp = static_cast<const uint16_t*>(x);
+    const auto* wp = static_cast<const uint8_t*>(w);
+    auto* yp = static_cast<OutT*>(y);
+    auto run = [&](const Plan& p) {
+        return p.tm == 4 ? launch_tile<F, 4, 1, 2, OutT>(xp, wp, yp, M, N, K, p.parts, stream)
+                         : launch_tile<F, 2, 1, 2, OutT>(xp, wp, yp, M, N, K, p.parts, stream);
+    };
+    const Plan plan = choose<F>(M, N, K);
+    const hipError_t e = run(plan);
+    // under graph capture without scratch for the planes: one part
+    if (e == hipErrorStreamCaptureUnsupported && plan.parts > 1) return run({plan.tm, 1});
+    return e;
+}
+
+}  // namespace
+
+bool prefill_supported(Fmt f, const void* x, const void* w, uint32_t M, uint32_t N, uint32_t K) {
+    return M > 64 && K >= kSuper && K <= (1u << 22) && static_cast<uint64_t>(M) * (K / kSuper) <= (1ull << 31) &&
+           (reinterpret_cast<uintptr_t>(x) & 15u) == 0 &&
+           (f == Fmt::Q6K || (reinterpret_cast<uintptr_t>(w) & 15u) == 0);
+}
+
+hipError_t launch_prefill(Fmt f, bool f16_out, const void* x, const void* w, void* y, uint32_t M, uint32_t N,
+                          uint32_t K, hipStream_t stream) {
+    if (f == Fmt::Q4K)
+        return f16_out ? launch<Fmt::Q4K, _Float16>(x, w, y, M, N, K, stream)
+                       : launch<Fmt::Q4K, float>(x, w, y, M, N, K, stream);
+    return f16_out ? launch<Fmt::Q6K, _Float16>(x, w, y, M, N, K, stream)
+                   : launch<Fmt::Q6K, float>(x, w, y, M, N, K, stream);
+}
+
+}  // namespace mote::kquant

@@ -1,0 +1,103 @@
+"""GPU parity of the many-token K-quant tiles (more than 64 tokens), at the
+edges of their tiles, of their K split between wave groups and of the K parts,
+judged on every output as the few-token kernels are (test_gpu_kquant.py):
+against the oracle's f64 linear over the oracle-decoded weights.
+
+The tiles' products are exact and summed in f32, so besides the tolerance of
+the few-token tests each shape is held to the error of that summation: K
+additions that round a partial sum of about sqrt(K) max|w| max|x| by 2^-24 each,
+independently, come to K 2^-24 max|w| max|x|; four times that is allowed (the
+Q4_K sub-block sums, carried in 22 bits, stay below it).
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from helpers import bits_to_f32
+from mote_amd import workloads as wl
+from mote_amd.device import DeviceBuffer, Stream
+from test_gpu_kquant import FORMATS, _blocks, _check, _fmt, _judge, _run
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [
+    # (M, N, K): one super-block (the second wave group idle), odd counts of
+    # blocks (uneven groups), one row past and short of a tile on both sides,
+    # a single column, several tiles of both heights, K parts (few tiles, long
+    # K) with a short last part
+    (65, 1, 256),
+    (128, 128, 512),
+    (129, 127, 768),
+    (66, 129, 2304),
+    (200, 33, 1280),
+    (257, 300, 4096),
+    (70, 40, 14336),
+    (130, 60, 9472),
+]
+
+
+@pytest.mark.parametrize("name", list(FORMATS))
+@pytest.mark.parametrize("m,n,k", SHAPES)
+def test_linear_many_tokens(stream, oracle, name, m, n, k):
+    seed = 800 + m * 3 + n + k
+    w = (wl.q4_k_weights if name == "q4_k" else wl.q6_k_weights)(seed, n, k)
+    x = wl.normal_f16(wl.seed_for(41, seed), m * k)
+    y64, max_w, max_x = _judge(oracle, name, x, w, m, n, k)
+    y = _run(stream, name, x, w, m, n, k)
+    _check(y, y64, k, max_w, max_x, what=f"{name} {m}x{n}x{k} f32")
+    bound = 4.0 * k * 2.0 ** -24 * max_w * max_x
+    assert float(np.abs(y - y64).max()) <= bound, f"{name} {m}x{n}x{k}: past f32 summation of exact products"
+    y16 = _run(stream, name, x, w, m, n, k, f16_out=True)
+    _check(y16, y64, k, max_w, max_x, 2.0 ** -11, what=f"{name} {m}x{n}x{k} f16")
+
+
+@pytest.mark.parametrize("name", list(FORMATS))
+@pytest.mark.parametrize("m,k", [(80, 1536), (72, 8192)])
+def test_many_tokens_every_finite_scale(stream, oracle, name, m, k):
+    n = 40
+    w = _blocks(name, 820 + k, n * k // 256)
+    x = wl.normal_f16(wl.seed_for(42, 1), m * k)
+    y64, max_w, max_x = _judge(oracle, name, x, w, m, n, k)
+    assert np.isfinite(y64).all()
+    _check(_run(stream, name, x, w, m, n, k), y64, k, max_w, max_x, what=f"{name} wide scales")
+
+
+@pytest.mark.parametrize("name", list(FORMATS))
+def test_many_tokens_non_finite(stream, oracle, name):
+    """Infinite and NaN activations, and activations whose sub-block sums pass
+    binary16's range: the outputs are the definition's."""
+    m, n, k = 70, 24, 12288
+    w = (wl.q4_k_weights if name == "q4_k" else wl.q6_k_weights)(830, n, k)
+    x = wl.normal_f16(wl.seed_for(43, m), m * k).copy()
+    x[5000] = 0x7C00
+    x[(m - 1) * k + 9000] = 0xFC00
+    x[k + 100] = 0x7E00
+    x[2 * k + 64:2 * k + 96] = 0x7000  # token 2: 32 activations of 8192
+    y64 = oracle.kquant_linear_f64(bits_to_f32(x), w, _fmt(oracle, name), m, n, k)
+    max_w = float(np.abs(oracle.dequantize_kquant_row(w, _fmt(oracle, name), n * k)).max())
+    y = _run(stream, name, x, w, m, n, k)
+    for cls in (np.isnan, np.isposinf, np.isneginf):
+        assert np.array_equal(cls(y), cls(y64)), f"{name}: {cls.__name__} positions differ"
+    ok = np.isfinite(y64)
+    _check(y[ok], y64[ok], k, max_w, 8192.0, what=f"{name} finite outputs")
+
+
+def test_q6_k_many_tokens_at_two_byte_offset(stream, oracle):
+    m, n, k = 70, 50, 1280
+    w = wl.q6_k_weights(840, n, k)
+    x = wl.normal_f16(wl.seed_for(44, 1), m * k)
+    y64, max_w, max_x = _judge(oracle, "q6_k", x, w, m, n, k)
+    _check(_run(stream, "q6_k", x, w, m, n, k, w_offset=2), y64, k, max_w, max_x, what="q6_k at 2 mod 4")
+
+
+@pytest.mark.parametrize("name", list(FORMATS))
+@pytest.mark.parametrize("x_offset", [2, 8])
+def test_many_tokens_unaligned_activations(stream, oracle, name, x_offset):
+    """Activations off the 16-byte grid keep the few-token kernels' route."""
+    m, n, k = 66, 20, 512
+    w = (wl.q4_k_weights if name == "q4_k" else wl.q6_k_weights)(850, n, k)
+    x = wl.normal_f16(wl.seed_for(45, 1), m * k)
+    y64, max_w, max_x = _judge(oracle, name, x, w, m, n, k)
+    _check(_run(stream, name, x, w, m, n, k, x_offset=x_offset), y64, k, max_w, max_x, what=f"{name} x unaligned")
