@@ -145,6 +145,10 @@ __global__ __launch_bounds__(64 * kTileWaves * KG) void kq_prefill_kernel(
     constexpr int kSlots = 4;                  // interval t, a quarter p = t % 4 of a super-block: slot p
     constexpr int NA = BM / (8 * kTileWaves);  // activation loads per wave and interval
     constexpr int NB = F == Fmt::Q6K ? 2 : 1;  // operands per 8 weights
+    // Block sums: the 64-row Q6_K tiles, which also serve few tokens, keep the
+    // two operands' sums apart (half as many roundings in a row: 1.2e-7 of the
+    // result at K = 4096, as the few-token tiles, against 1.45e-7).
+    constexpr int NC = NB == 2 && TM == 2 ? 2 : 1;
     constexpr uint32_t BB = block_bytes<F>();
     static_assert((KG == 1 || KG == 2) && TM % KG == 0, "the groups share the output tiles evenly");
     constexpr int kRing = kSlots * KG * kUnit;
@@ -317,13 +321,17 @@ __global__ __launch_bounds__(64 * kTileWaves * KG) void kq_prefill_kernel(
         }
     };
 
-    f32x16 acc[TM][TN], blk[TM][TN];
+    f32x16 acc[TM][TN], blk[NC][TM][TN];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = blk[i][j][r] = 0.0f;
+            for (int r = 0; r < 16; ++r) {
+                acc[i][j][r] = 0.0f;
+#pragma unroll
+                for (int c = 0; c < NC; ++c) blk[c][i][j][r] = 0.0f;
+            }
     const f32x16 zero = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
     f16x8 a[2][TM];
     const uint32_t a_row = lr * 128, a_x = (lr >> 1) & 7;
@@ -339,13 +347,16 @@ __global__ __launch_bounds__(64 * kTileWaves * KG) void kq_prefill_kernel(
 #pragma unroll
             for (int i = 0; i < TM; ++i)
 #pragma unroll
-                for (int j = 0; j < TN; ++j) blk[i][j] = mfma32(a[C][i], b[C][j][k], blk[i][j]);
+                for (int j = 0; j < TN; ++j) blk[k % NC][i][j] = mfma32(a[C][i], b[C][j][k], blk[k % NC][i][j]);
     };
     // The first slice of a super-block: the sums of the one before join the
     // result, tile by tile ahead of the tile's first product.
     auto fold = [&](int i, int j) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[i][j][r] = __builtin_fmaf(d_fold[j], blk[i][j][r], acc[i][j][r]);
+        for (int r = 0; r < 16; ++r) {
+            const float sum = NC == 2 ? blk[0][i][j][r] + blk[NC - 1][i][j][r] : blk[0][i][j][r];
+            acc[i][j][r] = __builtin_fmaf(d_fold[j], sum, acc[i][j][r]);
+        }
     };
     auto multiply_first = [&]() {
 #pragma unroll
@@ -355,7 +366,7 @@ __global__ __launch_bounds__(64 * kTileWaves * KG) void kq_prefill_kernel(
 #pragma unroll
                 for (int j = 0; j < TN; ++j) {
                     if (k == 0) fold(i, j);
-                    blk[i][j] = mfma32(a[0][i], b[0][j][k], k == 0 ? zero : blk[i][j]);
+                    blk[k % NC][i][j] = mfma32(a[0][i], b[0][j][k], k < NC ? zero : blk[k % NC][i][j]);
                 }
     };
     // Q4_K's minimum term of the super-block, one tile per slice of its second
@@ -657,6 +668,7 @@ hipError_t launch_tile(const uint16_t* x, const uint8_t* w, OutT* y, uint32_t M,
 struct Plan {
     int tm;
     uint32_t parts;
+    double us;
 };
 // The planes of the parts stay inside the scratch a library stream starts with.
 constexpr uint64_t kMaxPlaneBytes = 48ull << 20;
@@ -665,8 +677,7 @@ template <Fmt F>
 Plan choose(uint32_t M, uint32_t N, uint32_t K) {
     const uint32_t nb = K / kSuper;
     const double cus = device_cus();
-    Plan best{4, 1};
-    double best_cost = 0.0;
+    Plan best{4, 1, 0.0};
     for (int tm = 4; tm >= 2; tm -= 2) {
         const double block = F == Fmt::Q4K ? (tm == 4 ? 2.5 : 1.45) : (tm == 4 ? 3.2 : 2.2);
         const double tiles = static_cast<double>((M + 32u * tm - 1) / (32u * tm)) * ((N + 127u) / 128u);
@@ -676,13 +687,26 @@ Plan choose(uint32_t M, uint32_t N, uint32_t K) {
             const double rounds = std::ceil(tiles * parts / cus);
             double cost = rounds * (5.0 + block * ((nb + parts - 1) / parts));
             if (parts > 1) cost += 3.0 + 2.0 * plane_bytes / 4e6;
-            if (best_cost == 0.0 || cost < best_cost) {
-                best_cost = cost;
-                best = {tm, parts};
-            }
+            if (best.us == 0.0 || cost < best.us) best = {tm, parts, cost};
         }
     }
     return best;
+}
+
+// Up to 64 tokens the few-token tiles of kquant.hip compete.  Their time is
+// about 4 us and 6.2 (Q4_K) or 13.3 ns (Q6_K) per item, (16 rows, 16 tokens, 16
+// super-blocks), twice that with three token tiles, and 3 us for a part sum
+// (64 x 4096 x 14 336 26 / 51 us, 48 x 4096 x 14 336 39 / 77, 64 x 4096 x 4096
+// 9.7 / 17.5, 64 x 14 336 x 4096 32 / 60, 32 x 14 336 x 4096 19 / 34); here the
+// same shapes take 23.4 / 30.3, 22.0 / 29.6, 17 / 19, 23.2 / 27.6, 22 / 26.5.
+bool worth(Fmt f, uint32_t M, uint32_t N, uint32_t K) {
+    if (M > 64) return true;
+    if (M <= 16) return false;
+    const uint32_t token_tiles = (M + 15) / 16, kparts = (K / kSuper + 15) / 16;
+    const double items = static_cast<double>((N + 15) / 16) * token_tiles * kparts;
+    double few = 4.0 + items * (f == Fmt::Q4K ? 6.2e-3 : 13.3e-3) * (token_tiles == 3 ? 2.0 : 1.0);
+    if (kparts > 1) few += 3.0;
+    return (f == Fmt::Q4K ? choose<Fmt::Q4K>(M, N, K) : choose<Fmt::Q6K>(M, N, K)).us + 1.5 < 0.95 * few;
 }
 
 template <Fmt F, typename OutT>
@@ -697,14 +721,14 @@ hipError_t launch(const void* x, const void* w, void* y, uint32_t M, uint32_t N,
     const Plan plan = choose<F>(M, N, K);
     const hipError_t e = run(plan);
     // under graph capture without scratch for the planes: one part
-    if (e == hipErrorStreamCaptureUnsupported && plan.parts > 1) return run({plan.tm, 1});
+    if (e == hipErrorStreamCaptureUnsupported && plan.parts > 1) return run({plan.tm, 1, 0.0});
     return e;
 }
 
 }  // namespace
 
 bool prefill_supported(Fmt f, const void* x, const void* w, uint32_t M, uint32_t N, uint32_t K) {
-    return M > 64 && K >= kSuper && K <= (1u << 22) && static_cast<uint64_t>(M) * (K / kSuper) <= (1ull << 31) &&
+    return worth(f, M, N, K) && K >= kSuper && K <= (1u << 22) && static_cast<uint64_t>(M) * (K / kSuper) <= (1ull << 31) &&
            (reinterpret_cast<uintptr_t>(x) & 15u) == 0 &&
            (f == Fmt::Q6K || (reinterpret_cast<uintptr_t>(w) & 15u) == 0);
 }

@@ -1,5 +1,5 @@
-"""GPU parity of the many-token K-quant tiles (more than 64 tokens), at the
-edges of their tiles, of their K split between wave groups and of the K parts,
+"""GPU parity of the many-token K-quant tiles (more than 64 tokens, and 17 to
+64 where they are the faster ones), at the edges of their tiles, of their K split between wave groups and of the K parts,
 judged on every output as the few-token kernels are (test_gpu_kquant.py):
 against the oracle's f64 linear over the oracle-decoded weights.
 
@@ -35,6 +35,10 @@ SHAPES = [
     (257, 300, 4096),
     (70, 40, 14336),
     (130, 60, 9472),
+    # up to 64 tokens, wide enough to come here
+    (33, 3001, 768),
+    (48, 4100, 512),
+    (64, 7000, 1280),
 ]
 
 
