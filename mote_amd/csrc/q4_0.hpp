@@ -66,6 +66,12 @@ bool gemv_lds_supports(const Variant& v, const Problem& p);
 bool skinny_mfma_supports(const Variant& v, const Problem& p);
 bool prefill_supports(const Variant& v, const Problem& p);
 
+// The prefill tiles' body whose operands come through direct-to-LDS rings
+// (q4_0_prefill_ring.hip): the problems it takes, and a launch of its bm x bn
+// tiles (128 x 256, 128 x 128; gate/up 128 x 128).
+bool prefill_ring_supports(const Problem& p);
+hipError_t launch_prefill_ring(const Problem& p, int bm, int bn, bool gate_up);
+
 hipError_t launch_zero_fill(void* y, uint64_t count, OutType out, hipStream_t stream);
 // K above 2^31 - 1 (p.K unused; the fused gate/up when p.w_up is set): 64-bit
 // per-element products over K parts of each output, then the parts added in

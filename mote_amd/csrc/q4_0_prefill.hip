@@ -41,6 +41,11 @@
 // binary16 product rounds (q - 8) d, up to 14 significant bits, to 11 (a
 // relative error of at most 2^-11 per weight); that is well inside the
 // tolerance for Q4_0's 4-bit values but measured too coarse for 8-bit ones.
+//
+// The 128-row multi-pair Q4_0 tiles (`_k2`) run the body of
+// q4_0_prefill_ring.hip where K is a multiple of 256 and the operands are
+// 16-byte aligned (5 - 16 % faster, measured there); this body serves them
+// otherwise.
 #include "common.hpp"
 #include "q4_0.hpp"
 
@@ -475,6 +480,9 @@ template <int BM, int BN, bool GATE_UP, bool Q8 = false, int WM = 2, bool T32 = 
           int KP = 1>
 hipError_t launch_prefill(const Problem& p) {
     if (p.K % (64u * KP) != 0) return hipErrorInvalidValue;
+    // 128-row Q4_0 tiles: the ring body where the operands fit it.
+    if constexpr (SPEC && T32 && KP > 1 && BM == 128 && !Q8)
+        if (prefill_ring_supports(p)) return launch_prefill_ring(p, BM, BN, GATE_UP);
     const uint32_t m_tiles = (p.M + BM - 1) / BM;
     const uint32_t n_tiles = (p.N + BN - 1) / BN;
     const uint64_t total64 = static_cast<uint64_t>(m_tiles) * n_tiles;

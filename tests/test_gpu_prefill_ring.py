@@ -1,0 +1,87 @@
+"""The 128-row Q4_0 prefill tiles' ring body (q4_0_prefill_ring.hip) against the
+staging-wave body of the same tiles, which weights off the 16-byte grid take.
+Both decode every weight to the same binary16 value and sum exact products in
+f32, in another order: K additions that round a partial sum of about sqrt(K)
+max|w| max|x| by 2^-24 each, independently, in either body; twice their sum is
+allowed.  (Against the oracle both are judged by test_every_mfma_variant and
+the wide-scale tests.)"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from helpers import bits_to_f32, wide_q4_0_weights
+from mote_amd import ops, workloads as wl
+from mote_amd.device import DeviceBuffer
+
+pytestmark = pytest.mark.gpu
+
+
+def _at(array, offset):
+    b = DeviceBuffer(array.nbytes + offset)
+    b.upload(array, offset=offset)
+    return b, b.ptr + offset
+
+
+def _both(stream, call, x, weights, m, n, f16_out):
+    """The output with the weights on and off the 16-byte grid."""
+    out = []
+    xb, xp = _at(x, 0)
+    for offset in (0, 4):
+        held = [_at(w, offset) for w in weights]
+        yb = DeviceBuffer(m * n * (2 if f16_out else 4))
+        yb.upload(np.full(yb.nbytes, 0xA5, dtype=np.uint8))
+        call(xp, [p for _, p in held], yb.ptr)
+        stream.synchronize()
+        y = yb.download(np.uint16 if f16_out else np.float32)
+        out.append((bits_to_f32(y) if f16_out else y).astype(np.float64))
+    return out
+
+
+SHAPES = [
+    # (M, N, K): one super-pair (the second half of K idle), uneven halves, one
+    # row past and short of a tile on both sides, one column, several tiles
+    (128, 256, 256),
+    (129, 255, 768),
+    (65, 1, 512),
+    (127, 129, 2816),
+    (300, 513, 1024),
+]
+
+
+@pytest.mark.parametrize("variant", ["mfma_x32s_m128_n256_w1_k2", "mfma_x32s_m128_n128_w1_k2"])
+@pytest.mark.parametrize("m,n,k", SHAPES)
+@pytest.mark.parametrize("scales", ["ordinary", "wide"])
+def test_ring_matches_staging_body(stream, variant, m, n, k, scales):
+    d = ops.Q4_0Dispatch()
+    d.force(variant)
+    x = wl.normal_f16(wl.seed_for(61, m + k), m * k)
+    w = wl.q4_0_weights(wl.seed_for(61, n + k), n, k) if scales == "ordinary" else wide_q4_0_weights(62 + n, n, k, "full")
+    max_d = float(np.abs(w.reshape(-1, 18)[:, 0:2].copy().view(np.float16).astype(np.float64)).max())
+    bound = 4.0 * k * 2.0 ** -24 * 8.0 * max_d * float(np.abs(bits_to_f32(x)).max())
+    for f16_out in (False, True):
+        if f16_out and scales == "wide":
+            continue  # past binary16's range
+        got, want = _both(stream, lambda xp, wp, yp: d.linear(xp, wp[0], yp, m, n, k, stream, f16_out=f16_out), x, [w],
+                          m, n, f16_out)
+        tol = bound + (2.0 ** -10 * np.abs(want) if f16_out else 0.0)
+        assert np.all(np.abs(got - want) <= tol), f"{variant} {m}x{n}x{k}: {float(np.abs(got - want).max())} > {bound}"
+
+
+@pytest.mark.parametrize("m,n,k", [(128, 128, 256), (129, 127, 768), (200, 200, 1024)])
+def test_gate_up_ring_matches_staging_body(stream, m, n, k):
+    d = ops.Q4_0Dispatch()
+    d.force("gateup_mfma_x32s_m128_n128_w1_k2")
+    x = wl.normal_f16(wl.seed_for(63, m + k), m * k)
+    # unit outputs: the SiLU and the product then move an error by at most its
+    # slope (1.1) times the other factor
+    scale = np.float16(1.0 / (4.6 * np.sqrt(k)))
+    wg, wu = (wl.q4_0_weights(wl.seed_for(63, n + i), n, k).reshape(-1, 18).copy() for i in (0, 1))
+    for w in (wg, wu):
+        w[:, 0:2] = np.array([scale]).view(np.uint8)
+    e = 4.0 * k * 2.0 ** -24 * 8.0 * float(scale) * float(np.abs(bits_to_f32(x)).max())
+    got, want = _both(stream, lambda xp, wp, yp: d.gate_up_silu(xp, wp[0], wp[1], yp, m, n, k, stream), x,
+                      [wg.reshape(-1), wu.reshape(-1)], m, n, False)
+    tol = 8.0 * 2.2 * e + 2.0 ** -20 * np.abs(want)  # factors below 8; the device exponential
+    assert np.all(np.abs(got - want) <= tol), f"{float((np.abs(got - want) - tol).max())} past the tolerance"
