@@ -9,7 +9,9 @@
 
 namespace mote::kquant {
 
-enum class Fmt { Q4K, Q6K };
+// (Q8: eight consecutive Q8_0 blocks, 256 elements in 272 bytes; many-token
+// linear only.)
+enum class Fmt { Q4K, Q6K, Q8 };
 
 namespace {
 
@@ -17,7 +19,7 @@ constexpr uint32_t kSuper = 256;
 
 template <Fmt F>
 constexpr uint32_t block_bytes() {
-    return F == Fmt::Q4K ? 144u : 210u;
+    return F == Fmt::Q4K ? 144u : F == Fmt::Q6K ? 210u : 272u;
 }
 
 __device__ __forceinline__ float half_bits_to_float(uint32_t bits) {
@@ -94,6 +96,9 @@ __device__ inline float kq_value(const uint8_t* blk, uint32_t e) {
         const uint32_t byte = blk[16 + 32 * p + l];
         const float prod = d1 * static_cast<float>(h ? byte >> 4 : byte & 15u);
         return prod - m1;
+    } else if constexpr (F == Fmt::Q8) {
+        const uint8_t* b = blk + 34 * (e >> 5);
+        return half_bits_to_float(b[0] | (b[1] << 8)) * static_cast<float>(static_cast<int8_t>(b[2 + (e & 31u)]));
     } else {
         const uint32_t g = e >> 7, c = (e >> 5) & 3u, l = e & 31u;
         const uint32_t low = blk[64 * g + 32 * (c & 1u) + l] >> (4 * (c >> 1)) & 15u;

@@ -1,4 +1,4 @@
-// K-quant linear over many tokens on the matrix cores, y[M, N] = x[M, K] (f16)
+// K-quant (and Q8_0) linear over many tokens on the matrix cores, y[M, N] = x[M, K] (f16)
 // . W[N, K]^T with Q4_K or Q6_K weights (layouts in kquant.hip).
 //
 // A workgroup of 4 KG waves computes a 32 TM x 128 tile of y over one part of
@@ -9,9 +9,10 @@
 // (h, u) of quarter p of a super-block, its elements
 //   64 p + 32 h + 16 c + 8 u .. + 7,
 // so a lane's quants of a quarter are contiguous bytes: it loads them itself,
-// global memory to registers, and re-uses the registers for the same quarter
-// of the next super-block as soon as they are decoded (about three quarters
-// ahead of their use; no LDS traffic for the weights).
+// global memory to registers, half a super-block at a time, and re-uses the
+// registers for the same half of the next super-block as soon as they are
+// decoded (two to three quarters ahead of their use; no LDS traffic for the
+// weights).
 //
 // Weight operands are exact binary16 integers, as in the few-token tiles of
 // kquant.hip: Q4_K sc q (at most 63 x 15), one packed fma from 1024 + q or 64 +
@@ -38,15 +39,20 @@
 // values, as in the few-token tiles.
 //
 // Measured on MI355X (weights of three calls rotated): 512 x 4096 x 14 336 Q4_K
-// 84 us (716 TFLOP/s), where the four-token passes of the LDS-ring GEMV, which
+// 82 us (733 TFLOP/s), where the four-token passes of the LDS-ring GEMV, which
 // read every weight M / 4 times, took 1723; 256 x 14 336 x 4096 Q6_K 62 us
 // against 1203.  Bound by the interval's instruction stream: MFMAs fill 37 % of
 // the cycles, vector instructions and the LDS (A operands read once per wave)
 // a third each, imperfectly overlapped at two waves per SIMD.  128 x 256 tiles
 // of four waves with 512 registers (half the A reads per MFMA) measured level
-// (84 us); 64-row tiles 20 - 35 % slower per row.
+// (84 us); 96- and 64-row tiles take 8 and 20 % longer per row and are for
+// token counts and grids that 128-row tiles fill badly (300 x 4096 x 14 336: 65
+// us on 96-row tiles).  The Q8_0 linear has a kernel of its own
+// (q8_0_prefill_ring.hpp) and shares the launch.
 #include "kquant_blocks.hpp"
 #include "q4_0.hpp"
+#include "q8_0_prefill_ring.hpp"
+#include "tile_ops.hpp"
 
 #include <cmath>
 #include <type_traits>
@@ -54,48 +60,10 @@
 namespace mote::kquant {
 namespace {
 
-typedef __attribute__((address_space(3))) void* lds_ptr_t;
 // 16-byte vector at a 2-byte-aligned address (one unaligned dwordx4 load).
 typedef uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
 
 constexpr int kTileWaves = 4;                 // waves along N
-
-constexpr int vm_wait(int n) { return (n & 0xF) | ((n >> 4) << 14) | 0x0F70; }
-constexpr int kLgkmWait = 0xC07F;  // lgkmcnt(0) alone; ANDed with vm_wait(n): both
-
-// The builtins behind plain functions (usable from generic lambdas).
-typedef __amdgpu_buffer_rsrc_t Buffer;
-__device__ __forceinline__ Buffer buffer_at(const void* base) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, 0xFFFFFFFFu, 0x00020000);
-}
-__device__ __forceinline__ void load_lds16(Buffer src, uint32_t lane_offset, uint32_t offset, uint8_t* dst) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (lds_ptr_t)dst, 16, lane_offset, offset, 0, 0);
-}
-template <int I>
-__device__ __forceinline__ void wait_counts() { __builtin_amdgcn_s_waitcnt(I); }
-__device__ __forceinline__ void order_fence() { __builtin_amdgcn_sched_barrier(0); }
-// Keeps memory operations on their side of this point, in the compiler's
-// intermediate code and in its schedule: the counted waits below rely on the
-// order in which the loads are issued.
-__device__ __forceinline__ void issue_fence() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
-}
-__device__ __forceinline__ void group_barrier() { __builtin_amdgcn_s_barrier(); }
-__device__ __forceinline__ f32x16 mfma32(const f16x8& a, const f16x8& b, const f32x16& c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ uint32_t perm(uint32_t hi, uint32_t lo, uint32_t sel) {
-    return __builtin_amdgcn_perm(hi, lo, sel);
-}
-__device__ __forceinline__ f16x2 both(f16x2 v, bool high) {
-    const uint32_t b = __builtin_bit_cast(uint32_t, v);
-    return as_h2(perm(b, b, high ? 0x03020302u : 0x01000100u));
-}
-__device__ __forceinline__ f16x2 both(_Float16 v) { return f16x2{v, v}; }
-__device__ __forceinline__ f16x8 join(f16x2 a, f16x2 b, f16x2 c, f16x2 d) {
-    return f16x8{a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y};
-}
 
 // Keeps a converted scale in f32: as mixed-precision fmas from the binary16
 // word, two of which in a row need a wait state, the folds took twice as long.
@@ -119,9 +87,11 @@ struct Raw<Fmt::Q6K> {
     uint32_t d;
 };
 
+
 // The scales of the super-block being multiplied.
 template <Fmt F>
 struct Scales;
+
 template <>
 struct Scales<Fmt::Q4K> {
     uint32_t sc[2];  // sc_0..3, sc_4..7, a byte each
@@ -150,9 +120,9 @@ __global__ __launch_bounds__(64 * kTileWaves * KG) void kq_prefill_kernel(
     // result at K = 4096, as the few-token tiles, against 1.45e-7).
     constexpr int NC = NB == 2 && TM == 2 ? 2 : 1;
     constexpr uint32_t BB = block_bytes<F>();
-    static_assert((KG == 1 || KG == 2) && TM % KG == 0, "the groups share the output tiles evenly");
+    static_assert(KG == 1 || KG == 2, "the groups hand half of the output tiles over");
     constexpr int kRing = kSlots * KG * kUnit;
-    constexpr int kReduce = KG == 1 ? 0 : kTileWaves * KG * (TM / 2) * TN * 4096;
+    constexpr int kReduce = KG == 1 ? 0 : kTileWaves * KG * ((TM + 1) / 2) * TN * 4096;
     __shared__ __attribute__((aligned(1024))) uint8_t lds[kRing > kReduce ? kRing : kReduce];
 
     const uint32_t logical = (blockIdx.x % 8u) * per_xcd + blockIdx.x / 8u;
@@ -199,21 +169,25 @@ __global__ __launch_bounds__(64 * kTileWaves * KG) void kq_prefill_kernel(
     for (int j = 0; j < TN; ++j)
         wrow[j] = w + (static_cast<size_t>(min(n0 + (wn * TN + j) * 32 + lr, N - 1)) * nb + b0) * BB;
     Raw<F> raw[TN];
-    // The quants freed by quarter p, of super-block s (clamped): quarter p's
-    // (Q4_K), half p / 2's after its second quarter (Q6_K).
+    // After the second quarter of a half block, p = 1 or 3: that half's quants
+    // of super-block s (clamped).  A quarter at a time, as it is freed, fetched
+    // the lines of a row's half block twice.
     auto load_quants = [&](auto pc, uint32_t s) {
-        constexpr int P = decltype(pc)::value;
-        const size_t at = static_cast<size_t>(min(s, ns - 1)) * BB;
+        constexpr int P = decltype(pc)::value, g = P / 2;
+        if constexpr (P % 2 == 1) {
+            const size_t at = static_cast<size_t>(min(s, ns - 1)) * BB;
 #pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            const uint8_t* blk = wrow[j] + at;
-            if constexpr (F == Fmt::Q4K) {
-                raw[j].qs[P] = *reinterpret_cast<const u32x4*>(blk + 16 + 32 * P + 16 * lc);
-            } else if constexpr (P % 2 == 1) {
-                constexpr int g = P / 2;
-                raw[j].la[g] = *reinterpret_cast<const u32x4_a2*>(blk + 64 * g + 16 * lc);
-                raw[j].lb[g] = *reinterpret_cast<const u32x4_a2*>(blk + 64 * g + 32 + 16 * lc);
-                raw[j].qh[g] = *reinterpret_cast<const u32x4_a2*>(blk + 128 + 32 * g + 16 * lc);
+            for (int j = 0; j < TN; ++j) {
+                const uint8_t* blk = wrow[j] + at;
+                if constexpr (F == Fmt::Q4K) {
+#pragma unroll
+                    for (int p = 2 * g; p < 2 * g + 2; ++p)
+                        raw[j].qs[p] = *reinterpret_cast<const u32x4*>(blk + 16 + 32 * p + 16 * lc);
+                } else {
+                    raw[j].la[g] = *reinterpret_cast<const u32x4_a2*>(blk + 64 * g + 16 * lc);
+                    raw[j].lb[g] = *reinterpret_cast<const u32x4_a2*>(blk + 64 * g + 32 + 16 * lc);
+                    raw[j].qh[g] = *reinterpret_cast<const u32x4_a2*>(blk + 128 + 32 * g + 16 * lc);
+                }
             }
         }
     };
@@ -410,8 +384,9 @@ __global__ __launch_bounds__(64 * kTileWaves * KG) void kq_prefill_kernel(
     };
     // Loads a wave issues behind interval t's activations of four intervals on:
     // quants, the sums (p = 0), the next header (p = 2).
-    constexpr int kBehind[4] = {F == Fmt::Q4K ? TN + TM : 0, F == Fmt::Q4K ? TN : 3 * TN, F == Fmt::Q4K ? 2 * TN : 2 * TN,
-                                F == Fmt::Q4K ? TN : 3 * TN};
+    constexpr bool kQ4 = F == Fmt::Q4K;
+    constexpr int kHalf = (kQ4 ? 2 : 3) * TN;  // a half block's quants
+    constexpr int kBehind[4] = {kQ4 ? TM : 0, kHalf, kQ4 ? TN : 2 * TN, kHalf};
     using I0 = std::integral_constant<int, 0>;
     using I1 = std::integral_constant<int, 1>;
     using I2 = std::integral_constant<int, 2>;
@@ -420,22 +395,19 @@ __global__ __launch_bounds__(64 * kTileWaves * KG) void kq_prefill_kernel(
     if (ns > 0) {  // uniform over the wave; groups without work only meet the barriers
         load_a(0, 0);
         issue_fence();
-        load_quants(I0{}, 0);
-        issue_fence();
         load_a(1, 1);
         issue_fence();
         load_quants(I1{}, 0);
         issue_fence();
         load_a(2, 2);
         issue_fence();
-        load_quants(I2{}, 0);
         load_head(0);
         issue_fence();
         load_a(3, 3);
         issue_fence();
         load_quants(I3{}, 0);
         issue_fence();
-        wait_counts<vm_wait(3 * NA + (F == Fmt::Q4K ? 5 : 8) * TN)>();  // interval 0's activations
+        wait_counts<vm_wait(3 * NA + (kQ4 ? 5 : 8) * TN)>();  // interval 0's activations
     }
     group_barrier();
     order_fence();
@@ -507,10 +479,11 @@ __global__ __launch_bounds__(64 * kTileWaves * KG) void kq_prefill_kernel(
     wait_counts<vm_wait(0)>();
     __syncthreads();
 
-    // Two groups: each keeps half of the tiles and hands the other half over.
-    int tile0 = 0;
+    // Two groups: the first keeps row tiles 0 .. H - 1, the second the others;
+    // each hands over the rest.
+    constexpr int H = KG == 1 ? TM : (TM + 1) / 2;
+    const int kept = kg == 0 ? H : TM - H, tile0 = kg == 0 ? 0 : H;
     if constexpr (KG == 2) {
-        constexpr int H = TM / 2;
         float* red = reinterpret_cast<float*>(lds);
         auto slot = [&](int wv, int i, int j, int r) { return red + (((wv * H + i) * TN + j) * 4 + r) * 256 + lane * 4; };
         auto give = [&](const f32x16& v, int i, int j) {
@@ -520,7 +493,7 @@ __global__ __launch_bounds__(64 * kTileWaves * KG) void kq_prefill_kernel(
         };
         if (kg == 0) {
 #pragma unroll
-            for (int i = 0; i < H; ++i)
+            for (int i = 0; i < TM - H; ++i)
 #pragma unroll
                 for (int j = 0; j < TN; ++j) give(acc[H + i][j], i, j);
         } else {
@@ -529,13 +502,14 @@ __global__ __launch_bounds__(64 * kTileWaves * KG) void kq_prefill_kernel(
 #pragma unroll
                 for (int j = 0; j < TN; ++j) {
                     give(acc[i][j], i, j);
-                    acc[i][j] = acc[H + i][j];
+                    if (H + i < TM) acc[i][j] = acc[H + i][j];
                 }
         }
         __syncthreads();
         const int other = wave ^ kTileWaves;
 #pragma unroll
-        for (int i = 0; i < H; ++i)
+        for (int i = 0; i < H; ++i) {
+            if (i >= kept) break;  // uniform
 #pragma unroll
             for (int j = 0; j < TN; ++j)
 #pragma unroll
@@ -544,7 +518,7 @@ __global__ __launch_bounds__(64 * kTileWaves * KG) void kq_prefill_kernel(
 #pragma unroll
                     for (int k = 0; k < 4; ++k) acc[i][j][4 * r + k] += v[k];
                 }
-        tile0 = kg * H;
+        }
     }
     // Lane (r, c) holds column r of each tile, rows 8 (k / 4) + 4 c + k % 4.
 #pragma unroll
@@ -552,7 +526,8 @@ __global__ __launch_bounds__(64 * kTileWaves * KG) void kq_prefill_kernel(
         const uint32_t n = n0 + (wn * TN + j) * 32 + lr;
         if (n >= N) continue;
 #pragma unroll
-        for (int i = 0; i < TM / KG; ++i) {
+        for (int i = 0; i < H; ++i) {
+            if (i >= kept) break;
 #pragma unroll
             for (int k = 0; k < 16; ++k) {
                 const uint32_t m = m0 + (tile0 + i) * 32 + 8 * (k / 4) + 4 * lc + k % 4;
@@ -642,12 +617,20 @@ hipError_t launch_tile(const uint16_t* x, const uint8_t* w, OutT* y, uint32_t M,
     }
     const dim3 grid(per_xcd * 8), block(64 * kTileWaves * KG);
     if (parts == 1) {
-        hipLaunchKernelGGL((kq_prefill_kernel<F, TM, TN, KG, false, OutT>), grid, block, 0, stream, x, w, sums, y, partial, M,
-                           N, K, m_tiles, n_tiles, part_blocks, total, per_xcd);
+        if constexpr (F == Fmt::Q8)
+            hipLaunchKernelGGL((q8_prefill_kernel<TM, false, OutT>), grid, block, 0, stream, x, w, y, partial, M, N, K,
+                               m_tiles, n_tiles, part_blocks, total, per_xcd);
+        else
+            hipLaunchKernelGGL((kq_prefill_kernel<F, TM, TN, KG, false, OutT>), grid, block, 0, stream, x, w, sums, y,
+                               partial, M, N, K, m_tiles, n_tiles, part_blocks, total, per_xcd);
         return hipGetLastError();
     }
-    hipLaunchKernelGGL((kq_prefill_kernel<F, TM, TN, KG, true, float>), grid, block, 0, stream, x, w, sums,
-                       static_cast<float*>(nullptr), partial, M, N, K, m_tiles, n_tiles, part_blocks, total, per_xcd);
+    if constexpr (F == Fmt::Q8)
+        hipLaunchKernelGGL((q8_prefill_kernel<TM, true, float>), grid, block, 0, stream, x, w,
+                           static_cast<float*>(nullptr), partial, M, N, K, m_tiles, n_tiles, part_blocks, total, per_xcd);
+    else
+        hipLaunchKernelGGL((kq_prefill_kernel<F, TM, TN, KG, true, float>), grid, block, 0, stream, x, w, sums,
+                           static_cast<float*>(nullptr), partial, M, N, K, m_tiles, n_tiles, part_blocks, total, per_xcd);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL((kq_parts_reduce_kernel<OutT>), dim3(static_cast<uint32_t>((count + 255) / 256)), dim3(256), 0,
@@ -655,16 +638,16 @@ hipError_t launch_tile(const uint16_t* x, const uint8_t* w, OutT* y, uint32_t M,
     return hipGetLastError();
 }
 
-// Which tile and how many K parts: the least of
+// Which tile (32 tm rows) and how many K parts: the least of
 //   rounds x (start + blocks x block time) + reduction,
 // rounds of one workgroup per CU, blocks the super-blocks of a part, the
 // reduction 3 us and the planes written and read once at 4 TB/s.  The start, 5
-// us, and the block times in us are fits to MI355X timings, within 10 % at the
-// shapes fitted (measured against predicted, us): Q4_K 512 x 4096 x 14336 89 /
-// 90 (128-row tiles), 118 / 113 (64-row), 132 / 132 (64-row, two parts); 100 x
-// 4096 x 4096 26 / 28, 20.6 / 21, 18.5 / 17 (64-row, one, two, four parts); Q6_K
-// 256 x 14336 x 4096 157 / 184, 88 / 102, 63 / 61 (128-row, one, two, four), 74
-// / 74 (64-row, two).
+// us, and the block times in us are fits to MI355X timings, within 15 % at the
+// shapes fitted (measured against predicted, us): Q4_K 512 x 4096 x 14 336 82 /
+// 90 (128-row tiles), 101 / 109 (96-row), 99 / 113 (64-row), 100 x 4096 x 4096
+// 18 / 17 (64-row, four parts); Q6_K 256 x 14 336 x 4096 88 / 102, 63 / 61
+// (128-row, two, four parts); Q8_0 300 x 4096 x 14 336 80 / 93, 69 / 74, 79 / 85
+// (128-, 96-, 64-row), 256 x 14 336 x 4096 52 / 53 (64-row, two parts).
 struct Plan {
     int tm;
     uint32_t parts;
@@ -678,8 +661,9 @@ Plan choose(uint32_t M, uint32_t N, uint32_t K) {
     const uint32_t nb = K / kSuper;
     const double cus = device_cus();
     Plan best{4, 1, 0.0};
-    for (int tm = 4; tm >= 2; tm -= 2) {
-        const double block = F == Fmt::Q4K ? (tm == 4 ? 2.5 : 1.45) : (tm == 4 ? 3.2 : 2.2);
+    static constexpr double kBlockUs[3][3] = {{2.5, 1.95, 1.45}, {3.2, 2.7, 2.2}, {2.6, 2.0, 1.45}};
+    for (int tm = 4; tm >= 2; --tm) {
+        const double block = kBlockUs[static_cast<int>(F)][4 - tm];
         const double tiles = static_cast<double>((M + 32u * tm - 1) / (32u * tm)) * ((N + 127u) / 128u);
         for (uint32_t parts = 1; parts <= 8 && parts * 2 <= nb + 1; ++parts) {
             const double plane_bytes = 4.0 * M * N * parts;
@@ -700,7 +684,7 @@ Plan choose(uint32_t M, uint32_t N, uint32_t K) {
 // 9.7 / 17.5, 64 x 14 336 x 4096 32 / 60, 32 x 14 336 x 4096 19 / 34); here the
 // same shapes take 23.4 / 30.3, 22.0 / 29.6, 17 / 19, 23.2 / 27.6, 22 / 26.5.
 bool worth(Fmt f, uint32_t M, uint32_t N, uint32_t K) {
-    if (M > 64) return true;
+    if (M > 64 || f == Fmt::Q8) return true;
     if (M <= 16) return false;
     const uint32_t token_tiles = (M + 15) / 16, kparts = (K / kSuper + 15) / 16;
     const double items = static_cast<double>((N + 15) / 16) * token_tiles * kparts;
@@ -715,8 +699,9 @@ hipError_t launch(const void* x, const void* w, void* y, uint32_t M, uint32_t N,
     const auto* wp = static_cast<const uint8_t*>(w);
     auto* yp = static_cast<OutT*>(y);
     auto run = [&](const Plan& p) {
-        return p.tm == 4 ? launch_tile<F, 4, 1, 2, OutT>(xp, wp, yp, M, N, K, p.parts, stream)
-                         : launch_tile<F, 2, 1, 2, OutT>(xp, wp, yp, M, N, K, p.parts, stream);
+        return p.tm == 4   ? launch_tile<F, 4, 1, 2, OutT>(xp, wp, yp, M, N, K, p.parts, stream)
+               : p.tm == 3 ? launch_tile<F, 3, 1, 2, OutT>(xp, wp, yp, M, N, K, p.parts, stream)
+                           : launch_tile<F, 2, 1, 2, OutT>(xp, wp, yp, M, N, K, p.parts, stream);
     };
     const Plan plan = choose<F>(M, N, K);
     const hipError_t e = run(plan);
@@ -728,13 +713,16 @@ hipError_t launch(const void* x, const void* w, void* y, uint32_t M, uint32_t N,
 }  // namespace
 
 bool prefill_supported(Fmt f, const void* x, const void* w, uint32_t M, uint32_t N, uint32_t K) {
-    return worth(f, M, N, K) && K >= kSuper && K <= (1u << 22) && static_cast<uint64_t>(M) * (K / kSuper) <= (1ull << 31) &&
+    return K % kSuper == 0 && K >= kSuper && worth(f, M, N, K) && K <= (1u << 22) && static_cast<uint64_t>(M) * (K / kSuper) <= (1ull << 31) &&
            (reinterpret_cast<uintptr_t>(x) & 15u) == 0 &&
            (f == Fmt::Q6K || (reinterpret_cast<uintptr_t>(w) & 15u) == 0);
 }
 
 hipError_t launch_prefill(Fmt f, bool f16_out, const void* x, const void* w, void* y, uint32_t M, uint32_t N,
                           uint32_t K, hipStream_t stream) {
+    if (f == Fmt::Q8)
+        return f16_out ? launch<Fmt::Q8, _Float16>(x, w, y, M, N, K, stream)
+                       : launch<Fmt::Q8, float>(x, w, y, M, N, K, stream);
     if (f == Fmt::Q4K)
         return f16_out ? launch<Fmt::Q4K, _Float16>(x, w, y, M, N, K, stream)
                        : launch<Fmt::Q4K, float>(x, w, y, M, N, K, stream);

@@ -44,9 +44,11 @@
 //
 // The 128-row multi-pair Q4_0 tiles (`_k2`) run the body of
 // q4_0_prefill_ring.hip where K is a multiple of 256 and the operands are
-// 16-byte aligned (5 - 16 % faster, measured there); this body serves them
+// 16-byte aligned (5 - 16 % faster, measured there), the multi-pair Q8_0 tiles
+// those of q8_0_prefill_ring.hpp (7 - 48 % faster); this body serves them
 // otherwise.
 #include "common.hpp"
+#include "kquant_blocks.hpp"
 #include "q4_0.hpp"
 
 #include <type_traits>
@@ -483,6 +485,16 @@ hipError_t launch_prefill(const Problem& p) {
     // 128-row Q4_0 tiles: the ring body where the operands fit it.
     if constexpr (SPEC && T32 && KP > 1 && BM == 128 && !Q8)
         if (prefill_ring_supports(p)) return launch_prefill_ring(p, BM, BN, GATE_UP);
+    // Multi-pair Q8_0 tiles: the exact-integer tiles where the operands fit them
+    // (their own choice of rows per tile and K parts); without scratch for a
+    // choice of theirs under graph capture, this body.
+    if constexpr (SPEC && T32 && KP > 1 && Q8) {
+        if (kquant::prefill_supported(kquant::Fmt::Q8, p.x, p.w, p.M, p.N, p.K)) {
+            const hipError_t e = kquant::launch_prefill(kquant::Fmt::Q8, p.out == OutType::F16, p.x, p.w, p.y, p.M,
+                                                        p.N, p.K, p.stream);
+            if (e != hipErrorStreamCaptureUnsupported) return e;
+        }
+    }
     const uint32_t m_tiles = (p.M + BM - 1) / BM;
     const uint32_t n_tiles = (p.N + BN - 1) / BN;
     const uint64_t total64 = static_cast<uint64_t>(m_tiles) * n_tiles;

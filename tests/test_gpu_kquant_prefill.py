@@ -39,6 +39,8 @@ SHAPES = [
     (33, 3001, 768),
     (48, 4100, 512),
     (64, 7000, 1280),
+    # 96-row tiles
+    (300, 14336, 256),
 ]
 
 
