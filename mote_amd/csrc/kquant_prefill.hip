@@ -33,7 +33,7 @@
 // the slice's MFMAs cover the first LDS reads and decode of the next interval.
 // The groups' partial tiles meet in LDS (fixed order); K parts, used where the
 // tiles are too few for the chip, meet in scratch planes that
-// kq_parts_reduce_kernel adds in part order.
+// parts_reduce_kernel adds in part order.
 //
 // A result that is not finite is recomputed element by element with GGML's
 // values, as in the few-token tiles.
@@ -567,17 +567,6 @@ __global__ __launch_bounds__(256) void kq_sums_kernel(const uint16_t* __restrict
     dst[8] = __builtin_bit_cast(uint16_t, lo);
 }
 
-// y[i] = the sum of the K parts' planes at i, in part order, converted.
-template <typename OutT>
-__global__ __launch_bounds__(256) void kq_parts_reduce_kernel(const float* __restrict__ partial, uint32_t parts,
-                                                              uint64_t count, OutT* __restrict__ y) {
-    const uint64_t i = static_cast<uint64_t>(blockIdx.x) * 256 + threadIdx.x;
-    if (i >= count) return;
-    float v = partial[i];
-    for (uint32_t k = 1; k < parts; ++k) v += partial[k * count + i];
-    y[i] = to_out<OutT>(v);
-}
-
 template <Fmt F, int TM, int TN, int KG, typename OutT>
 hipError_t launch_tile(const uint16_t* x, const uint8_t* w, OutT* y, uint32_t M, uint32_t N, uint32_t K,
                        uint32_t parts, hipStream_t stream) {
@@ -633,7 +622,7 @@ hipError_t launch_tile(const uint16_t* x, const uint8_t* w, OutT* y, uint32_t M,
                            static_cast<float*>(nullptr), partial, M, N, K, m_tiles, n_tiles, part_blocks, total, per_xcd);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((kq_parts_reduce_kernel<OutT>), dim3(static_cast<uint32_t>((count + 255) / 256)), dim3(256), 0,
+    hipLaunchKernelGGL((parts_reduce_kernel<OutT>), dim3(static_cast<uint32_t>((count + 255) / 256)), dim3(256), 0,
                        stream, partial, parts, count, y);
     return hipGetLastError();
 }

@@ -71,6 +71,11 @@ bool prefill_supports(const Variant& v, const Problem& p);
 // tiles (128 x 256, 128 x 128; gate/up 128 x 128).
 bool prefill_ring_supports(const Problem& p);
 hipError_t launch_prefill_ring(const Problem& p, int bm, int bn, bool gate_up);
+// The linear on 128-row ring tiles over K parts where that is faster than bm x
+// bn tiles over all of K; hipErrorNotSupported, or hipErrorStreamCaptureUnsupported
+// (a stream under capture with too little scratch), with nothing queued, where
+// it is not or cannot.
+hipError_t launch_prefill_ring_parts(const Problem& p, int bm, int bn);
 
 hipError_t launch_zero_fill(void* y, uint64_t count, OutType out, hipStream_t stream);
 // K above 2^31 - 1 (p.K unused; the fused gate/up when p.w_up is set): 64-bit

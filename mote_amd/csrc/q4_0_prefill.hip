@@ -482,9 +482,17 @@ template <int BM, int BN, bool GATE_UP, bool Q8 = false, int WM = 2, bool T32 = 
           int KP = 1>
 hipError_t launch_prefill(const Problem& p) {
     if (p.K % (64u * KP) != 0) return hipErrorInvalidValue;
-    // 128-row Q4_0 tiles: the ring body where the operands fit it.
-    if constexpr (SPEC && T32 && KP > 1 && BM == 128 && !Q8)
-        if (prefill_ring_supports(p)) return launch_prefill_ring(p, BM, BN, GATE_UP);
+    // Q4_0 multi-pair tiles where the operands fit the ring body: over K parts
+    // if that is faster, else the 128-row tiles as they are.
+    if constexpr (SPEC && T32 && KP > 1 && !Q8) {
+        if (prefill_ring_supports(p)) {
+            if constexpr (!GATE_UP) {
+                const hipError_t e = launch_prefill_ring_parts(p, BM, BN);
+                if (e != hipErrorNotSupported && e != hipErrorStreamCaptureUnsupported) return e;
+            }
+            if constexpr (BM == 128) return launch_prefill_ring(p, BM, BN, GATE_UP);
+        }
+    }
     // Multi-pair Q8_0 tiles: the exact-integer tiles where the operands fit them
     // (their own choice of rows per tile and K parts); without scratch for a
     // choice of theirs under graph capture, this body.

@@ -39,6 +39,7 @@
 #include "q4_0.hpp"
 #include "tile_ops.hpp"
 
+#include <cmath>
 #include <type_traits>
 
 namespace mote::q4_0 {
@@ -71,10 +72,11 @@ __device__ __forceinline__ f16x8 dequant8_run(uint32_t q0, uint32_t q1, f16x2 d)
     return f16x8{v0.x, v0.y, v1.x, v1.y, v2.x, v2.y, v3.x, v3.y};
 }
 
-template <int TM, int WN, bool GATE_UP, typename OutT>
+template <int TM, int WN, bool GATE_UP, bool SK, typename OutT>
 __global__ __launch_bounds__(64 * WN * kGroups) void prefill_ring_kernel(
     const uint16_t* __restrict__ x, const uint8_t* __restrict__ wg, const uint8_t* __restrict__ wu,
-    OutT* __restrict__ y, uint32_t M, uint32_t N, uint32_t K, uint32_t m_tiles, uint32_t total, uint32_t per_xcd) {
+    OutT* __restrict__ y, float* __restrict__ partial, uint32_t M, uint32_t N, uint32_t K, uint32_t m_tiles,
+    uint32_t n_tiles, uint32_t part_pairs, uint32_t total, uint32_t per_xcd) {
     constexpr int W = WN * kGroups;
     constexpr int BM = 32 * TM;
     constexpr uint32_t BN = (GATE_UP ? 32 : 64) * WN;  // output columns
@@ -87,7 +89,8 @@ __global__ __launch_bounds__(64 * WN * kGroups) void prefill_ring_kernel(
 
     const uint32_t logical = (blockIdx.x % 8u) * per_xcd + blockIdx.x / 8u;
     if (logical >= total) return;
-    const uint32_t tile_n = logical / m_tiles, tile_m = logical - tile_n * m_tiles;
+    const uint32_t tile_m = logical % m_tiles, rest = logical / m_tiles;
+    const uint32_t tile_n = rest % n_tiles, part = rest / n_tiles;
     const uint32_t m0 = tile_m * BM, n0 = tile_n * BN;
     const int lane = static_cast<int>(threadIdx.x) & 63;
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
@@ -95,10 +98,11 @@ __global__ __launch_bounds__(64 * WN * kGroups) void prefill_ring_kernel(
     const int lr = lane & 31, lc = lane >> 5;
     const uint32_t nsuper = K >> 8;
     const uint32_t row_bytes = nsuper * 144u;
-    // this half's super-pairs: [s0, s0 + ns)
-    const uint32_t per = (nsuper + kGroups - 1) / kGroups;
-    const uint32_t s0 = min(static_cast<uint32_t>(kg) * per, nsuper);
-    const uint32_t ns = min(per, nsuper - s0);
+    // this half of the part's super-pairs: [s0, s0 + ns)
+    const uint32_t p0 = part * part_pairs, p1 = min(p0 + part_pairs, nsuper);
+    const uint32_t per = (p1 - p0 + kGroups - 1) / kGroups;
+    const uint32_t s0 = min(p0 + static_cast<uint32_t>(kg) * per, p1);
+    const uint32_t ns = min(per, p1 - s0);
     const uint32_t last = ns * 4 - 1;  // (no loads where ns is 0)
 
     const Buffer xsrc = buffer_at(reinterpret_cast<const uint8_t*>(x) + (static_cast<size_t>(m0) * K + s0 * 256u) * 2);
@@ -327,17 +331,27 @@ __global__ __launch_bounds__(64 * WN * kGroups) void prefill_ring_kernel(
                 const uint32_t m = m0 + (kg * H + i) * 32 + 8 * (k / 4) + 4 * lc + k % 4;
                 float v = acc[i][j][k];
                 if constexpr (GATE_UP) v = silu(v) * acc[i][1][k];
-                if (m < M) y[static_cast<size_t>(m) * N + n] = to_out<OutT>(v);
+                if (m >= M) continue;
+                if constexpr (SK)  // this K part's plane of the partial sums
+                    partial[(static_cast<size_t>(part) * M + m) * N + n] = v;
+                else
+                    y[static_cast<size_t>(m) * N + n] = to_out<OutT>(v);
             }
     }
 }
 
+// parts > 1 (linear): K parts in planes of the stream's scratch, added by a
+// second kernel.  hipErrorStreamCaptureUnsupported, with nothing queued, when
+// the stream is under capture and holds too little of it.
 template <int TM, int WN, bool GATE_UP>
-hipError_t launch_ring(const Problem& p) {
+hipError_t launch_ring(const Problem& p, uint32_t parts) {
     constexpr uint32_t BM = 32 * TM, BN = (GATE_UP ? 32 : 64) * WN;
     const uint32_t m_tiles = (p.M + BM - 1) / BM;
     const uint32_t n_tiles = (p.N + BN - 1) / BN;
-    const uint64_t total64 = static_cast<uint64_t>(m_tiles) * n_tiles;
+    const uint32_t nsuper = p.K / 256u;
+    const uint32_t part_pairs = (nsuper + parts - 1) / parts;
+    parts = (nsuper + part_pairs - 1) / part_pairs;
+    const uint64_t total64 = static_cast<uint64_t>(m_tiles) * n_tiles * parts;
     if (total64 > 0x7ffffff0ull) return hipErrorInvalidConfiguration;
     const uint32_t total = static_cast<uint32_t>(total64);
     const uint32_t per_xcd = (total + 7u) / 8u;
@@ -345,12 +359,42 @@ hipError_t launch_ring(const Problem& p) {
     const auto* x = static_cast<const uint16_t*>(p.x);
     const auto* wg = static_cast<const uint8_t*>(p.w);
     const auto* wu = static_cast<const uint8_t*>(p.w_up);
+    if constexpr (!GATE_UP) {
+        if (parts > 1) {
+            const uint64_t count = static_cast<uint64_t>(p.M) * p.N;
+            const size_t need = kSplitKCounterBytes + count * parts * sizeof(float);
+            ScratchPool::Lease lease;  // holds the scratch until both kernels are queued
+            const hipError_t a = acquire_scratch(p.stream, need, &lease);
+            if (a != hipSuccess) return a;
+            auto* const base = static_cast<uint8_t*>(lease.ptr());
+            if (lease.fresh()) {  // the arrival counters every user of the pool leaves zero
+                const hipError_t z = launch_zero_fill(base, kSplitKCounterBytes / 4, OutType::F32, p.stream);
+                if (z != hipSuccess) return z;
+            }
+            auto* planes = reinterpret_cast<float*>(base + kSplitKCounterBytes);
+            hipLaunchKernelGGL((prefill_ring_kernel<TM, WN, false, true, float>), grid, block, 0, p.stream, x, wg, wu,
+                               static_cast<float*>(nullptr), planes, p.M, p.N, p.K, m_tiles, n_tiles, part_pairs, total,
+                               per_xcd);
+            const hipError_t e = hipGetLastError();
+            if (e != hipSuccess) return e;
+            const dim3 rgrid(static_cast<uint32_t>((count + 255) / 256)), rblock(256);
+            if (p.out == OutType::F32)
+                hipLaunchKernelGGL((parts_reduce_kernel<float>), rgrid, rblock, 0, p.stream, planes, parts, count,
+                                   static_cast<float*>(p.y));
+            else
+                hipLaunchKernelGGL((parts_reduce_kernel<_Float16>), rgrid, rblock, 0, p.stream, planes, parts, count,
+                                   static_cast<_Float16*>(p.y));
+            return hipGetLastError();
+        }
+    }
     if (p.out == OutType::F32)
-        hipLaunchKernelGGL((prefill_ring_kernel<TM, WN, GATE_UP, float>), grid, block, 0, p.stream, x, wg, wu,
-                           static_cast<float*>(p.y), p.M, p.N, p.K, m_tiles, total, per_xcd);
+        hipLaunchKernelGGL((prefill_ring_kernel<TM, WN, GATE_UP, false, float>), grid, block, 0, p.stream, x, wg, wu,
+                           static_cast<float*>(p.y), static_cast<float*>(nullptr), p.M, p.N, p.K, m_tiles, n_tiles,
+                           part_pairs, total, per_xcd);
     else
-        hipLaunchKernelGGL((prefill_ring_kernel<TM, WN, GATE_UP, _Float16>), grid, block, 0, p.stream, x, wg, wu,
-                           static_cast<_Float16*>(p.y), p.M, p.N, p.K, m_tiles, total, per_xcd);
+        hipLaunchKernelGGL((prefill_ring_kernel<TM, WN, GATE_UP, false, _Float16>), grid, block, 0, p.stream, x, wg, wu,
+                           static_cast<_Float16*>(p.y), static_cast<float*>(nullptr), p.M, p.N, p.K, m_tiles, n_tiles,
+                           part_pairs, total, per_xcd);
     return hipGetLastError();
 }
 
@@ -363,10 +407,57 @@ bool prefill_ring_supports(const Problem& p) {
     return p.K % 256 == 0 && p.K > 0 && p.K < (1u << 20) && on16(p.x) && on16(p.w) && on16(p.w_up);
 }
 
+// Where K is long and the tiles are few, K parts of 128-row tiles fill the chip:
+// the least of rounds of one workgroup per CU x (5 us + super-pairs of a part x
+// their time) + reduction, against a bm x bn tiling's own rounds.  Fits to
+// MI355X timings in us per super-pair: 3.6 (128 x 256), 2.2 (128 x 128), the
+// staging-wave tiles 1.25 (64 x 128), 0.85 (64 x 64); the reduction 3 us and the
+// planes written and read once at 4 TB/s, planes up to 48 MiB (inside the
+// scratch a library stream starts with).  Measured against the tiles it
+// replaced (us): 128 / 256 x 14 336 x 4096 51.0 -> 30.1, 56.3 -> 43.2; 400 x 14
+// 336 x 5120 118 -> 82; 100 x 13 824 x 5120 49.4 -> 31.7; 65 x 28 672 x 8192 114
+// -> 73; 32 x 11 008 x 4096 39.4 -> 22.8.  Not where the caller brings scratch
+// of its own (the allocation-free entry point): calls that may overlap share it.
+hipError_t launch_prefill_ring_parts(const Problem& p, int bm, int bn) {
+    if (p.scratch != nullptr) return hipErrorNotSupported;
+    static const int cus = [] {
+        int dev = 0, n = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
+            n = 256;
+        return n;
+    }();
+    const uint32_t nsuper = p.K / 256u;
+    auto cost = [&](int tm, int tn, double each, uint32_t parts) {
+        const double tiles = static_cast<double>((p.M + tm - 1u) / tm) * ((p.N + tn - 1u) / tn) * parts;
+        double us = std::ceil(tiles / cus) * (5.0 + each * ((nsuper + parts - 1) / parts));
+        if (parts > 1) us += 3.0 + 8.0 * p.M * p.N * parts / 4e6;
+        return us;
+    };
+    const double own = cost(bm, bn, bm == 128 ? (bn == 256 ? 3.6 : 2.2) : (bn == 128 ? 1.25 : 0.85), 1);
+    double best = 0.92 * own;
+    int tile = 0;
+    uint32_t parts = 1;
+    for (int tn = 256; tn >= 128; tn /= 2)
+        for (uint32_t k = 1; k <= 8 && k * 2 <= nsuper + 1; ++k) {
+            if (k > 1 && 4.0 * p.M * p.N * k > 48.0 * 1048576.0) break;
+            const double us = cost(128, tn, tn == 256 ? 3.6 : 2.2, k);
+            if (us < best) {
+                best = us;
+                tile = tn;
+                parts = k;
+            }
+        }
+    if (tile == 0) return hipErrorNotSupported;
+    return tile == 256 ? launch_ring<4, 4, false>(p, parts) : launch_ring<4, 2, false>(p, parts);
+}
+
 hipError_t launch_prefill_ring(const Problem& p, int bm, int bn, bool gate_up) {
     if (bm != 128) return hipErrorInvalidValue;
-    if (gate_up) return bn == 128 ? launch_ring<4, 4, true>(p) : hipErrorInvalidValue;
-    return bn == 256 ? launch_ring<4, 4, false>(p) : bn == 128 ? launch_ring<4, 2, false>(p) : hipErrorInvalidValue;
+    if (gate_up) return bn == 128 ? launch_ring<4, 4, true>(p, 1) : hipErrorInvalidValue;
+    return bn == 256   ? launch_ring<4, 4, false>(p, 1)
+           : bn == 128 ? launch_ring<4, 2, false>(p, 1)
+                       : hipErrorInvalidValue;
 }
 
 }  // namespace mote::q4_0

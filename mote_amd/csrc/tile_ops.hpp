@@ -1,5 +1,5 @@
 // What the direct-to-LDS prefill tiles share: counted waits, the 32 x 32 x 16
-// MFMA, loads to LDS, packed binary16 helpers.
+// MFMA, loads to LDS, packed binary16 helpers, the sum over K parts.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -53,6 +53,18 @@ __device__ __forceinline__ f16x2 both(f16x2 v, bool high) {
 __device__ __forceinline__ f16x2 both(_Float16 v) { return f16x2{v, v}; }
 __device__ __forceinline__ f16x8 join(f16x2 a, f16x2 b, f16x2 c, f16x2 d) {
     return f16x8{a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y};
+}
+
+
+// y[i] = the sum of the K parts' planes at i, in part order, converted.
+template <typename OutT>
+__global__ __launch_bounds__(256) void parts_reduce_kernel(const float* __restrict__ partial, uint32_t parts,
+                                                              uint64_t count, OutT* __restrict__ y) {
+    const uint64_t i = static_cast<uint64_t>(blockIdx.x) * 256 + threadIdx.x;
+    if (i >= count) return;
+    float v = partial[i];
+    for (uint32_t k = 1; k < parts; ++k) v += partial[k * count + i];
+    y[i] = to_out<OutT>(v);
 }
 
 }  // namespace

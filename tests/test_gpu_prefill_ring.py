@@ -69,6 +69,15 @@ def test_ring_matches_staging_body(stream, variant, m, n, k, scales):
         assert np.all(np.abs(got - want) <= tol), f"{variant} {m}x{n}x{k}: {float(np.abs(got - want).max())} > {bound}"
 
 
+@pytest.mark.parametrize("variant", ["mfma_x32s_m64_n64_w2_k4", "mfma_x32s_m64_n128_w1_k4", "mfma_x32s_m128_n128_w1_k2"])
+@pytest.mark.parametrize("m,n,k", [(70, 96, 14336), (130, 129, 9472), (33, 257, 11008)])
+@pytest.mark.parametrize("scales", ["ordinary", "wide"])
+def test_k_parts_match_staging_body(stream, variant, m, n, k, scales):
+    """Few tiles and long K: 128-row ring tiles over K parts (a short last
+    part at K = 9472 and 11 008)."""
+    test_ring_matches_staging_body(stream, variant, m, n, k, scales)
+
+
 @pytest.mark.parametrize("m,n,k", [(128, 128, 256), (129, 127, 768), (200, 200, 1024)])
 def test_gate_up_ring_matches_staging_body(stream, m, n, k):
     d = ops.Q4_0Dispatch()
