@@ -1,7 +1,7 @@
 // K-quant (and Q8_0) linear over many tokens on the matrix cores, y[M, N] = x[M, K] (f16)
 // . W[N, K]^T with Q4_K or Q6_K weights (layouts in kquant.hip).
 //
-// A workgroup of 4 KG waves computes a 32 TM x 128 tile of y over one part of
+// A workgroup of 4 x 2 waves computes a 32 TM x 128 tile of y over one part of
 // K.  Wave (kg, wn) owns 32 weight rows (columns 32 wn .. of the tile) for
 // group kg's share of the part's super-blocks, TM tiles of
 // v_mfma_f32_32x32x16_f16 with the activations as the A operand.  Lane (r, c)
@@ -63,7 +63,8 @@ namespace {
 // 16-byte vector at a 2-byte-aligned address (one unaligned dwordx4 load).
 typedef uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
 
-constexpr int kTileWaves = 4;                 // waves along N
+constexpr int kTileWaves = 4;   // waves along N
+constexpr int kTileGroups = 2;  // groups of them along K
 
 // Keeps a converted scale in f32: as mixed-precision fmas from the binary16
 // word, two of which in a row need a wait state, the folds took twice as long.
@@ -104,11 +105,12 @@ struct Scales<Fmt::Q6K> {
     float d;
 };
 
-template <Fmt F, int TM, int TN, int KG, bool SK, typename OutT>
-__global__ __launch_bounds__(64 * kTileWaves * KG) void kq_prefill_kernel(
+template <Fmt F, int TM, bool SK, typename OutT>
+__global__ __launch_bounds__(64 * kTileWaves * kTileGroups) void kq_prefill_kernel(
     const uint16_t* __restrict__ x, const uint8_t* __restrict__ w, const uint16_t* __restrict__ sums,
     OutT* __restrict__ y, float* __restrict__ partial, uint32_t M, uint32_t N, uint32_t K, uint32_t m_tiles,
     uint32_t n_tiles, uint32_t part_blocks, uint32_t total, uint32_t per_xcd) {
+    constexpr int KG = kTileGroups, TN = 1;  // TN: 32-row weight tiles per wave (two fill 512 registers)
     constexpr int BM = 32 * TM;
     constexpr uint32_t BN = 32 * TN * kTileWaves;
     constexpr int kUnit = BM * 128;            // LDS bytes of one group's activations of an interval
@@ -120,9 +122,8 @@ __global__ __launch_bounds__(64 * kTileWaves * KG) void kq_prefill_kernel(
     // result at K = 4096, as the few-token tiles, against 1.45e-7).
     constexpr int NC = NB == 2 && TM == 2 ? 2 : 1;
     constexpr uint32_t BB = block_bytes<F>();
-    static_assert(KG == 1 || KG == 2, "the groups hand half of the output tiles over");
     constexpr int kRing = kSlots * KG * kUnit;
-    constexpr int kReduce = KG == 1 ? 0 : kTileWaves * KG * ((TM + 1) / 2) * TN * 4096;
+    constexpr int kReduce = kTileWaves * KG * ((TM + 1) / 2) * TN * 4096;
     __shared__ __attribute__((aligned(1024))) uint8_t lds[kRing > kReduce ? kRing : kReduce];
 
     const uint32_t logical = (blockIdx.x % 8u) * per_xcd + blockIdx.x / 8u;
@@ -481,44 +482,42 @@ __global__ __launch_bounds__(64 * kTileWaves * KG) void kq_prefill_kernel(
 
     // Two groups: the first keeps row tiles 0 .. H - 1, the second the others;
     // each hands over the rest.
-    constexpr int H = KG == 1 ? TM : (TM + 1) / 2;
+    constexpr int H = (TM + 1) / 2;
     const int kept = kg == 0 ? H : TM - H, tile0 = kg == 0 ? 0 : H;
-    if constexpr (KG == 2) {
-        float* red = reinterpret_cast<float*>(lds);
-        auto slot = [&](int wv, int i, int j, int r) { return red + (((wv * H + i) * TN + j) * 4 + r) * 256 + lane * 4; };
-        auto give = [&](const f32x16& v, int i, int j) {
+    float* red = reinterpret_cast<float*>(lds);
+    auto slot = [&](int wv, int i, int j, int r) { return red + (((wv * H + i) * TN + j) * 4 + r) * 256 + lane * 4; };
+    auto give = [&](const f32x16& v, int i, int j) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-                *reinterpret_cast<f32x4*>(slot(wave, i, j, r)) = f32x4{v[4 * r], v[4 * r + 1], v[4 * r + 2], v[4 * r + 3]};
-        };
-        if (kg == 0) {
+        for (int r = 0; r < 4; ++r)
+            *reinterpret_cast<f32x4*>(slot(wave, i, j, r)) = f32x4{v[4 * r], v[4 * r + 1], v[4 * r + 2], v[4 * r + 3]};
+    };
+    if (kg == 0) {
 #pragma unroll
-            for (int i = 0; i < TM - H; ++i)
+        for (int i = 0; i < TM - H; ++i)
 #pragma unroll
-                for (int j = 0; j < TN; ++j) give(acc[H + i][j], i, j);
-        } else {
+            for (int j = 0; j < TN; ++j) give(acc[H + i][j], i, j);
+    } else {
 #pragma unroll
-            for (int i = 0; i < H; ++i)
+        for (int i = 0; i < H; ++i)
 #pragma unroll
-                for (int j = 0; j < TN; ++j) {
-                    give(acc[i][j], i, j);
-                    if (H + i < TM) acc[i][j] = acc[H + i][j];
-                }
-        }
-        __syncthreads();
-        const int other = wave ^ kTileWaves;
+            for (int j = 0; j < TN; ++j) {
+                give(acc[i][j], i, j);
+                if (H + i < TM) acc[i][j] = acc[H + i][j];
+            }
+    }
+    __syncthreads();
+    const int other = wave ^ kTileWaves;
 #pragma unroll
-        for (int i = 0; i < H; ++i) {
-            if (i >= kept) break;  // uniform
+    for (int i = 0; i < H; ++i) {
+        if (i >= kept) break;  // uniform
 #pragma unroll
-            for (int j = 0; j < TN; ++j)
+        for (int j = 0; j < TN; ++j)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const f32x4 v = *reinterpret_cast<const f32x4*>(slot(other, i, j, r));
+            for (int r = 0; r < 4; ++r) {
+                const f32x4 v = *reinterpret_cast<const f32x4*>(slot(other, i, j, r));
 #pragma unroll
-                    for (int k = 0; k < 4; ++k) acc[i][j][4 * r + k] += v[k];
-                }
-        }
+                for (int k = 0; k < 4; ++k) acc[i][j][4 * r + k] += v[k];
+            }
     }
     // Lane (r, c) holds column r of each tile, rows 8 (k / 4) + 4 c + k % 4.
 #pragma unroll
@@ -567,11 +566,11 @@ __global__ __launch_bounds__(256) void kq_sums_kernel(const uint16_t* __restrict
     dst[8] = __builtin_bit_cast(uint16_t, lo);
 }
 
-template <Fmt F, int TM, int TN, int KG, typename OutT>
+template <Fmt F, int TM, typename OutT>
 hipError_t launch_tile(const uint16_t* x, const uint8_t* w, OutT* y, uint32_t M, uint32_t N, uint32_t K,
                        uint32_t parts, hipStream_t stream) {
     const uint32_t nb = K / kSuper;
-    const uint32_t m_tiles = (M + 32 * TM - 1) / (32 * TM), n_tiles = (N + 32 * TN * kTileWaves - 1) / (32 * TN * kTileWaves);
+    const uint32_t m_tiles = (M + 32 * TM - 1) / (32 * TM), n_tiles = (N + 32 * kTileWaves - 1) / (32 * kTileWaves);
     const uint32_t part_blocks = (nb + parts - 1) / parts;
     parts = (nb + part_blocks - 1) / part_blocks;
     const uint64_t total64 = static_cast<uint64_t>(m_tiles) * n_tiles * parts;
@@ -604,13 +603,13 @@ hipError_t launch_tile(const uint16_t* x, const uint8_t* w, OutT* y, uint32_t M,
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
-    const dim3 grid(per_xcd * 8), block(64 * kTileWaves * KG);
+    const dim3 grid(per_xcd * 8), block(64 * kTileWaves * kTileGroups);
     if (parts == 1) {
         if constexpr (F == Fmt::Q8)
             hipLaunchKernelGGL((q8_prefill_kernel<TM, false, OutT>), grid, block, 0, stream, x, w, y, partial, M, N, K,
                                m_tiles, n_tiles, part_blocks, total, per_xcd);
         else
-            hipLaunchKernelGGL((kq_prefill_kernel<F, TM, TN, KG, false, OutT>), grid, block, 0, stream, x, w, sums, y,
+            hipLaunchKernelGGL((kq_prefill_kernel<F, TM, false, OutT>), grid, block, 0, stream, x, w, sums, y,
                                partial, M, N, K, m_tiles, n_tiles, part_blocks, total, per_xcd);
         return hipGetLastError();
     }
@@ -618,7 +617,7 @@ hipError_t launch_tile(const uint16_t* x, const uint8_t* w, OutT* y, uint32_t M,
         hipLaunchKernelGGL((q8_prefill_kernel<TM, true, float>), grid, block, 0, stream, x, w,
                            static_cast<float*>(nullptr), partial, M, N, K, m_tiles, n_tiles, part_blocks, total, per_xcd);
     else
-        hipLaunchKernelGGL((kq_prefill_kernel<F, TM, TN, KG, true, float>), grid, block, 0, stream, x, w, sums,
+        hipLaunchKernelGGL((kq_prefill_kernel<F, TM, true, float>), grid, block, 0, stream, x, w, sums,
                            static_cast<float*>(nullptr), partial, M, N, K, m_tiles, n_tiles, part_blocks, total, per_xcd);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
@@ -688,9 +687,9 @@ hipError_t launch(const void* x, const void* w, void* y, uint32_t M, uint32_t N,
     const auto* wp = static_cast<const uint8_t*>(w);
     auto* yp = static_cast<OutT*>(y);
     auto run = [&](const Plan& p) {
-        return p.tm == 4   ? launch_tile<F, 4, 1, 2, OutT>(xp, wp, yp, M, N, K, p.parts, stream)
-               : p.tm == 3 ? launch_tile<F, 3, 1, 2, OutT>(xp, wp, yp, M, N, K, p.parts, stream)
-                           : launch_tile<F, 2, 1, 2, OutT>(xp, wp, yp, M, N, K, p.parts, stream);
+        return p.tm == 4   ? launch_tile<F, 4, OutT>(xp, wp, yp, M, N, K, p.parts, stream)
+               : p.tm == 3 ? launch_tile<F, 3, OutT>(xp, wp, yp, M, N, K, p.parts, stream)
+                           : launch_tile<F, 2, OutT>(xp, wp, yp, M, N, K, p.parts, stream);
     };
     const Plan plan = choose<F>(M, N, K);
     const hipError_t e = run(plan);
