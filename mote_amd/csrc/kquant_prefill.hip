@@ -621,8 +621,7 @@ hipError_t launch_tile(const uint16_t* x, const uint8_t* w, OutT* y, uint32_t M,
                            static_cast<float*>(nullptr), partial, M, N, K, m_tiles, n_tiles, part_blocks, total, per_xcd);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((parts_reduce_kernel<OutT>), dim3(static_cast<uint32_t>((count + 255) / 256)), dim3(256), 0,
-                       stream, partial, parts, count, y);
+    hipLaunchKernelGGL((parts_reduce_kernel<OutT>), dim3(parts_reduce_grid(count)), dim3(256), 0, stream, partial, parts, count, y);
     return hipGetLastError();
 }
 

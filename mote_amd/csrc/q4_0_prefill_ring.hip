@@ -377,7 +377,7 @@ hipError_t launch_ring(const Problem& p, uint32_t parts) {
                                per_xcd);
             const hipError_t e = hipGetLastError();
             if (e != hipSuccess) return e;
-            const dim3 rgrid(static_cast<uint32_t>((count + 255) / 256)), rblock(256);
+            const dim3 rgrid(parts_reduce_grid(count)), rblock(256);
             if (p.out == OutType::F32)
                 hipLaunchKernelGGL((parts_reduce_kernel<float>), rgrid, rblock, 0, p.stream, planes, parts, count,
                                    static_cast<float*>(p.y));

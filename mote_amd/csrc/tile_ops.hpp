@@ -56,16 +56,36 @@ __device__ __forceinline__ f16x8 join(f16x2 a, f16x2 b, f16x2 c, f16x2 d) {
 }
 
 
-// y[i] = the sum of the K parts' planes at i, in part order, converted.
+// y[i] = the sum of the K parts' planes at i, in part order, converted; four
+// consecutive outputs per thread (16-byte loads and stores at the planes' 4- and
+// the output's element alignment; against one per thread, whole calls: 256 x 14
+// 336 x 4096 Q4_0 43.7 -> 43.0 us, Q6_K 62.9 -> 62.0, Q8_0 48.5 -> 47.8).
+typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef _Float16 f16x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
+
 template <typename OutT>
 __global__ __launch_bounds__(256) void parts_reduce_kernel(const float* __restrict__ partial, uint32_t parts,
-                                                              uint64_t count, OutT* __restrict__ y) {
-    const uint64_t i = static_cast<uint64_t>(blockIdx.x) * 256 + threadIdx.x;
-    if (i >= count) return;
-    float v = partial[i];
-    for (uint32_t k = 1; k < parts; ++k) v += partial[k * count + i];
-    y[i] = to_out<OutT>(v);
+                                                           uint64_t count, OutT* __restrict__ y) {
+    const uint64_t i = (static_cast<uint64_t>(blockIdx.x) * 256 + threadIdx.x) * 4;
+    if (i + 4 <= count) {
+        f32x4 v = *reinterpret_cast<const f32x4_a4*>(partial + i);
+        for (uint32_t k = 1; k < parts; ++k) v += *reinterpret_cast<const f32x4_a4*>(partial + k * count + i);
+        if constexpr (sizeof(OutT) == 4)
+            *reinterpret_cast<f32x4_a4*>(y + i) = v;
+        else
+            *reinterpret_cast<f16x4_a2*>(y + i) =
+                f16x4_a2{to_out<OutT>(v.x), to_out<OutT>(v.y), to_out<OutT>(v.z), to_out<OutT>(v.w)};
+        return;
+    }
+    for (uint64_t e = i; e < count; ++e) {
+        float v = partial[e];
+        for (uint32_t k = 1; k < parts; ++k) v += partial[k * count + e];
+        y[e] = to_out<OutT>(v);
+    }
 }
+
+// Its grid: 1024 outputs per workgroup.
+inline uint32_t parts_reduce_grid(uint64_t count) { return static_cast<uint32_t>((count + 1023) / 1024); }
 
 }  // namespace
 }  // namespace mote
