@@ -27,8 +27,21 @@ extern "C" {
  * crates/mote-backend-hip/src/ffi.rs:42-61.  Raw hipError_t; -1 for a null
  * out-parameter.  mote_hip_stream_create also allocates the stream's 64 MiB
  * split-K scratch (so split-K linears on it allocate nothing up to that
- * size); mote_hip_stream_destroy does not wait for the stream, and frees that
- * scratch once the work queued before it has completed. */
+ * size) and, where memory allows, 64 MiB of prompt scratch;
+ * mote_hip_stream_destroy does not wait for the stream, and frees the scratch
+ * once the work queued before it has completed.
+ *
+ * Prompt scratch: linears on the many-token tiles (more than 64 tokens, and
+ * fewer where those tiles are the faster ones) never allocate.  On a stream made
+ * by mote_hip_stream_create, outside graph capture, they may divide K over
+ * workgroups whose partial sums meet in the stream's prompt scratch (Q4_K keeps
+ * its activation sums there too).  Under capture, and on any other stream, they
+ * use no scratch: Q4_K, Q6_K, Q8_0 and Q4_0 prompts then run over all of K in one
+ * workgroup per tile, equal to the tolerance but not bit for bit to the divided
+ * call, and up to twice as slow where K is long and the tiles are few.  So a
+ * graph of such calls holds no memory of the library's: it may be replayed on
+ * any stream, beside other graphs and eager calls, and after its capture stream
+ * is gone. */
 int mote_hip_get_device_count(int* count);
 int mote_hip_set_device(int ordinal);
 int mote_hip_malloc(void** pointer, size_t bytes);
@@ -65,7 +78,8 @@ int mote_hip_quantized_linear_q4_0_f32(const void* input, const void* weights, v
 /* [new] No counterpart in the reference.  mote_hip_quantized_linear_q4_0_f32
  * for callers that cannot allocate device memory (code under HIP graph
  * capture, serving loops or harnesses that forbid hipMalloc): the same
- * arguments, checks, statuses, plans and kernels, but the split-K partial
+ * arguments, checks, statuses, plans and kernels (prompts in the stream's
+ * prompt scratch included), but the split-K partial
  * tiles (1-64 tokens where K exceeds one K slice) go to the library's static
  * 16 MiB device array instead of a per-stream buffer the library allocates;
  * nothing is allocated on any call.  Every call on one GPU shares that

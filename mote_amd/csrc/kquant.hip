@@ -1468,7 +1468,7 @@ hipError_t launch_gemv(const void* x, const void* w, void* y, uint32_t M, uint32
                        hipStream_t stream) {
     if (prefill_supported(F, x, w, M, N, K)) {
         const hipError_t e = launch_prefill(F, std::is_same_v<OutT, _Float16>, x, w, y, M, N, K, stream);
-        if (e != hipErrorStreamCaptureUnsupported) return e;
+        if (e != hipErrorNotSupported) return e;  // else: up to 64 tokens on a stream without scratch
     }
     if (kq_mfma_supported<F>(x, w, M, K)) {
         const hipError_t e = launch_kq_mfma<F, OutT>(x, w, y, M, N, K, stream);

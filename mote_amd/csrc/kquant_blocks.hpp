@@ -124,9 +124,9 @@ __device__ inline float kq_exact_thread(const uint8_t* row, const uint16_t* xrow
 int device_cus();
 
 // The linear over many tokens on the matrix cores (kquant_prefill.hip):
-// whether it takes the call, and the call (F16: binary16 result).
-// hipErrorStreamCaptureUnsupported, with nothing queued, when its scratch would
-// have to grow under graph capture.
+// whether it takes the call, and the call (F16: binary16 result).  On a stream
+// without prompt scratch (q4_0.hpp) it runs over all of K at once, except for up
+// to 64 tokens: hipErrorNotSupported, with nothing queued.
 bool prefill_supported(Fmt f, const void* x, const void* w, uint32_t M, uint32_t N, uint32_t K);
 hipError_t launch_prefill(Fmt f, bool f16_out, const void* x, const void* w, void* y, uint32_t M, uint32_t N,
                           uint32_t K, hipStream_t stream);

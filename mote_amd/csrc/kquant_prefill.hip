@@ -33,7 +33,11 @@
 // the slice's MFMAs cover the first LDS reads and decode of the next interval.
 // The groups' partial tiles meet in LDS (fixed order); K parts, used where the
 // tiles are too few for the chip, meet in scratch planes that
-// parts_reduce_kernel adds in part order.
+// parts_reduce_kernel adds in part order.  Planes and sums live in the stream's
+// prompt scratch (q4_0.hpp).  Without it there is one part, and Q4_K's sums are
+// added up from the operands in registers, 16 elements per lane, two MFMAs per
+// super-block (OWN): 32 dot products per tile and quarter in every wave, which 96-
+// and 64-row tiles have registers for.  512 x 4096 x 14 336 122 us against 85.
 //
 // A result that is not finite is recomputed element by element with GGML's
 // values, as in the few-token tiles.
@@ -105,7 +109,9 @@ struct Scales<Fmt::Q6K> {
     float d;
 };
 
-template <Fmt F, int TM, bool SK, typename OutT>
+// OWN (Q4_K): each wave adds up the sub-blocks' activations itself instead of
+// reading kq_sums_kernel's.
+template <Fmt F, int TM, bool SK, typename OutT, bool OWN = false>
 __global__ __launch_bounds__(64 * kTileWaves * kTileGroups) void kq_prefill_kernel(
     const uint16_t* __restrict__ x, const uint8_t* __restrict__ w, const uint16_t* __restrict__ sums,
     OutT* __restrict__ y, float* __restrict__ partial, uint32_t M, uint32_t N, uint32_t K, uint32_t m_tiles,
@@ -349,7 +355,7 @@ __global__ __launch_bounds__(64 * kTileWaves * kTileGroups) void kq_prefill_kern
     // halves of the sub-block sums.
     f16x8 sx[TM];
     auto load_sums = [&](uint32_t s) {
-        if constexpr (F == Fmt::Q4K) {
+        if constexpr (F == Fmt::Q4K && !OWN) {
             const uint16_t* src = sums + static_cast<size_t>(b0 + s) * 16 + 8 * lc;
 #pragma unroll
             for (int i = 0; i < TM; ++i)
@@ -366,7 +372,7 @@ __global__ __launch_bounds__(64 * kTileWaves * kTileGroups) void kq_prefill_kern
     };
     auto minimum = [&](auto pc, auto ic, auto slice) {
         constexpr int I = 4 * (decltype(pc)::value - 2) + decltype(ic)::value;
-        if constexpr (F == Fmt::Q4K) {
+        if constexpr (F == Fmt::Q4K && !OWN) {
             if constexpr (I >= 0 && I < TM) {
                 f32x16 mn[TN];
 #pragma unroll
@@ -383,11 +389,53 @@ __global__ __launch_bounds__(64 * kTileWaves * kTileGroups) void kq_prefill_kern
             slice();
         }
     };
+    // OWN: the lane's part of sub-block j's sum, its elements 16 c .. 16 c + 15, as
+    // binary16 hi and lo halves at j of 8 (in each c: the MFMAs add both), from
+    // the slices' operands; after the last slice the minimum term of every tile.
+    float run[TM];
+    uint32_t own[TM][2][4];
+    auto add_slice = [&](auto pc, auto ic) {
+        if constexpr (OWN) {
+            constexpr int P = decltype(pc)::value, S = decltype(ic)::value, h = S / 2, u = S % 2;
+            const uint32_t one = 0x3C003C00u;
+#pragma unroll
+            for (int i = 0; i < TM; ++i) {
+                const u32x4 v = __builtin_bit_cast(u32x4, a[u][i]);
+                const float s = dot2(v.w, one, dot2(v.z, one, dot2(v.y, one, dot2(v.x, one, u ? run[i] : 0.0f))));
+                if constexpr (u == 0) {
+                    run[i] = s;
+                } else {
+                    const _Float16 hi = static_cast<_Float16>(s);
+                    const _Float16 lo = static_cast<_Float16>(s - static_cast<float>(hi));
+                    const uint32_t b[2] = {__builtin_bit_cast(uint16_t, hi), __builtin_bit_cast(uint16_t, lo)};
+#pragma unroll
+                    for (int k = 0; k < 2; ++k) own[i][k][P] = h ? own[i][k][P] | (b[k] << 16) : b[k];
+                }
+            }
+        }
+    };
+    auto own_minimum = [&]() {
+        if constexpr (OWN) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    f32x16 mn = zero;
+#pragma unroll
+                    for (int k = 0; k < 2; ++k) {
+                        const u32x4 v = {own[i][k][0], own[i][k][1], own[i][k][2], own[i][k][3]};
+                        mn = mfma32(__builtin_bit_cast(f16x8, v), mins(j), mn);
+                    }
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) acc[i][j][r] = __builtin_fmaf(-sl[j].dmin, mn[r], acc[i][j][r]);
+                }
+        }
+    };
     // Loads a wave issues behind interval t's activations of four intervals on:
     // quants, the sums (p = 0), the next header (p = 2).
     constexpr bool kQ4 = F == Fmt::Q4K;
     constexpr int kHalf = (kQ4 ? 2 : 3) * TN;  // a half block's quants
-    constexpr int kBehind[4] = {kQ4 ? TM : 0, kHalf, kQ4 ? TN : 2 * TN, kHalf};
+    constexpr int kBehind[4] = {kQ4 && !OWN ? TM : 0, kHalf, kQ4 ? TN : 2 * TN, kHalf};
     using I0 = std::integral_constant<int, 0>;
     using I1 = std::integral_constant<int, 1>;
     using I2 = std::integral_constant<int, 2>;
@@ -425,18 +473,21 @@ __global__ __launch_bounds__(64 * kTileWaves * kTileGroups) void kq_prefill_kern
             read_a(P, 1, a[1]);
             minimum(pc, I0{}, [&] {
                 if constexpr (P == 0) multiply_first(); else multiply(I0{});
+                add_slice(pc, I0{});
                 decode(pc, I1{}, b[1]);
             });
             order_fence();
             read_a(P, 2, a[0]);
             minimum(pc, I1{}, [&] {
                 multiply(I1{});
+                add_slice(pc, I1{});
                 decode(pc, I2{}, b[0]);
             });
             order_fence();
             read_a(P, 3, a[1]);
             minimum(pc, I2{}, [&] {
                 multiply(I0{});
+                add_slice(pc, I2{});
                 decode(pc, I3{}, b[1]);
             });
             issue_fence();
@@ -455,7 +506,9 @@ __global__ __launch_bounds__(64 * kTileWaves * kTileGroups) void kq_prefill_kern
             issue_fence();
             minimum(pc, I3{}, [&] {
                 multiply(I1{});
+                add_slice(pc, I3{});
                 if constexpr (P == 3) {
+                    own_minimum();
 #pragma unroll
                     for (int j = 0; j < TN; ++j) d_fold[j] = sl[j].d;
                     unpack_head();
@@ -566,9 +619,11 @@ __global__ __launch_bounds__(256) void kq_sums_kernel(const uint16_t* __restrict
     dst[8] = __builtin_bit_cast(uint16_t, lo);
 }
 
+// One launch over M tokens: parts > 1 into `planes` (added by a second kernel),
+// Q4_K's activation sums through `sums` or, where null, OWN (64 and 96 rows).
 template <Fmt F, int TM, typename OutT>
 hipError_t launch_tile(const uint16_t* x, const uint8_t* w, OutT* y, uint32_t M, uint32_t N, uint32_t K,
-                       uint32_t parts, hipStream_t stream) {
+                       uint32_t parts, float* planes, uint16_t* sums, hipStream_t stream) {
     const uint32_t nb = K / kSuper;
     const uint32_t m_tiles = (M + 32 * TM - 1) / (32 * TM), n_tiles = (N + 32 * kTileWaves - 1) / (32 * kTileWaves);
     const uint32_t part_blocks = (nb + parts - 1) / parts;
@@ -576,27 +631,7 @@ hipError_t launch_tile(const uint16_t* x, const uint8_t* w, OutT* y, uint32_t M,
     const uint64_t total64 = static_cast<uint64_t>(m_tiles) * n_tiles * parts;
     if (total64 > 0x7ffffff0ull) return hipErrorInvalidConfiguration;
     const uint32_t total = static_cast<uint32_t>(total64), per_xcd = (total + 7) / 8;
-    // Scratch: the arrival counters every user of the pool leaves in place, the
-    // parts' planes, the activation sums.
-    const uint64_t count = static_cast<uint64_t>(M) * N;
-    const uint64_t plane_bytes = parts > 1 ? (count * parts * sizeof(float) + 15) / 16 * 16 : 0;
-    const uint64_t sum_bytes = F == Fmt::Q4K ? static_cast<uint64_t>(M) * nb * 32 : 0;
-    q4_0::ScratchPool::Lease lease;
-    float* partial = nullptr;
-    uint16_t* sums = nullptr;
-    if (plane_bytes + sum_bytes > 0) {
-        const hipError_t e = q4_0::acquire_scratch(stream, q4_0::kSplitKCounterBytes + plane_bytes + sum_bytes, &lease);
-        if (e != hipSuccess) return e;
-        auto* base = static_cast<uint8_t*>(lease.ptr());
-        if (lease.fresh()) {
-            const hipError_t z =
-                q4_0::launch_zero_fill(base, q4_0::kSplitKCounterBytes / 4, q4_0::OutType::F32, stream);
-            if (z != hipSuccess) return z;
-        }
-        partial = reinterpret_cast<float*>(base + q4_0::kSplitKCounterBytes);
-        sums = reinterpret_cast<uint16_t*>(base + q4_0::kSplitKCounterBytes + plane_bytes);
-    }
-    if constexpr (F == Fmt::Q4K) {
+    if (sums != nullptr) {
         const uint64_t subs = static_cast<uint64_t>(M) * nb * 8;
         hipLaunchKernelGGL(kq_sums_kernel, dim3(static_cast<uint32_t>((subs + 255) / 256)), dim3(256), 0, stream, x,
                            sums, subs);
@@ -605,23 +640,37 @@ hipError_t launch_tile(const uint16_t* x, const uint8_t* w, OutT* y, uint32_t M,
     }
     const dim3 grid(per_xcd * 8), block(64 * kTileWaves * kTileGroups);
     if (parts == 1) {
-        if constexpr (F == Fmt::Q8)
-            hipLaunchKernelGGL((q8_prefill_kernel<TM, false, OutT>), grid, block, 0, stream, x, w, y, partial, M, N, K,
+        if constexpr (F == Fmt::Q8) {
+            hipLaunchKernelGGL((q8_prefill_kernel<TM, false, OutT>), grid, block, 0, stream, x, w, y, planes, M, N, K,
                                m_tiles, n_tiles, part_blocks, total, per_xcd);
-        else
-            hipLaunchKernelGGL((kq_prefill_kernel<F, TM, false, OutT>), grid, block, 0, stream, x, w, sums, y,
-                               partial, M, N, K, m_tiles, n_tiles, part_blocks, total, per_xcd);
-        return hipGetLastError();
+            return hipGetLastError();
+        } else {
+            if constexpr (F == Fmt::Q4K) {
+                if (sums == nullptr) {
+                    if constexpr (TM < 4)
+                        hipLaunchKernelGGL((kq_prefill_kernel<F, TM, false, OutT, true>), grid, block, 0, stream, x, w,
+                                           sums, y, planes, M, N, K, m_tiles, n_tiles, part_blocks, total, per_xcd);
+                    else
+                        return hipErrorInvalidValue;
+                    return hipGetLastError();
+                }
+            }
+            hipLaunchKernelGGL((kq_prefill_kernel<F, TM, false, OutT>), grid, block, 0, stream, x, w, sums, y, planes,
+                               M, N, K, m_tiles, n_tiles, part_blocks, total, per_xcd);
+            return hipGetLastError();
+        }
     }
     if constexpr (F == Fmt::Q8)
         hipLaunchKernelGGL((q8_prefill_kernel<TM, true, float>), grid, block, 0, stream, x, w,
-                           static_cast<float*>(nullptr), partial, M, N, K, m_tiles, n_tiles, part_blocks, total, per_xcd);
+                           static_cast<float*>(nullptr), planes, M, N, K, m_tiles, n_tiles, part_blocks, total, per_xcd);
     else
         hipLaunchKernelGGL((kq_prefill_kernel<F, TM, true, float>), grid, block, 0, stream, x, w, sums,
-                           static_cast<float*>(nullptr), partial, M, N, K, m_tiles, n_tiles, part_blocks, total, per_xcd);
+                           static_cast<float*>(nullptr), planes, M, N, K, m_tiles, n_tiles, part_blocks, total, per_xcd);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((parts_reduce_kernel<OutT>), dim3(parts_reduce_grid(count)), dim3(256), 0, stream, partial, parts, count, y);
+    const uint64_t count = static_cast<uint64_t>(M) * N;
+    hipLaunchKernelGGL((parts_reduce_kernel<OutT>), dim3(parts_reduce_grid(count)), dim3(256), 0, stream, planes, parts,
+                       count, y);
     return hipGetLastError();
 }
 
@@ -640,19 +689,21 @@ struct Plan {
     uint32_t parts;
     double us;
 };
-// The planes of the parts stay inside the scratch a library stream starts with.
+// The planes of the parts and, behind them, Q4_K's sums fill a stream's scratch.
 constexpr uint64_t kMaxPlaneBytes = 48ull << 20;
 
+// Without scratch: one part, and for Q4_K the tiles that add up the
+// activations themselves (the 128-row ones would spill).
 template <Fmt F>
-Plan choose(uint32_t M, uint32_t N, uint32_t K) {
+Plan choose(uint32_t M, uint32_t N, uint32_t K, bool scratch = true) {
     const uint32_t nb = K / kSuper;
     const double cus = device_cus();
     Plan best{4, 1, 0.0};
     static constexpr double kBlockUs[3][3] = {{2.5, 1.95, 1.45}, {3.2, 2.7, 2.2}, {2.6, 2.0, 1.45}};
-    for (int tm = 4; tm >= 2; --tm) {
+    for (int tm = F == Fmt::Q4K && !scratch ? 3 : 4; tm >= 2; --tm) {
         const double block = kBlockUs[static_cast<int>(F)][4 - tm];
         const double tiles = static_cast<double>((M + 32u * tm - 1) / (32u * tm)) * ((N + 127u) / 128u);
-        for (uint32_t parts = 1; parts <= 8 && parts * 2 <= nb + 1; ++parts) {
+        for (uint32_t parts = 1; parts <= (scratch ? 8u : 1u) && parts * 2 <= nb + 1; ++parts) {
             const double plane_bytes = 4.0 * M * N * parts;
             if (parts > 1 && plane_bytes > static_cast<double>(kMaxPlaneBytes)) break;
             const double rounds = std::ceil(tiles * parts / cus);
@@ -685,16 +736,43 @@ hipError_t launch(const void* x, const void* w, void* y, uint32_t M, uint32_t N,
     const auto* xp = static_cast<const uint16_t*>(x);
     const auto* wp = static_cast<const uint8_t*>(w);
     auto* yp = static_cast<OutT*>(y);
-    auto run = [&](const Plan& p) {
-        return p.tm == 4   ? launch_tile<F, 4, OutT>(xp, wp, yp, M, N, K, p.parts, stream)
-               : p.tm == 3 ? launch_tile<F, 3, OutT>(xp, wp, yp, M, N, K, p.parts, stream)
-                           : launch_tile<F, 2, OutT>(xp, wp, yp, M, N, K, p.parts, stream);
+    auto run = [&](const Plan& p, uint32_t m0, uint32_t rows, float* planes, uint16_t* sums) {
+        const uint16_t* xm = xp + static_cast<size_t>(m0) * K;
+        OutT* ym = yp + static_cast<size_t>(m0) * N;
+        return p.tm == 4   ? launch_tile<F, 4, OutT>(xm, wp, ym, rows, N, K, p.parts, planes, sums, stream)
+               : p.tm == 3 ? launch_tile<F, 3, OutT>(xm, wp, ym, rows, N, K, p.parts, planes, sums, stream)
+                           : launch_tile<F, 2, OutT>(xm, wp, ym, rows, N, K, p.parts, planes, sums, stream);
     };
     const Plan plan = choose<F>(M, N, K);
-    const hipError_t e = run(plan);
-    // under graph capture without scratch for the planes: one part
-    if (e == hipErrorStreamCaptureUnsupported && plan.parts > 1) return run({plan.tm, 1, 0.0});
-    return e;
+    const uint64_t row_sums = F == Fmt::Q4K ? static_cast<uint64_t>(K / kSuper) * 32 : 0;
+    if (plan.parts == 1 && row_sums == 0) return run(plan, 0, M, nullptr, nullptr);
+    // Tokens whose sums do not fit beside the planes run in turns, whole tiles
+    // each where that is possible.
+    constexpr uint64_t kSumBytes = q4_0::kPromptScratchBytes - kMaxPlaneBytes;
+    uint32_t step = M;
+    if constexpr (F == Fmt::Q4K) {
+        if (row_sums * M > kSumBytes) {
+            step = static_cast<uint32_t>(kSumBytes / row_sums);
+            if (step > 32u * plan.tm) step -= step % (32u * plan.tm);
+        }
+    }
+    const uint64_t plane_bytes =
+        plan.parts > 1 ? (static_cast<uint64_t>(step) * N * plan.parts * sizeof(float) + 15) / 16 * 16 : 0;
+    q4_0::ScratchPool::Lease lease;  // holds the scratch until every kernel is queued
+    const hipError_t a = q4_0::acquire_prompt_scratch(stream, plane_bytes + row_sums * step, &lease);
+    if (a == hipErrorNotSupported) {
+        if (M <= 64 && F != Fmt::Q8) return a;  // the kernels of few tokens
+        return run(choose<F>(M, N, K, false), 0, M, nullptr, nullptr);
+    }
+    if (a != hipSuccess) return a;
+    auto* base = static_cast<uint8_t*>(lease.ptr());
+    for (uint64_t m0 = 0; m0 < M; m0 += step) {
+        const hipError_t e = run(plan, static_cast<uint32_t>(m0), static_cast<uint32_t>(M - m0 < step ? M - m0 : step),
+                                 reinterpret_cast<float*>(base),
+                                 row_sums > 0 ? reinterpret_cast<uint16_t*>(base + plane_bytes) : nullptr);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 }  // namespace

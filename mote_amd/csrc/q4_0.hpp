@@ -72,9 +72,8 @@ bool prefill_supports(const Variant& v, const Problem& p);
 bool prefill_ring_supports(const Problem& p);
 hipError_t launch_prefill_ring(const Problem& p, int bm, int bn, bool gate_up);
 // The linear on 128-row ring tiles over K parts where that is faster than bm x
-// bn tiles over all of K; hipErrorNotSupported, or hipErrorStreamCaptureUnsupported
-// (a stream under capture with too little scratch), with nothing queued, where
-// it is not or cannot.
+// bn tiles over all of K; hipErrorNotSupported, with nothing queued, where it is
+// not or the stream has no scratch for the parts.
 hipError_t launch_prefill_ring_parts(const Problem& p, int bm, int bn);
 
 hipError_t launch_zero_fill(void* y, uint64_t count, OutType out, hipStream_t stream);
@@ -93,6 +92,18 @@ hipError_t acquire_scratch(hipStream_t stream, size_t bytes, ScratchPool::Lease*
 // Sizes a stream's scratch to at least `bytes` ahead of its first split-K
 // call (a new buffer gets its tile counters cleared on the stream).
 hipError_t reserve_stream_scratch(hipStream_t stream, size_t bytes);
+// Scratch of the calls of many tokens (the K parts' planes, the Q4_K activation
+// sums): a buffer of kPromptScratchBytes apart from the split-K one, which only
+// streams made by mote_hip_stream_create have, from their creation on.
+// acquire_prompt_scratch never allocates: hipErrorNotSupported, with nothing
+// queued, on any other stream (its handle may name another queue in each thread,
+// or be reused while work is left), under graph capture (a graph may be
+// replayed beside eager calls of its stream, beside another graph, or after
+// the stream is gone) and for more bytes; such calls run without scratch.
+constexpr size_t kPromptScratchBytes = size_t{64} << 20;
+hipError_t acquire_prompt_scratch(hipStream_t stream, size_t bytes, ScratchPool::Lease* lease);
+// Gives a stream its buffer; a failure leaves the stream without one.
+hipError_t reserve_prompt_scratch(hipStream_t stream);
 // Frees the parked scratch of destroyed streams whose work has completed.
 hipError_t reap_parked_scratch();
 // Forgets a stream's scratch without waiting for its queued work: the buffers

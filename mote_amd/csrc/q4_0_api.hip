@@ -1108,6 +1108,10 @@ ScratchPool& scratch_pool() {
     static ScratchPool* pool = new ScratchPool(device_alloc, device_free);  // lives until exit
     return *pool;
 }
+ScratchPool& prompt_pool() {
+    static ScratchPool* pool = new ScratchPool(device_alloc, device_free);
+    return *pool;
+}
 
 }  // namespace
 
@@ -1135,6 +1139,30 @@ hipError_t reserve_stream_scratch(hipStream_t stream, size_t bytes) {
     return launch_zero_fill(lease.ptr(), kSplitKCounterBytes / 4, OutType::F32, stream);
 }
 
+hipError_t acquire_prompt_scratch(hipStream_t stream, size_t bytes, ScratchPool::Lease* lease) {
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    ScratchPool::Lease held;
+    if (prompt_pool().acquire(dev, stream, bytes, &held, false) != 0) return hipErrorNotSupported;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    e = hipStreamIsCapturing(stream, &capture);
+    if (e != hipSuccess) return e;
+    if (capture != hipStreamCaptureStatusNone) return hipErrorNotSupported;
+    *lease = std::move(held);
+    return hipSuccess;
+}
+
+hipError_t reserve_prompt_scratch(hipStream_t stream) {
+    int dev = 0;
+    const hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    ScratchPool::Lease lease;
+    const int status = prompt_pool().acquire(dev, stream, kPromptScratchBytes, &lease);
+    if (status != 0) (void)hipGetLastError();  // not the next call's error
+    return static_cast<hipError_t>(status);
+}
+
 hipError_t reap_parked_scratch() { return reap_parked(); }
 
 hipError_t park_stream_scratch(hipStream_t stream) {
@@ -1142,6 +1170,7 @@ hipError_t park_stream_scratch(hipStream_t stream) {
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
     std::vector<void*> buffers = scratch_pool().detach(dev, stream);
+    for (void* b : prompt_pool().detach(dev, stream)) buffers.push_back(b);
     if (buffers.empty()) return reap_parked();
     hipEvent_t done = nullptr;
     e = hipEventCreateWithFlags(&done, hipEventDisableTiming);

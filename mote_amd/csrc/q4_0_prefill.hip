@@ -488,20 +488,17 @@ hipError_t launch_prefill(const Problem& p) {
         if (prefill_ring_supports(p)) {
             if constexpr (!GATE_UP) {
                 const hipError_t e = launch_prefill_ring_parts(p, BM, BN);
-                if (e != hipErrorNotSupported && e != hipErrorStreamCaptureUnsupported) return e;
+                if (e != hipErrorNotSupported) return e;
             }
             if constexpr (BM == 128) return launch_prefill_ring(p, BM, BN, GATE_UP);
         }
     }
     // Multi-pair Q8_0 tiles: the exact-integer tiles where the operands fit them
-    // (their own choice of rows per tile and K parts); without scratch for a
-    // choice of theirs under graph capture, this body.
+    // (their own choice of rows per tile and K parts).
     if constexpr (SPEC && T32 && KP > 1 && Q8) {
-        if (kquant::prefill_supported(kquant::Fmt::Q8, p.x, p.w, p.M, p.N, p.K)) {
-            const hipError_t e = kquant::launch_prefill(kquant::Fmt::Q8, p.out == OutType::F16, p.x, p.w, p.y, p.M,
-                                                        p.N, p.K, p.stream);
-            if (e != hipErrorStreamCaptureUnsupported) return e;
-        }
+        if (kquant::prefill_supported(kquant::Fmt::Q8, p.x, p.w, p.M, p.N, p.K))
+            return kquant::launch_prefill(kquant::Fmt::Q8, p.out == OutType::F16, p.x, p.w, p.y, p.M, p.N, p.K,
+                                          p.stream);
     }
     const uint32_t m_tiles = (p.M + BM - 1) / BM;
     const uint32_t n_tiles = (p.N + BN - 1) / BN;

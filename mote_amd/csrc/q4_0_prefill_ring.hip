@@ -340,9 +340,9 @@ __global__ __launch_bounds__(64 * WN * kGroups) void prefill_ring_kernel(
     }
 }
 
-// parts > 1 (linear): K parts in planes of the stream's scratch, added by a
-// second kernel.  hipErrorStreamCaptureUnsupported, with nothing queued, when
-// the stream is under capture and holds too little of it.
+// parts > 1 (linear): K parts in planes of the stream's prompt scratch, added by
+// a second kernel.  hipErrorNotSupported, with nothing queued, where the stream
+// has none (acquire_prompt_scratch).
 template <int TM, int WN, bool GATE_UP>
 hipError_t launch_ring(const Problem& p, uint32_t parts) {
     constexpr uint32_t BM = 32 * TM, BN = (GATE_UP ? 32 : 64) * WN;
@@ -362,16 +362,10 @@ hipError_t launch_ring(const Problem& p, uint32_t parts) {
     if constexpr (!GATE_UP) {
         if (parts > 1) {
             const uint64_t count = static_cast<uint64_t>(p.M) * p.N;
-            const size_t need = kSplitKCounterBytes + count * parts * sizeof(float);
             ScratchPool::Lease lease;  // holds the scratch until both kernels are queued
-            const hipError_t a = acquire_scratch(p.stream, need, &lease);
+            const hipError_t a = acquire_prompt_scratch(p.stream, count * parts * sizeof(float), &lease);
             if (a != hipSuccess) return a;
-            auto* const base = static_cast<uint8_t*>(lease.ptr());
-            if (lease.fresh()) {  // the arrival counters every user of the pool leaves zero
-                const hipError_t z = launch_zero_fill(base, kSplitKCounterBytes / 4, OutType::F32, p.stream);
-                if (z != hipSuccess) return z;
-            }
-            auto* planes = reinterpret_cast<float*>(base + kSplitKCounterBytes);
+            auto* const planes = static_cast<float*>(lease.ptr());
             hipLaunchKernelGGL((prefill_ring_kernel<TM, WN, false, true, float>), grid, block, 0, p.stream, x, wg, wu,
                                static_cast<float*>(nullptr), planes, p.M, p.N, p.K, m_tiles, n_tiles, part_pairs, total,
                                per_xcd);
@@ -412,14 +406,12 @@ bool prefill_ring_supports(const Problem& p) {
 // their time) + reduction, against a bm x bn tiling's own rounds.  Fits to
 // MI355X timings in us per super-pair: 3.6 (128 x 256), 2.2 (128 x 128), the
 // staging-wave tiles 1.25 (64 x 128), 0.85 (64 x 64); the reduction 3 us and the
-// planes written and read once at 4 TB/s, planes up to 48 MiB (inside the
-// scratch a library stream starts with).  Measured against the tiles it
+// planes written and read once at 4 TB/s, planes up to 48 MiB (inside a
+// library stream's prompt scratch).  Measured against the tiles it
 // replaced (us): 128 / 256 x 14 336 x 4096 51.0 -> 30.1, 56.3 -> 43.2; 400 x 14
 // 336 x 5120 118 -> 82; 100 x 13 824 x 5120 49.4 -> 31.7; 65 x 28 672 x 8192 114
-// -> 73; 32 x 11 008 x 4096 39.4 -> 22.8.  Not where the caller brings scratch
-// of its own (the allocation-free entry point): calls that may overlap share it.
+// -> 73; 32 x 11 008 x 4096 39.4 -> 22.8.
 hipError_t launch_prefill_ring_parts(const Problem& p, int bm, int bn) {
-    if (p.scratch != nullptr) return hipErrorNotSupported;
     static const int cus = [] {
         int dev = 0, n = 0;
         if (hipGetDevice(&dev) != hipSuccess ||

@@ -50,7 +50,9 @@ constexpr std::size_t kStreamScratchBytes = std::size_t{64} << 20;
 
 // As in the reference (crates/mote-backend-hip/src/hipblaslt_shim.cpp:296-305),
 // plus the stream's split-K scratch; a stream whose scratch cannot be
-// allocated is destroyed again and the error returned.
+// allocated is destroyed again and the error returned.  The scratch of the calls
+// of many tokens comes with the stream too; where there is no memory for it
+// those calls run without.
 MOTE_EXPORT int mote_hip_stream_create(void** stream) noexcept {
     if (stream == nullptr) return kInvalidArgument;
     *stream = nullptr;
@@ -59,6 +61,7 @@ MOTE_EXPORT int mote_hip_stream_create(void** stream) noexcept {
     if (status != hipSuccess) return static_cast<int>(status);
     try {
         status = mote::q4_0::reserve_stream_scratch(native, kStreamScratchBytes);
+        if (status == hipSuccess) (void)mote::q4_0::reserve_prompt_scratch(native);
     } catch (...) {
         status = hipErrorUnknown;
     }
@@ -75,7 +78,7 @@ MOTE_EXPORT int mote_hip_stream_create(void** stream) noexcept {
 }
 
 // Destroys the stream without waiting for its queued work, as the reference
-// does (crates/mote-backend-hip/src/hipblaslt_shim.cpp:307).  The split-K
+// does (crates/mote-backend-hip/src/hipblaslt_shim.cpp:307).  The
 // scratch the library keeps for the stream is detached first, so a stream
 // created later at the same address starts without it, and freed once the
 // work queued before the destroy has completed (an event recorded on the

@@ -79,9 +79,14 @@ class ScratchPool {
         std::shared_ptr<Entry> entry;
         {
             std::lock_guard<std::mutex> guard(map_mu_);
-            auto& slot = entries_[{device, stream}];
-            if (!slot) slot = std::make_shared<Entry>();
-            entry = slot;
+            const auto found = entries_.find({device, stream});
+            if (found != entries_.end()) {
+                entry = found->second;
+            } else {
+                if (!may_allocate) return kWouldAllocate;  // and no entry is left for the stream
+                entry = std::make_shared<Entry>();
+                entries_[{device, stream}] = entry;
+            }
         }
         std::unique_lock<std::mutex> lock(entry->mu);
         lease->fresh_ = false;

@@ -214,6 +214,7 @@ void test_acquire_that_may_not_allocate() {
         CHECK(pool.acquire(0, stream, 64, &a, false) == ScratchPool::kWouldAllocate);
         CHECK(!a.held());
         CHECK(g_allocs == allocs0);
+        CHECK(pool.streams() == 0);
     }
     void* first = nullptr;
     {
