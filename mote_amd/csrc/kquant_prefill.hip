@@ -127,6 +127,13 @@ __global__ __launch_bounds__(64 * kTileWaves * kTileGroups) void kq_prefill_kern
     // two operands' sums apart (half as many roundings in a row: 1.2e-7 of the
     // result at K = 4096, as the few-token tiles, against 1.45e-7).
     constexpr int NC = NB == 2 && TM == 2 ? 2 : 1;
+    // ... and add up the result in runs of kRun super-blocks, then the runs:
+    // a single chain over one K part of 56 super-blocks was coarser than the
+    // few-token tiles' sixteen waves (64 x 14 336 x 32 768 Q4_K 1.68e-7 of the
+    // result against 1.35e-7, Q6_K 1.36e-7 against 1.28e-7; in runs 1.32e-7 and
+    // 1.17e-7, at the same time).
+    constexpr bool RUNS = TM == 2;
+    constexpr uint32_t kRun = 8;
     constexpr uint32_t BB = block_bytes<F>();
     constexpr int kRing = kSlots * KG * kUnit;
     constexpr int kReduce = kTileWaves * KG * ((TM + 1) / 2) * TN * 4096;
@@ -302,7 +309,7 @@ __global__ __launch_bounds__(64 * kTileWaves * kTileGroups) void kq_prefill_kern
         }
     };
 
-    f32x16 acc[TM][TN], blk[NC][TM][TN];
+    f32x16 acc[TM][TN], blk[NC][TM][TN], runs[RUNS ? TM : 1][TN];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -310,6 +317,7 @@ __global__ __launch_bounds__(64 * kTileWaves * kTileGroups) void kq_prefill_kern
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 acc[i][j][r] = 0.0f;
+                if constexpr (RUNS) runs[i][j][r] = 0.0f;
 #pragma unroll
                 for (int c = 0; c < NC; ++c) blk[c][i][j][r] = 0.0f;
             }
@@ -523,11 +531,25 @@ __global__ __launch_bounds__(64 * kTileWaves * kTileGroups) void kq_prefill_kern
             interval(I1{}, s);
             interval(I2{}, s);
             interval(I3{}, s);
+            if constexpr (RUNS) {
+                if (s % kRun == kRun - 1) {
+#pragma unroll
+                    for (int i = 0; i < TM; ++i)
+#pragma unroll
+                        for (int j = 0; j < TN; ++j) {
+                            runs[i][j] += acc[i][j];
+                            acc[i][j] = zero;
+                        }
+                }
+            }
         }
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int j = 0; j < TN; ++j) fold(i, j);
+            for (int j = 0; j < TN; ++j) {
+                fold(i, j);
+                if constexpr (RUNS) acc[i][j] += runs[i][j];
+            }
     }
     for (uint32_t t = ns * 4; t < per * 4; ++t) group_barrier();
     wait_counts<vm_wait(0)>();

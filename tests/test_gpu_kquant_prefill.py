@@ -18,6 +18,7 @@ import pytest
 from helpers import bits_to_f32
 from mote_amd import workloads as wl
 from mote_amd.device import DeviceBuffer, Stream
+from mote_amd.hip_runtime import HipRuntime
 from test_gpu_kquant import FORMATS, _blocks, _check, _fmt, _judge, _run
 
 pytestmark = pytest.mark.gpu
@@ -107,3 +108,32 @@ def test_many_tokens_unaligned_activations(stream, oracle, name, x_offset):
     x = wl.normal_f16(wl.seed_for(45, 1), m * k)
     y64, max_w, max_x = _judge(oracle, name, x, w, m, n, k)
     _check(_run(stream, name, x, w, m, n, k, x_offset=x_offset), y64, k, max_w, max_x, what=f"{name} x unaligned")
+
+
+def test_long_k_is_no_coarser_than_the_few_token_tiles(stream, oracle):
+    """64 tokens, K = 14 336, columns enough for one K part: the many-token tiles
+    against the few-token ones, which the same call runs under capture.  Both
+    errors are means over 65 536 outputs (0.4 % either way); 3 % is allowed."""
+    m, rows, n, k = 64, 1024, 32768, 14336
+    w, x = wl.q4_k_weights(860, rows, k), wl.normal_f16(861, m * k)
+    y64 = oracle.kquant_linear_f64(bits_to_f32(x), w, oracle.Q4_K, m, rows, k)
+    xb, wb = DeviceBuffer.from_array(x), DeviceBuffer.from_array(np.tile(w.reshape(-1), n // rows))
+    yb, hip = DeviceBuffer(m * n * 4), HipRuntime()
+
+    def call():
+        FORMATS["q4_k"][2](xb.ptr, wb.ptr, yb.ptr, m, n, k, stream)
+
+    def error():
+        stream.synchronize()
+        y = yb.download(np.float32).reshape(m, n)[:, :rows].astype(np.float64)
+        return float(np.linalg.norm(y - y64) / np.linalg.norm(y64))
+
+    call()
+    many = error()
+    graph = hip.capture(stream, call)
+    try:
+        hip.launch_graph(graph, stream)
+        few = error()
+    finally:
+        hip.destroy_graph(graph)
+    assert many <= 1.03 * few, f"relative error {many:.3e}, few-token tiles {few:.3e}"
