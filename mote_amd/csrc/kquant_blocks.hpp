@@ -68,7 +68,9 @@ __device__ __forceinline__ u32x4 load16_a2(const uint8_t* p) {
 // form can overflow, so they agree to rounding; an infinite or NaN scale (or
 // a non-finite activation) makes the folded sum not finite, and then it can
 // put +-inf where the per-element values give NaN (inf * 0 for q = 0 or
-// sc = 0, products of both signs).  A wave whose reduced sum is not finite (a
+// sc = 0, products of both signs).  (The few-token Q4_K tiles get there with
+// finite activations whose sum over a sub-block passes binary16's range, too.)
+// A wave whose reduced sum is not finite (a
 // wave-uniform test) recomputes its share of the row element by element, so
 // the NaN and infinities land where the definition puts them.
 // ---------------------------------------------------------------------------

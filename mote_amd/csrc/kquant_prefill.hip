@@ -19,8 +19,9 @@
 // q; Q6_K sc (q - 32) = 8 s (q - 32) + t (q - 32) with s = sc >> 3, t = sc & 7,
 // two operands (q - 32) s and (q - 32) t / 8 into the same accumulator.  Every
 // product with an activation is exact in f32; once per super-block
-//   Q4_K: y += d C - dmin C',  C' = sum_j m_j S_j (two MFMA operands: S_j, the
-//         activations' sum over sub-block j, as binary16 hi + lo, against m_j)
+//   Q4_K: y += d C - dmin C',  C' = sum_j m_j S_j (two bfloat16 MFMAs: S_j, the
+//         f32 sum of the activations over sub-block j, in three pieces, exact
+//         and of any size, against m_j)
 //   Q6_K: y += 8 d C.
 // So the decode costs 10 (Q4_K) or 20 (Q6_K) vector instructions per 8
 // weights and TM MFMAs (2 TM for Q6_K), and the per-super-block fold 16 TM.
@@ -31,11 +32,16 @@
 // operand read covers per cycle fall on the 64 banks once (swizzled by the row,
 // every read took 8 cycles instead of 4).  One barrier per interval, before its last slice:
 // the slice's MFMAs cover the first LDS reads and decode of the next interval.
+// The Q4_K sums come through LDS too (kq_sums_kernel writes them before), one
+// super-block ahead: as binary16 hi + lo loaded to registers they made sums
+// past 65504 recompute the token's outputs one by one, and the 128-row tile
+// spilled and waited for every load in flight once per super-block (512 x 4096
+// x 14 336 83.9 us against 81.7, 256 x 14 336 x 4096 47.6 against 46.9).
 // The groups' partial tiles meet in LDS (fixed order); K parts, used where the
 // tiles are too few for the chip, meet in scratch planes that
 // parts_reduce_kernel adds in part order.  Planes and sums live in the stream's
 // prompt scratch (q4_0.hpp).  Without it there is one part, and Q4_K's sums are
-// added up from the operands in registers, 16 elements per lane, two MFMAs per
+// added up from the operands in registers, 16 elements per lane, three MFMAs per
 // super-block (OWN): 32 dot products per tile and quarter in every wave, which 96-
 // and 64-row tiles have registers for.  512 x 4096 x 14 336 122 us against 85.
 //
@@ -100,7 +106,7 @@ struct Scales;
 template <>
 struct Scales<Fmt::Q4K> {
     uint32_t sc[2];  // sc_0..3, sc_4..7, a byte each
-    uint32_t m[2];   // m_0..3, m_4..7
+    uint32_t m[4];   // m_0, m_1; .. m_6, m_7 as bfloat16
     float d, dmin;
 };
 template <>
@@ -108,6 +114,24 @@ struct Scales<Fmt::Q6K> {
     uint32_t sc[4];  // quarter p: its scales at bytes 0 (h = 0) and 2 (h = 1)
     float d;
 };
+
+// A float as three bfloat16 (eight significant bits each, cut off: exact).
+struct Pieces {
+    uint32_t p[3];
+};
+__device__ __forceinline__ Pieces pieces(float v) {
+    const uint32_t a = __builtin_bit_cast(uint32_t, v) & 0xFFFF0000u;
+    const float r = v - __builtin_bit_cast(float, a);
+    const uint32_t b = __builtin_bit_cast(uint32_t, r) & 0xFFFF0000u;
+    const uint32_t c = __builtin_bit_cast(uint32_t, r - __builtin_bit_cast(float, b));
+    return {{a >> 16, b >> 16, c >> 16}};
+}
+// Two bytes of w, at selectors a and b, as a pair of bfloat16.
+template <int A, int B>
+__device__ __forceinline__ uint32_t bytes_bf16(uint32_t w) {
+    const float a = static_cast<float>((w >> (8 * A)) & 0xFFu), b = static_cast<float>((w >> (8 * B)) & 0xFFu);
+    return perm(__builtin_bit_cast(uint32_t, b), __builtin_bit_cast(uint32_t, a), 0x07060302u);
+}
 
 // OWN (Q4_K): each wave adds up the sub-blocks' activations itself instead of
 // reading kq_sums_kernel's.
@@ -136,8 +160,13 @@ __global__ __launch_bounds__(64 * kTileWaves * kTileGroups) void kq_prefill_kern
     constexpr uint32_t kRun = 8;
     constexpr uint32_t BB = block_bytes<F>();
     constexpr int kRing = kSlots * KG * kUnit;
+    // The activations' sums: 64 bytes per row, two super-blocks of each group.
+    constexpr bool SUMS = F == Fmt::Q4K && !OWN;
+    constexpr int NS = SUMS ? (BM * 64 + kTileWaves * 1024 - 1) / (kTileWaves * 1024) : 0;  // loads per wave
+    constexpr int kSumUnit = NS * kTileWaves * 1024;
     constexpr int kReduce = kTileWaves * KG * ((TM + 1) / 2) * TN * 4096;
-    __shared__ __attribute__((aligned(1024))) uint8_t lds[kRing > kReduce ? kRing : kReduce];
+    static_assert(kRing >= kReduce && kRing + 2 * KG * kSumUnit <= 160 * 1024, "LDS");
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[kRing + 2 * KG * kSumUnit];
 
     const uint32_t logical = (blockIdx.x % 8u) * per_xcd + blockIdx.x / 8u;
     if (logical >= total) return;
@@ -227,8 +256,12 @@ __global__ __launch_bounds__(64 * kTileWaves * kTileGroups) void kq_prefill_kern
                 const u32x4 head = raw[j].head;
                 sl[j].sc[0] = head.y & 0x3F3F3F3Fu;
                 sl[j].sc[1] = (head.w & 0x0F0F0F0Fu) | ((head.y >> 2) & 0x30303030u);
-                sl[j].m[0] = head.z & 0x3F3F3F3Fu;
-                sl[j].m[1] = ((head.w >> 4) & 0x0F0F0F0Fu) | ((head.z >> 2) & 0x30303030u);
+                const uint32_t lo = head.z & 0x3F3F3F3Fu;
+                const uint32_t hi = ((head.w >> 4) & 0x0F0F0F0Fu) | ((head.z >> 2) & 0x30303030u);
+                sl[j].m[0] = bytes_bf16<0, 1>(lo);
+                sl[j].m[1] = bytes_bf16<2, 3>(lo);
+                sl[j].m[2] = bytes_bf16<0, 1>(hi);
+                sl[j].m[3] = bytes_bf16<2, 3>(hi);
                 sl[j].d = as_f32(half_lo_to_float(head.x));
                 sl[j].dmin = as_f32(half_hi_to_float(head.x));
             } else {
@@ -359,32 +392,42 @@ __global__ __launch_bounds__(64 * kTileWaves * kTileGroups) void kq_prefill_kern
                 }
     };
     // Q4_K's minimum term of the super-block, one tile per slice of its second
-    // half: token row r of tile i holds the eight hi (c = 0) or lo (c = 1)
-    // halves of the sub-block sums.
-    f16x8 sx[TM];
-    auto load_sums = [&](uint32_t s) {
-        if constexpr (F == Fmt::Q4K && !OWN) {
-            const uint16_t* src = sums + static_cast<size_t>(b0 + s) * 16 + 8 * lc;
+    // half.  A row's sums are four 16-byte chunks: the three bfloat16 pieces of
+    // the eight sub-blocks' sums, and zeros; half wave c of the two products
+    // supplies chunk c, then chunk 2 + c.  In LDS a row's chunk q is at q ^ (row / 4) % 4.
+    bf16x8 sx[2][2];
+    uint8_t* const sum_unit = lds + kRing + kg * kSumUnit;
+    uint32_t soff[NS > 0 ? NS : 1];
+    const Buffer ssrc = buffer_at(reinterpret_cast<const uint8_t*>(sums) + (static_cast<size_t>(m0) * nb + b0) * 64);
 #pragma unroll
-            for (int i = 0; i < TM; ++i)
-                sx[i] = *reinterpret_cast<const f16x8*>(src + static_cast<size_t>(min(m0 + i * 32 + lr, M - 1)) * nb * 16);
-        }
+    for (int i = 0; i < NS; ++i) {
+        const uint32_t at = (wn * NS + i) * 64 + lane, row = at >> 2;
+        soff[i] = (min(m0 + row, M - 1) - m0) * (nb * 64) + (((at & 3) ^ ((row >> 2) & 3)) * 16);
+    }
+    auto load_sums = [&](uint32_t s) {
+#pragma unroll
+        for (int i = 0; i < NS; ++i)
+            load_lds16(ssrc, soff[i], min(s, ns - 1) * 64u,
+                       sum_unit + (s & 1u) * (KG * kSumUnit) + (wn * NS + i) * 1024);
+    };
+    auto read_sums = [&](uint32_t s, int i) {
+        const uint8_t* row = sum_unit + (s & 1u) * (KG * kSumUnit) + (i * 32 + lr) * 64;
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+            sx[i & 1][k] = *reinterpret_cast<const bf16x8*>(row + (((2 * k + lc) ^ ((lr >> 2) & 3)) * 16));
     };
     auto mins = [&](int j) {
-        if constexpr (F == Fmt::Q4K) {
-            const f16x2 b = both(static_cast<_Float16>(-1024.0f));
-            const uint32_t e = 0x64646464u, lo = sl[j].m[0], hi = sl[j].m[1];
-            return join(as_h2(perm(e, lo, 0x04010400u)) + b, as_h2(perm(e, lo, 0x04030402u)) + b,
-                        as_h2(perm(e, hi, 0x04010400u)) + b, as_h2(perm(e, hi, 0x04030402u)) + b);
-        }
+        if constexpr (F == Fmt::Q4K)
+            return __builtin_bit_cast(bf16x8, u32x4{sl[j].m[0], sl[j].m[1], sl[j].m[2], sl[j].m[3]});
     };
-    auto minimum = [&](auto pc, auto ic, auto slice) {
+    auto minimum = [&](auto pc, auto ic, uint32_t s, auto slice) {
         constexpr int I = 4 * (decltype(pc)::value - 2) + decltype(ic)::value;
-        if constexpr (F == Fmt::Q4K && !OWN) {
+        if constexpr (SUMS) {
+            if constexpr (I + 1 >= 0 && I + 1 < TM) read_sums(s, I + 1);
             if constexpr (I >= 0 && I < TM) {
                 f32x16 mn[TN];
 #pragma unroll
-                for (int j = 0; j < TN; ++j) mn[j] = mfma32(sx[I], mins(j), zero);
+                for (int j = 0; j < TN; ++j) mn[j] = mfma32(sx[I & 1][1], mins(j), mfma32(sx[I & 1][0], mins(j), zero));
                 slice();
 #pragma unroll
                 for (int j = 0; j < TN; ++j)
@@ -397,11 +440,11 @@ __global__ __launch_bounds__(64 * kTileWaves * kTileGroups) void kq_prefill_kern
             slice();
         }
     };
-    // OWN: the lane's part of sub-block j's sum, its elements 16 c .. 16 c + 15, as
-    // binary16 hi and lo halves at j of 8 (in each c: the MFMAs add both), from
-    // the slices' operands; after the last slice the minimum term of every tile.
+    // OWN: the lane's part of sub-block j's sum, its elements 16 c .. 16 c + 15, in
+    // three pieces at j of 8 (in each c: the MFMAs add both), from the slices'
+    // operands; after the last slice the minimum term of every tile.
     float run[TM];
-    uint32_t own[TM][2][4];
+    uint32_t own[TM][3][4];
     auto add_slice = [&](auto pc, auto ic) {
         if constexpr (OWN) {
             constexpr int P = decltype(pc)::value, S = decltype(ic)::value, h = S / 2, u = S % 2;
@@ -413,11 +456,9 @@ __global__ __launch_bounds__(64 * kTileWaves * kTileGroups) void kq_prefill_kern
                 if constexpr (u == 0) {
                     run[i] = s;
                 } else {
-                    const _Float16 hi = static_cast<_Float16>(s);
-                    const _Float16 lo = static_cast<_Float16>(s - static_cast<float>(hi));
-                    const uint32_t b[2] = {__builtin_bit_cast(uint16_t, hi), __builtin_bit_cast(uint16_t, lo)};
+                    const Pieces b = pieces(s);
 #pragma unroll
-                    for (int k = 0; k < 2; ++k) own[i][k][P] = h ? own[i][k][P] | (b[k] << 16) : b[k];
+                    for (int k = 0; k < 3; ++k) own[i][k][P] = h ? own[i][k][P] | (b.p[k] << 16) : b.p[k];
                 }
             }
         }
@@ -430,9 +471,9 @@ __global__ __launch_bounds__(64 * kTileWaves * kTileGroups) void kq_prefill_kern
                 for (int j = 0; j < TN; ++j) {
                     f32x16 mn = zero;
 #pragma unroll
-                    for (int k = 0; k < 2; ++k) {
+                    for (int k = 0; k < 3; ++k) {
                         const u32x4 v = {own[i][k][0], own[i][k][1], own[i][k][2], own[i][k][3]};
-                        mn = mfma32(__builtin_bit_cast(f16x8, v), mins(j), mn);
+                        mn = mfma32(__builtin_bit_cast(bf16x8, v), mins(j), mn);
                     }
 #pragma unroll
                     for (int r = 0; r < 16; ++r) acc[i][j][r] = __builtin_fmaf(-sl[j].dmin, mn[r], acc[i][j][r]);
@@ -440,16 +481,18 @@ __global__ __launch_bounds__(64 * kTileWaves * kTileGroups) void kq_prefill_kern
         }
     };
     // Loads a wave issues behind interval t's activations of four intervals on:
-    // quants, the sums (p = 0), the next header (p = 2).
+    // quants, the next super-block's sums (p = 0) and header (p = 2).
     constexpr bool kQ4 = F == Fmt::Q4K;
     constexpr int kHalf = (kQ4 ? 2 : 3) * TN;  // a half block's quants
-    constexpr int kBehind[4] = {kQ4 && !OWN ? TM : 0, kHalf, kQ4 ? TN : 2 * TN, kHalf};
+    constexpr int kBehind[4] = {NS, kHalf, kQ4 ? TN : 2 * TN, kHalf};
     using I0 = std::integral_constant<int, 0>;
     using I1 = std::integral_constant<int, 1>;
     using I2 = std::integral_constant<int, 2>;
     using I3 = std::integral_constant<int, 3>;
 
     if (ns > 0) {  // uniform over the wave; groups without work only meet the barriers
+        load_sums(0);
+        issue_fence();
         load_a(0, 0);
         issue_fence();
         load_a(1, 1);
@@ -479,21 +522,21 @@ __global__ __launch_bounds__(64 * kTileWaves * kTileGroups) void kq_prefill_kern
             constexpr int P = decltype(pc)::value;
             using PN = std::integral_constant<int, (P + 1) & 3>;
             read_a(P, 1, a[1]);
-            minimum(pc, I0{}, [&] {
+            minimum(pc, I0{}, s, [&] {
                 if constexpr (P == 0) multiply_first(); else multiply(I0{});
                 add_slice(pc, I0{});
                 decode(pc, I1{}, b[1]);
             });
             order_fence();
             read_a(P, 2, a[0]);
-            minimum(pc, I1{}, [&] {
+            minimum(pc, I1{}, s, [&] {
                 multiply(I1{});
                 add_slice(pc, I1{});
                 decode(pc, I2{}, b[0]);
             });
             order_fence();
             read_a(P, 3, a[1]);
-            minimum(pc, I2{}, [&] {
+            minimum(pc, I2{}, s, [&] {
                 multiply(I0{});
                 add_slice(pc, I2{});
                 decode(pc, I3{}, b[1]);
@@ -510,9 +553,9 @@ __global__ __launch_bounds__(64 * kTileWaves * kTileGroups) void kq_prefill_kern
             issue_fence();
             load_quants(pc, s + 1);
             if constexpr (P == 2) load_head(s + 1);
-            if constexpr (P == 0) load_sums(s);
+            if constexpr (P == 0) load_sums(s + 1);
             issue_fence();
-            minimum(pc, I3{}, [&] {
+            minimum(pc, I3{}, s, [&] {
                 multiply(I1{});
                 add_slice(pc, I3{});
                 if constexpr (P == 3) {
@@ -619,9 +662,9 @@ __global__ __launch_bounds__(64 * kTileWaves * kTileGroups) void kq_prefill_kern
     }
 }
 
-// sums[m][b][0..7] and [8..15]: the binary16 hi and lo halves of the sums of
-// token m's activations over the eight sub-blocks of super-block b.  One thread
-// per sub-block.
+// sums[m][b][0..7], [8..15], [16..23]: the three pieces of the sums of token m's
+// activations over the eight sub-blocks of super-block b, [24..31] zeros.  One
+// thread per sub-block.
 __global__ __launch_bounds__(256) void kq_sums_kernel(const uint16_t* __restrict__ x, uint16_t* __restrict__ sums,
                                                       uint64_t count) {
     const uint64_t i = static_cast<uint64_t>(blockIdx.x) * 256 + threadIdx.x;
@@ -634,11 +677,11 @@ __global__ __launch_bounds__(256) void kq_sums_kernel(const uint16_t* __restrict
         const u32x4 v = src[k];
         s = dot2(v.w, one, dot2(v.z, one, dot2(v.y, one, dot2(v.x, one, s))));
     }
-    const _Float16 hi = static_cast<_Float16>(s);
-    const _Float16 lo = static_cast<_Float16>(s - static_cast<float>(hi));
-    uint16_t* dst = sums + (i / 8) * 16 + i % 8;
-    dst[0] = __builtin_bit_cast(uint16_t, hi);
-    dst[8] = __builtin_bit_cast(uint16_t, lo);
+    const Pieces p = pieces(s);
+    uint16_t* dst = sums + (i / 8) * 32 + i % 8;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) dst[8 * k] = static_cast<uint16_t>(p.p[k]);
+    dst[24] = 0;
 }
 
 // One launch over M tokens: parts > 1 into `planes` (added by a second kernel),
@@ -766,7 +809,7 @@ hipError_t launch(const void* x, const void* w, void* y, uint32_t M, uint32_t N,
                            : launch_tile<F, 2, OutT>(xm, wp, ym, rows, N, K, p.parts, planes, sums, stream);
     };
     const Plan plan = choose<F>(M, N, K);
-    const uint64_t row_sums = F == Fmt::Q4K ? static_cast<uint64_t>(K / kSuper) * 32 : 0;
+    const uint64_t row_sums = F == Fmt::Q4K ? static_cast<uint64_t>(K / kSuper) * 64 : 0;
     if (plan.parts == 1 && row_sums == 0) return run(plan, 0, M, nullptr, nullptr);
     // Tokens whose sums do not fit beside the planes run in turns, whole tiles
     // each where that is possible.

@@ -6,8 +6,7 @@ against the oracle's f64 linear over the oracle-decoded weights.
 The tiles' products are exact and summed in f32, so besides the tolerance of
 the few-token tests each shape is held to the error of that summation: K
 additions that round a partial sum of about sqrt(K) max|w| max|x| by 2^-24 each,
-independently, come to K 2^-24 max|w| max|x|; four times that is allowed (the
-Q4_K sub-block sums, carried in 22 bits, stay below it).
+independently, come to K 2^-24 max|w| max|x|; four times that is allowed.
 """
 
 from __future__ import annotations
@@ -137,3 +136,25 @@ def test_long_k_is_no_coarser_than_the_few_token_tiles(stream, oracle):
     finally:
         hip.destroy_graph(graph)
     assert many <= 1.03 * few, f"relative error {many:.3e}, few-token tiles {few:.3e}"
+
+
+@pytest.mark.parametrize("m,n,k", [(70, 300, 4096), (70, 64, 14336), (300, 14336, 512)])
+@pytest.mark.parametrize("scratch", [True, False])
+def test_q4_k_sums_past_binary16(stream, oracle, m, n, k, scratch):
+    """Positive activations whose sub-block sums reach 2^20, and the same over 64:
+    the sums are carried in full, so the outputs are the same but for the
+    factor, exactly."""
+    w = wl.q4_k_weights(870, n, k)
+    rng = np.random.default_rng(871)
+    x = rng.uniform(100.0, 1000.0, m * k).astype(np.float16)
+    large = (x * np.float16(64.0)).view(np.uint16)
+    s = stream if scratch else HipRuntime().foreign_stream()
+    try:
+        y, z = (_run(s, "q4_k", v, w, m, n, k) for v in (x.view(np.uint16), large))
+    finally:
+        if not scratch:
+            s.close()
+    rows = [0, 1, 31, 32, 63, 64, m - 1]
+    y64, max_w, max_x = _judge(oracle, "q4_k", x.view(np.uint16).reshape(m, k)[rows].reshape(-1), w, len(rows), n, k)
+    assert float(np.abs(y.reshape(m, n)[rows] - y64.reshape(len(rows), n)).max()) <= 4.0 * k * 2.0 ** -24 * max_w * max_x
+    assert np.array_equal(z, 64.0 * y)
