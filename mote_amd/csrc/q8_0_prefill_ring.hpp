@@ -8,9 +8,15 @@
 // block's 32 products per output are two v_mfma_f32_32x32x16_f16 from zero, and
 //   y += d C
 // in f32 once per block.  (The tiles of q4_0_prefill.hip carry v d as binary16
-// hi + lo, four MFMAs per block, and stay for other K and alignments.)  An
-// output that is not finite (an infinite or NaN scale or activation) is
-// recomputed element by element.
+// hi + lo, four MFMAs per block, and stay for other K and alignments.)
+//
+// Outputs that are not finite: with a finite scale a block's d C is infinite or
+// NaN just where its sum of (v d) x is.  With an infinite one, d C is NaN where C
+// is 0, and so is that sum (it has a zero or both signs); else d C is infinite,
+// where a zero value or activation, or both signs, make the sum NaN.  So a NaN
+// stands, and an infinity does unless one of the row's scales is not finite: then
+// those blocks are added up element by element.  (Recomputing every such output
+// by its thread took 30 ms where 300 x 4096 x 4096 has NaN activations.)
 //
 // An interval is 64 k (a block pair) of each half with one barrier, as in
 // q4_0_prefill_ring.hip: activations in three slots of swizzled 128-byte rows;
@@ -37,6 +43,27 @@
 
 namespace mote::kquant {
 namespace {
+
+// Whether one of `blocks` block scales from `row` on is not finite.
+__device__ inline bool q8_scales_not_finite(const uint8_t* row, uint32_t blocks) {
+    bool any = false;
+#pragma unroll 8
+    for (uint32_t b = 0; b < blocks; ++b)
+        any |= (*reinterpret_cast<const uint16_t*>(row + b * 34u) & 0x7C00u) == 0x7C00u;
+    return any;
+}
+// The output that came out as the infinity v: NaN if the sum over a block whose
+// scale is not finite is.
+__device__ inline float q8_infinite(float v, const uint8_t* row, const uint16_t* xrow, uint32_t blocks) {
+    for (uint32_t b = 0; b < blocks; ++b) {
+        if (!q8_scales_not_finite(row + b * 34u, 1)) continue;
+        float s = 0.0f;
+        for (uint32_t e = 0; e < 32; ++e)
+            s += half_bits_to_float(xrow[b * 32 + e]) * kq_value<Fmt::Q8>(row + b * 34u, e);
+        if (s != s) return s;
+    }
+    return v;
+}
 
 template <int TM, bool SK, typename OutT>
 __global__ __launch_bounds__(512) void q8_prefill_kernel(const uint16_t* __restrict__ x, const uint8_t* __restrict__ w,
@@ -276,6 +303,15 @@ __global__ __launch_bounds__(512) void q8_prefill_kernel(const uint16_t* __restr
     // Lane (r, c) holds column r of each tile, rows 8 (k / 4) + 4 c + k % 4.
     const uint32_t n = n0 + wn * 32 + lr;
     if (n >= N) return;
+    const uint8_t* const wrow = w + (static_cast<size_t>(n) * nb + pb0) * BB;
+    const uint32_t blocks = (pb1 - pb0) * 8;
+    auto infinite = [](float v) { return (__builtin_bit_cast(uint32_t, v) & 0x7FFFFFFFu) == 0x7F800000u; };
+    bool inf = false;
+#pragma unroll
+    for (int i = 0; i < H; ++i)
+#pragma unroll
+        for (int k = 0; k < 16; ++k) inf |= i < kept && infinite(acc[i][k]);
+    const bool recompute = wave_any(inf) && q8_scales_not_finite(wrow, blocks);
 #pragma unroll
     for (int i = 0; i < H; ++i) {
         if (i >= kept) break;
@@ -284,9 +320,8 @@ __global__ __launch_bounds__(512) void q8_prefill_kernel(const uint16_t* __restr
             const uint32_t m = m0 + (tile0 + i) * 32 + 8 * (k / 4) + 4 * lc + k % 4;
             if (m >= M) continue;
             float v = acc[i][k];
-            if (__builtin_expect(not_finite(v), 0))
-                v = kq_exact_thread<Fmt::Q8>(w + (static_cast<size_t>(n) * nb + pb0) * BB,
-                                             x + static_cast<size_t>(m) * K + static_cast<size_t>(pb0) * kSuper, pb1 - pb0);
+            if (__builtin_expect(recompute, 0) && infinite(v))
+                v = q8_infinite(v, wrow, x + static_cast<size_t>(m) * K + static_cast<size_t>(pb0) * kSuper, blocks);
             if constexpr (SK)
                 partial[(static_cast<size_t>(part) * M + m) * N + n] = v;
             else

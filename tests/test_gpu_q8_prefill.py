@@ -11,8 +11,10 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
-from helpers import bits_to_f32, block_scales, linear_f64_full
+from helpers import bits_to_f32, block_scales, linear_f64_full, linear_tolerance, wide_q8_0_weights
 from mote_amd import ops, workloads as wl
+from mote_amd.device import DeviceBuffer
+from mote_amd.hip_runtime import HipRuntime
 from test_gpu_q8_0 import check, normal_x, run, weights
 
 pytestmark = pytest.mark.gpu
@@ -60,3 +62,65 @@ def test_dispatched_ragged_k(stream, oracle, m, n, k):
     """The linear's own choice at K a multiple of 128 only."""
     x, w = normal_x(wl.seed_for(73, m + k), m, k), weights(wl.seed_for(73, n + k), n, k)
     check(oracle, run(stream, x, w, m, n, k), x, w, m, n, k, what=f"{m}x{n}x{k}")
+
+
+@pytest.mark.parametrize("m,n,k", [(70, 100, 1024), (130, 60, 9472)])
+@pytest.mark.parametrize("scales", ["full", "special"])
+@pytest.mark.parametrize("special_x", [False, True])
+def test_exact_tiles_not_finite(stream, oracle, m, n, k, scales, special_x):
+    """Infinite and NaN scales and activations, and both: the outputs' NaN and
+    infinities are where the f64 judge has them."""
+    rng = np.random.default_rng(74 + k)
+    w = wide_q8_0_weights(75 + n, n, k, scales)
+    if scales == "special":  # few of the blocks, so that not every output is NaN
+        keep = wide_q8_0_weights(75 + n, n, k, "full").reshape(-1, 34)
+        pick = rng.random(len(keep)) < 0.05
+        w = np.where(pick[:, None], w.reshape(-1, 34), keep)
+        # blocks of one sign: with x > 0, infinite sums that stay infinite
+        w[pick & (rng.random(len(keep)) < 0.5), 2:] = 3
+        w = w.reshape(-1)
+    x = normal_x(wl.seed_for(76, k), m, k).copy()
+    x[: m * k // 2] &= 0x7FFF
+    if special_x:
+        at = rng.choice(x.size, m // 4, replace=False)
+        x[at] = rng.choice(np.array([0x7C00, 0xFC00, 0x7E00], dtype=np.uint16), at.size)
+    d = ops.Q4_0Dispatch()
+    d.force("q8_mfma_x32s_m128_n128_w1_k2")
+    y = run(stream, x, w, m, n, k, dispatch=d)
+    y64 = linear_f64_full(oracle, x, w, m, n, k, oracle.Q8_0)
+    for cls in (np.isnan, np.isposinf, np.isneginf):
+        assert np.array_equal(cls(y), cls(y64)), f"{cls.__name__}: {int(cls(y).sum())} against {int(cls(y64).sum())}"
+    if scales == "special":
+        assert np.isinf(y64).any() and np.isnan(y64).any()
+    scale = np.abs(block_scales(w, n, k, 34))
+    max_d, max_x = float(scale[np.isfinite(scale)].max()), np.abs(bits_to_f32(x))
+    ok = np.isfinite(y64)
+    tol = linear_tolerance(y64, k, max_d, float(max_x[np.isfinite(max_x)].max()))
+    assert np.all(np.abs(y[ok] - y64[ok]) <= tol[ok])
+
+
+def test_not_finite_activations_cost_no_more(stream):
+    """300 tokens of NaN, and of one infinity each, against finite ones: the time of
+    a call may triple at most (recomputed output by output it grows a
+    hundredfold)."""
+    m, n, k = 300, 4096, 4096
+    hip = HipRuntime()
+    w = DeviceBuffer.from_array(weights(wl.seed_for(77, n), n, k))
+    x = normal_x(wl.seed_for(77, k), m, k)
+    nan, inf = np.full_like(x, 0x7E00), x.copy()
+    inf[5::k] = 0x7C00
+    y = DeviceBuffer(m * n * 4)
+    times = []
+    begin, end = hip.create(), hip.create()
+    for bits in (x, nan, inf):
+        xb = DeviceBuffer.from_array(bits)
+        best = 1e9
+        for _ in range(4):
+            hip.record(begin, stream)
+            ops.quantized_linear_q8_0_f32(xb.ptr, w.ptr, y.ptr, m, n, k, stream)
+            hip.record(end, stream)
+            best = min(best, hip.elapsed_ms(begin, end))
+        times.append(best)
+    for e in (begin, end):
+        hip.destroy(e)
+    assert max(times) <= 3.0 * times[0], f"finite, NaN, infinite: {times} ms"
