@@ -158,3 +158,30 @@ def test_q4_k_sums_past_binary16(stream, oracle, m, n, k, scratch):
     y64, max_w, max_x = _judge(oracle, "q4_k", x.view(np.uint16).reshape(m, k)[rows].reshape(-1), w, len(rows), n, k)
     assert float(np.abs(y.reshape(m, n)[rows] - y64.reshape(len(rows), n)).max()) <= 4.0 * k * 2.0 ** -24 * max_w * max_x
     assert np.array_equal(z, 64.0 * y)
+
+
+@pytest.mark.parametrize("name", list(FORMATS))
+def test_many_tokens_not_finite_time(stream, name):
+    """300 tokens of NaN, and of one infinity each: every output is not finite and
+    is looked at again over the activations that make it so.  That takes some 50
+    times a finite call; over all elements, in one lane each, it took 1000."""
+    m, n, k = 300, 4096, 4096
+    hip, linear = HipRuntime(), FORMATS[name][2]
+    w = DeviceBuffer.from_array((wl.q4_k_weights if name == "q4_k" else wl.q6_k_weights)(880, n, k))
+    x = wl.normal_f16(881, m * k)
+    nan, inf = np.full_like(x, 0x7E00), x.copy()
+    inf[5::k] = 0x7C00
+    y = DeviceBuffer(m * n * 4)
+    begin, end, times = hip.create(), hip.create(), []
+    for bits in (x, nan, inf):
+        xb = DeviceBuffer.from_array(bits)
+        best = 1e9
+        for _ in range(3):
+            hip.record(begin, stream)
+            linear(xb.ptr, w.ptr, y.ptr, m, n, k, stream)
+            hip.record(end, stream)
+            best = min(best, hip.elapsed_ms(begin, end))
+        times.append(best)
+    for e in (begin, end):
+        hip.destroy(e)
+    assert max(times) <= 200.0 * times[0], f"{name}: finite, NaN, infinite {times} ms"
