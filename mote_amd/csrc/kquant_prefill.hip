@@ -518,21 +518,21 @@ __global__ __launch_bounds__(64 * kTileWaves * kTileGroups) void kq_prefill_kern
 
     if (ns > 0) {  // uniform over the wave; groups without work only meet the barriers
         load_sums(0);
-        issue_fence();
+        order_fence();
         load_a(0, 0);
-        issue_fence();
+        order_fence();
         load_a(1, 1);
-        issue_fence();
+        order_fence();
         load_quants(I1{}, 0);
-        issue_fence();
+        order_fence();
         load_a(2, 2);
-        issue_fence();
+        order_fence();
         load_head(0);
-        issue_fence();
+        order_fence();
         load_a(3, 3);
-        issue_fence();
+        order_fence();
         load_quants(I3{}, 0);
-        issue_fence();
+        order_fence();
         wait_counts<vm_wait(3 * NA + (kQ4 ? 5 : 8) * TN)>();  // interval 0's activations
     }
     group_barrier();
@@ -567,7 +567,7 @@ __global__ __launch_bounds__(64 * kTileWaves * kTileGroups) void kq_prefill_kern
                 add_slice(pc, I2{});
                 decode(pc, I3{}, b[1]);
             });
-            issue_fence();
+            order_fence();
             // The next interval's activations have landed (what may be
             // outstanding is all younger), and every wave has read this one's.
             wait_counts<vm_wait(2 * NA + kBehind[(P + 1) & 3] + kBehind[(P + 2) & 3] + kBehind[(P + 3) & 3]) &
@@ -576,11 +576,11 @@ __global__ __launch_bounds__(64 * kTileWaves * kTileGroups) void kq_prefill_kern
             order_fence();
             read_a((P + 1) & 3, 0, a[0]);
             load_a(4 * s + P + 4, P);
-            issue_fence();
+            order_fence();
             load_quants(pc, s + 1);
             if constexpr (P == 2) load_head(s + 1);
             if constexpr (P == 0) load_sums(s + 1);
-            issue_fence();
+            order_fence();
             minimum(pc, I3{}, s, [&] {
                 multiply(I1{});
                 add_slice(pc, I3{});

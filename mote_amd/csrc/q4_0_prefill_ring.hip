@@ -219,10 +219,15 @@ __global__ __launch_bounds__(64 * WN * kGroups) void prefill_ring_kernel(
 
     if (ns > 0) {  // uniform over the wave; a half without work only meets the barriers
         load_x(0, 0);
+        order_fence();
         load_w(0, 0);
+        order_fence();
         load_x(1, 1);
+        order_fence();
         load_w(1, 1);
+        order_fence();
         load_x(2, 2);
+        order_fence();
         wait_counts<vm_wait(2 * NX + kLoadsW)>();
     }
     group_barrier();
@@ -244,6 +249,7 @@ __global__ __launch_bounds__(64 * WN * kGroups) void prefill_ring_kernel(
                 rescale(big ? kQ4BigDown : 1.0f / kQ4BigDown);
             }
             load_w(t + 2, P & 1);  // this interval's pairs are in registers
+            memory_fence();
             read_x(slot, 1, a[1]);
             multiply(0);
             decode(I1{}, b[1]);
@@ -255,6 +261,7 @@ __global__ __launch_bounds__(64 * WN * kGroups) void prefill_ring_kernel(
             read_x(slot, 3, a[1]);
             // interval t + 1 has landed (at most t + 2's loads are outstanding)
             wait_counts<vm_wait(NX + kLoadsW)>();
+            memory_fence();
             read_w((P + 1) & 1);
             multiply(0);
             decode(I3{}, b[1]);
@@ -265,6 +272,7 @@ __global__ __launch_bounds__(64 * WN * kGroups) void prefill_ring_kernel(
             order_fence();
             read_x(next, 0, a[0]);
             load_x(t + 3, slot);
+            memory_fence();
             multiply(1);
             unpack(PN{});
             decode(I0{}, b[0]);

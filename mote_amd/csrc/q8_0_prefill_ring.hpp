@@ -205,10 +205,15 @@ __global__ __launch_bounds__(512) void q8_prefill_kernel(const uint16_t* __restr
 
     if (ns > 0) {  // uniform over the wave; a half without work only meets the barriers
         load_x(0, 0);
+        order_fence();
         load_w(0, 0);
+        order_fence();
         load_x(1, 1);
+        order_fence();
         load_w(1, 1);
+        order_fence();
         load_x(2, 2);
+        order_fence();
         wait_counts<vm_wait(2 * NX + NW)>();
     }
     group_barrier();
@@ -226,6 +231,7 @@ __global__ __launch_bounds__(512) void q8_prefill_kernel(const uint16_t* __restr
             using PN = std::integral_constant<int, (P + 1) & 3>;
             const uint32_t next = slot == kSlotsX - 1 ? 0 : slot + 1;
             load_w(t + 2, P & 1);  // this interval's pairs are in registers
+            memory_fence();
             read_x(slot, 1, a[1]);
             multiply_first(d_before);
             decode(I1{}, b[1]);
@@ -237,6 +243,7 @@ __global__ __launch_bounds__(512) void q8_prefill_kernel(const uint16_t* __restr
             read_x(slot, 3, a[1]);
             // interval t + 1 has landed (at most t + 2's loads are outstanding)
             wait_counts<vm_wait(NX + NW)>();
+            memory_fence();
             read_w((P + 1) & 1);
             multiply_first(d[0]);
             decode(I3{}, b[1]);
@@ -247,6 +254,7 @@ __global__ __launch_bounds__(512) void q8_prefill_kernel(const uint16_t* __restr
             order_fence();
             read_x(next, 0, a[0]);
             load_x(t + 3, slot);
+            memory_fence();
             multiply();
             d_before = d[1];
             unpack(PN{});

@@ -31,12 +31,14 @@ __device__ __forceinline__ void load_lds16(const uint8_t* src, uint8_t* dst) {
 }
 template <int I>
 __device__ __forceinline__ void wait_counts() { __builtin_amdgcn_s_waitcnt(I); }
-__device__ __forceinline__ void order_fence() { __builtin_amdgcn_sched_barrier(0); }
 // Keeps memory operations on their side of this point, in the compiler's
 // intermediate code and in its schedule: counted waits rely on the
-// order in which the loads are issued.
-__device__ __forceinline__ void issue_fence() {
-    asm volatile("" ::: "memory");
+// order in which the loads are issued, LDS reads on staying behind the wait and
+// the barrier that their data needs.
+__device__ __forceinline__ void memory_fence() { asm volatile("" ::: "memory"); }
+// ... and everything else on its side in the schedule.
+__device__ __forceinline__ void order_fence() {
+    memory_fence();
     __builtin_amdgcn_sched_barrier(0);
 }
 __device__ __forceinline__ void group_barrier() { __builtin_amdgcn_s_barrier(); }
