@@ -145,6 +145,17 @@ int mote_hip_quantized_linear_q6_k_f32(const void* input, const void* weights, v
                                        uint64_t rows, uint64_t output_features,
                                        uint64_t input_features, void* stream);
 
+/* [new] A Q8_0, Q4_K or Q6_K linear (format: the GGML type 8, 12 or 14) on one
+ * form of the many-token tiles: tile_rows 64, 96 or 128, K divided into k_parts
+ * (0: one part, no scratch; Q4_K then not on 128 rows).  The linears choose
+ * among these themselves; tests use it to run each on the same problem.  K a
+ * multiple of 256 up to 2^22, input and weights (Q6_K: 2-byte) 16-byte aligned;
+ * 1 for anything else, 801 (hipErrorNotSupported) where the stream has no
+ * prompt scratch for it, else the launch status. */
+int mote_hip_prompt_linear_tiles(int format, const void* input, const void* weights, void* output,
+                                 uint64_t rows, uint64_t output_features, uint64_t input_features,
+                                 int output_f16, int tile_rows, int k_parts, void* stream);
+
 /* [new] On-device decode of rows x K elements to f32 (output 4-byte
  * aligned), bit-identical to GGML's dequantize_row_q4_K / dequantize_row_q6_K.
  * Status: null, K % 256 != 0 or misaligned -> 1; empty -> 0. */
@@ -172,7 +183,11 @@ int mote_q4_0_dispatch_set_autotune(void* handle, int enabled);
  * second kernel adds them in the same order.  Results are bit-identical. */
 int mote_q4_0_dispatch_set_splitk_fold(void* handle, int enabled);
 /* Forces one variant by name (NULL or "" clears); tests use it to run every
- * kernel on the same problem. */
+ * kernel on the same problem.  A forced Q4_0 prompt variant runs its own tiles
+ * over all of K, where the unforced one may choose 128-row tiles over K parts;
+ * "name/P" (128-row multi-pair linear tiles, P = 2 to 8) runs it over P parts.
+ * The multi-pair Q8_0 names run the exact-integer tiles of their own choice
+ * where K is a multiple of 256. */
 int mote_q4_0_dispatch_force_variant(void* handle, const char* name);
 int mote_q4_0_dispatch_linear(void* handle, const void* input, const void* weights,
                               void* output, uint64_t rows, uint64_t output_features,

@@ -57,6 +57,7 @@ SIGNATURES = {
     "mote_hip_quantized_linear_q4_k_f32": (_I, [_P, _P, _P, _U64, _U64, _U64, _P]),
     "mote_hip_quantized_linear_q6_k_f16": (_I, [_P, _P, _P, _U64, _U64, _U64, _P]),
     "mote_hip_quantized_linear_q6_k_f32": (_I, [_P, _P, _P, _U64, _U64, _U64, _P]),
+    "mote_hip_prompt_linear_tiles": (_I, [_I, _P, _P, _P, _U64, _U64, _U64, _I, _I, _I, _P]),
     "mote_hip_dequantize_q4_k_f32": (_I, [_P, _P, _U64, _U64, _P]),
     "mote_hip_dequantize_q6_k_f32": (_I, [_P, _P, _U64, _U64, _P]),
     "mote_q4_0_dispatch_create": (_I, [ctypes.POINTER(_P)]),

@@ -61,6 +61,7 @@
 // token counts and grids that 128-row tiles fill badly (300 x 4096 x 14 336: 65
 // us on 96-row tiles).  The Q8_0 linear has a kernel of its own
 // (q8_0_prefill_ring.hpp) and shares the launch.
+#include "export.hpp"
 #include "kquant_blocks.hpp"
 #include "q4_0.hpp"
 #include "q8_0_prefill_ring.hpp"
@@ -830,8 +831,10 @@ bool worth(Fmt f, uint32_t M, uint32_t N, uint32_t K) {
     return (f == Fmt::Q4K ? choose<Fmt::Q4K>(M, N, K) : choose<Fmt::Q6K>(M, N, K)).us + 1.5 < 0.95 * few;
 }
 
+// forced: this plan, parts 0 for one part without scratch; null: the rule's.
 template <Fmt F, typename OutT>
-hipError_t launch(const void* x, const void* w, void* y, uint32_t M, uint32_t N, uint32_t K, hipStream_t stream) {
+hipError_t launch(const void* x, const void* w, void* y, uint32_t M, uint32_t N, uint32_t K, hipStream_t stream,
+                  const Plan* forced = nullptr) {
     const auto* xp = static_cast<const uint16_t*>(x);
     const auto* wp = static_cast<const uint8_t*>(w);
     auto* yp = static_cast<OutT*>(y);
@@ -842,7 +845,8 @@ hipError_t launch(const void* x, const void* w, void* y, uint32_t M, uint32_t N,
                : p.tm == 3 ? launch_tile<F, 3, OutT>(xm, wp, ym, rows, N, K, p.parts, planes, sums, stream)
                            : launch_tile<F, 2, OutT>(xm, wp, ym, rows, N, K, p.parts, planes, sums, stream);
     };
-    const Plan plan = choose<F>(M, N, K);
+    if (forced && forced->parts == 0) return run({forced->tm, 1, 0.0}, 0, M, nullptr, nullptr);
+    const Plan plan = forced ? *forced : choose<F>(M, N, K);
     const uint64_t row_sums = F == Fmt::Q4K ? static_cast<uint64_t>(K / kSuper) * 64 : 0;
     if (plan.parts == 1 && row_sums == 0) return run(plan, 0, M, nullptr, nullptr);
     // Tokens whose sums do not fit beside the planes run in turns, whole tiles
@@ -859,7 +863,7 @@ hipError_t launch(const void* x, const void* w, void* y, uint32_t M, uint32_t N,
         plan.parts > 1 ? (static_cast<uint64_t>(step) * N * plan.parts * sizeof(float) + 15) / 16 * 16 : 0;
     q4_0::ScratchPool::Lease lease;  // holds the scratch until every kernel is queued
     const hipError_t a = q4_0::acquire_prompt_scratch(stream, plane_bytes + row_sums * step, &lease);
-    if (a == hipErrorNotSupported) {
+    if (a == hipErrorNotSupported && !forced) {
         if (M <= 64 && F != Fmt::Q8) return a;  // the kernels of few tokens
         return run(choose<F>(M, N, K, false), 0, M, nullptr, nullptr);
     }
@@ -876,22 +880,57 @@ hipError_t launch(const void* x, const void* w, void* y, uint32_t M, uint32_t N,
 
 }  // namespace
 
-bool prefill_supported(Fmt f, const void* x, const void* w, uint32_t M, uint32_t N, uint32_t K) {
-    return K % kSuper == 0 && K >= kSuper && worth(f, M, N, K) && K <= (1u << 22) && static_cast<uint64_t>(M) * (K / kSuper) <= (1ull << 31) &&
+namespace {
+bool fits(Fmt f, const void* x, const void* w, uint32_t M, uint32_t K) {
+    return K % kSuper == 0 && K >= kSuper && K <= (1u << 22) && static_cast<uint64_t>(M) * (K / kSuper) <= (1ull << 31) &&
            (reinterpret_cast<uintptr_t>(x) & 15u) == 0 &&
-           (f == Fmt::Q6K || (reinterpret_cast<uintptr_t>(w) & 15u) == 0);
+           (reinterpret_cast<uintptr_t>(w) & (f == Fmt::Q6K ? 1u : 15u)) == 0;
+}
+
+hipError_t launch_any(Fmt f, bool f16_out, const void* x, const void* w, void* y, uint32_t M, uint32_t N, uint32_t K,
+                      hipStream_t stream, const Plan* forced) {
+    if (f == Fmt::Q8)
+        return f16_out ? launch<Fmt::Q8, _Float16>(x, w, y, M, N, K, stream, forced)
+                       : launch<Fmt::Q8, float>(x, w, y, M, N, K, stream, forced);
+    if (f == Fmt::Q4K)
+        return f16_out ? launch<Fmt::Q4K, _Float16>(x, w, y, M, N, K, stream, forced)
+                       : launch<Fmt::Q4K, float>(x, w, y, M, N, K, stream, forced);
+    return f16_out ? launch<Fmt::Q6K, _Float16>(x, w, y, M, N, K, stream, forced)
+                   : launch<Fmt::Q6K, float>(x, w, y, M, N, K, stream, forced);
+}
+}  // namespace
+
+bool prefill_supported(Fmt f, const void* x, const void* w, uint32_t M, uint32_t N, uint32_t K) {
+    return fits(f, x, w, M, K) && worth(f, M, N, K);
 }
 
 hipError_t launch_prefill(Fmt f, bool f16_out, const void* x, const void* w, void* y, uint32_t M, uint32_t N,
                           uint32_t K, hipStream_t stream) {
-    if (f == Fmt::Q8)
-        return f16_out ? launch<Fmt::Q8, _Float16>(x, w, y, M, N, K, stream)
-                       : launch<Fmt::Q8, float>(x, w, y, M, N, K, stream);
-    if (f == Fmt::Q4K)
-        return f16_out ? launch<Fmt::Q4K, _Float16>(x, w, y, M, N, K, stream)
-                       : launch<Fmt::Q4K, float>(x, w, y, M, N, K, stream);
-    return f16_out ? launch<Fmt::Q6K, _Float16>(x, w, y, M, N, K, stream)
-                   : launch<Fmt::Q6K, float>(x, w, y, M, N, K, stream);
+    return launch_any(f, f16_out, x, w, y, M, N, K, stream, nullptr);
 }
 
 }  // namespace mote::kquant
+
+MOTE_EXPORT int mote_hip_prompt_linear_tiles(int format, const void* input, const void* weights, void* output,
+                                             uint64_t rows, uint64_t output_features, uint64_t input_features,
+                                             int output_f16, int tile_rows, int k_parts, void* stream) noexcept {
+    using namespace mote::kquant;
+    if (!input || !weights || !output || !stream) return hipErrorInvalidValue;
+    if (format != 8 && format != 12 && format != 14) return hipErrorInvalidValue;
+    if (tile_rows != 64 && tile_rows != 96 && tile_rows != 128) return hipErrorInvalidValue;
+    const Fmt f = format == 8 ? Fmt::Q8 : format == 12 ? Fmt::Q4K : Fmt::Q6K;
+    if (k_parts < 0 || (k_parts == 0 && f == Fmt::Q4K && tile_rows == 128)) return hipErrorInvalidValue;
+    if (rows == 0 || output_features == 0 || rows > UINT32_MAX || output_features > UINT32_MAX / rows ||
+        input_features > (1u << 22))
+        return hipErrorInvalidValue;
+    const auto M = static_cast<uint32_t>(rows), N = static_cast<uint32_t>(output_features);
+    const auto K = static_cast<uint32_t>(input_features);
+    if (!fits(f, input, weights, M, K) || static_cast<uint32_t>(k_parts) > K / kSuper) return hipErrorInvalidValue;
+    try {
+        const Plan plan{tile_rows / 32, static_cast<uint32_t>(k_parts), 0.0};
+        return static_cast<int>(launch_any(f, output_f16 != 0, input, weights, output, M, N, K,
+                                           static_cast<hipStream_t>(stream), &plan));
+    } catch (...) {
+        return hipErrorUnknown;
+    }
+}

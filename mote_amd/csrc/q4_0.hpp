@@ -29,6 +29,9 @@ struct Problem {
     // MI355X the fold measured slower (its workgroups wait for their
     // write-through partial stores and the arrival atomic before exiting).
     bool splitk_fold = false;
+    // Prompt tiles of the linear: 0, K parts where that is the faster choice;
+    // else a forced variant's own tiles, over so many.
+    uint32_t ring_parts = 0;
 };
 
 // Split-K scratch layout: kSplitKCounterBytes of per-tile arrival counters
@@ -70,7 +73,7 @@ bool prefill_supports(const Variant& v, const Problem& p);
 // (q4_0_prefill_ring.hip): the problems it takes, and a launch of its bm x bn
 // tiles (128 x 256, 128 x 128; gate/up 128 x 128).
 bool prefill_ring_supports(const Problem& p);
-hipError_t launch_prefill_ring(const Problem& p, int bm, int bn, bool gate_up);
+hipError_t launch_prefill_ring(const Problem& p, int bm, int bn, bool gate_up, uint32_t parts = 1);
 // The linear on 128-row ring tiles over K parts where that is faster than bm x
 // bn tiles over all of K; hipErrorNotSupported, with nothing queued, where it is
 // not or the stream has no scratch for the parts.

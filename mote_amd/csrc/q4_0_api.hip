@@ -49,8 +49,20 @@ struct Dispatcher {
     bool autotune = false;
     bool splitk_fold = false;
     std::string forced;
+    uint32_t forced_parts = 1;
     std::string last_error;
 };
+
+// "name", or "name/P" for P = 2 to 8 K parts.
+void force(Dispatcher& d, const std::string& name) {
+    const size_t slash = name.find('/');
+    d.forced = name;
+    d.forced_parts = 1;
+    if (slash + 2 == name.size() && name[slash + 1] >= '2' && name[slash + 1] <= '8') {
+        d.forced = name.substr(0, slash);
+        d.forced_parts = static_cast<uint32_t>(name[slash + 1] - '0');
+    }
+}
 
 std::vector<const Variant*> all_variants() {
     std::vector<const Variant*> out;
@@ -912,6 +924,7 @@ int run(Dispatcher& d, const Problem& problem, Op op) {
     p.splitk_fold = d.splitk_fold;
     const Variant* v = nullptr;
     if (!d.forced.empty()) {
+        p.ring_parts = d.forced_parts;
         v = find_variant(d.forced);
         if (!v || !kind_matches(*v, op) || !supports(*v, p))
             return fail(&d, hipErrorInvalidValue,
@@ -976,6 +989,7 @@ int run_no_alloc(Dispatcher& d, const Problem& problem) {
     p.splitk_fold = d.splitk_fold;
     const Variant* v = nullptr;
     if (!d.forced.empty()) {
+        p.ring_parts = d.forced_parts;
         v = find_variant(d.forced);
         if (!v || !kind_matches(*v, Op::Linear) || !supports(*v, p)) return hipErrorInvalidValue;
     } else {
@@ -998,7 +1012,7 @@ Dispatcher& default_dispatcher() {
         const char* tune = std::getenv("MOTE_Q4_0_AUTOTUNE");
         x->autotune = tune && tune[0] == '1';
         const char* forced = std::getenv("MOTE_Q4_0_VARIANT");
-        if (forced) x->forced = forced;
+        if (forced) force(*x, forced);
         return x;
     }();
     return *d;
@@ -1375,11 +1389,15 @@ MOTE_EXPORT int mote_q4_0_dispatch_force_variant(void* handle, const char* name)
         d->forced.clear();
         return 0;
     }
-    if (!find_variant(name)) {
+    Dispatcher wanted;
+    force(wanted, name);
+    const Variant* v = find_variant(wanted.forced);
+    if (!v || (wanted.forced_parts > 1 && v->kind != Kind::Mfma)) {
         d->last_error = std::string("unknown Q4_0 variant '") + name + "'";
         return hipErrorInvalidValue;
     }
-    d->forced = name;
+    d->forced = wanted.forced;
+    d->forced_parts = wanted.forced_parts;
     return 0;
 }
 

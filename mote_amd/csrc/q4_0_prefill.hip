@@ -487,12 +487,15 @@ hipError_t launch_prefill(const Problem& p) {
     if constexpr (SPEC && T32 && KP > 1 && !Q8) {
         if (prefill_ring_supports(p)) {
             if constexpr (!GATE_UP) {
-                const hipError_t e = launch_prefill_ring_parts(p, BM, BN);
-                if (e != hipErrorNotSupported) return e;
+                if (p.ring_parts == 0) {
+                    const hipError_t e = launch_prefill_ring_parts(p, BM, BN);
+                    if (e != hipErrorNotSupported) return e;
+                }
             }
-            if constexpr (BM == 128) return launch_prefill_ring(p, BM, BN, GATE_UP);
+            if constexpr (BM == 128) return launch_prefill_ring(p, BM, BN, GATE_UP, p.ring_parts > 1 ? p.ring_parts : 1);
         }
     }
+    if (p.ring_parts > 1) return hipErrorInvalidValue;  // forced on tiles that take no parts
     // Multi-pair Q8_0 tiles: the exact-integer tiles where the operands fit them
     // (their own choice of rows per tile and K parts).
     if constexpr (SPEC && T32 && KP > 1 && Q8) {

@@ -452,11 +452,11 @@ hipError_t launch_prefill_ring_parts(const Problem& p, int bm, int bn) {
     return tile == 256 ? launch_ring<4, 4, false>(p, parts) : launch_ring<4, 2, false>(p, parts);
 }
 
-hipError_t launch_prefill_ring(const Problem& p, int bm, int bn, bool gate_up) {
+hipError_t launch_prefill_ring(const Problem& p, int bm, int bn, bool gate_up, uint32_t parts) {
     if (bm != 128) return hipErrorInvalidValue;
-    if (gate_up) return bn == 128 ? launch_ring<4, 4, true>(p, 1) : hipErrorInvalidValue;
-    return bn == 256   ? launch_ring<4, 4, false>(p, 1)
-           : bn == 128 ? launch_ring<4, 2, false>(p, 1)
+    if (gate_up) return bn == 128 && parts == 1 ? launch_ring<4, 4, true>(p, 1) : hipErrorInvalidValue;
+    return bn == 256   ? launch_ring<4, 4, false>(p, parts)
+           : bn == 128 ? launch_ring<4, 2, false>(p, parts)
                        : hipErrorInvalidValue;
 }
 

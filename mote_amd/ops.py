@@ -66,6 +66,14 @@ def quantized_linear_q6_k_f32(x, w, y, rows, n, k, stream) -> None:
     check(lib().mote_hip_quantized_linear_q6_k_f32(x, w, y, rows, n, k, _s(stream)), "launch Q6_K linear kernel")
 
 
+def prompt_linear_tiles(fmt, x, w, y, rows, n, k, stream, tile_rows, k_parts, f16_out: bool = False) -> None:
+    """A "q8_0", "q4_k" or "q6_k" linear on one form of the many-token tiles
+    (k_parts 0: without scratch), for tests."""
+    ggml_type = {"q8_0": 8, "q4_k": 12, "q6_k": 14}[fmt]
+    check(lib().mote_hip_prompt_linear_tiles(ggml_type, x, w, y, rows, n, k, int(f16_out), tile_rows, k_parts,
+                                             _s(stream)), "launch prompt tiles")
+
+
 def dequantize_q4_k_f32(w, out, rows, k, stream) -> None:
     check(lib().mote_hip_dequantize_q4_k_f32(w, out, rows, k, _s(stream)), "launch Q4_K decode kernel")
 

@@ -110,6 +110,20 @@ def test_k_quant_status_codes(lib):
         assert d(FAKE, FAKE, 4, 0, STREAM) == 0
 
 
+def test_prompt_tiles_status_codes(lib):
+    fn = lib.mote_hip_prompt_linear_tiles
+    good = [8, FAKE, FAKE, FAKE, 65, 5, 256, 0, 64, 1, STREAM]
+    bad = {0: [4, 10, 13], 1: [None, FAKE + 8], 2: [None, FAKE + 8], 3: [None], 4: [0, 1 << 32], 5: [0, 1 << 31],
+           6: [0, 128, 384, (1 << 22) + 256], 8: [0, 32, 256], 9: [-1, 2], 10: [None]}
+    for at, values in bad.items():
+        for v in values:
+            args = list(good)
+            args[at] = v
+            assert fn(*args) == 1, (at, v)
+    assert fn(12, FAKE, FAKE, FAKE, 65, 5, 256, 0, 128, 0, STREAM) == 1  # Q4_K without scratch: 64 or 96 rows
+    assert fn(14, FAKE, FAKE + 1, FAKE, 65, 5, 256, 0, 64, 1, STREAM) == 1
+
+
 def test_norm_status_codes(lib):
     r = lib.mote_hip_rms_norm_f16
     assert r(None, FAKE, FAKE, 1, 8, 1e-6, STREAM) == -1

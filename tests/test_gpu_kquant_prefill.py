@@ -11,11 +11,13 @@ independently, come to K 2^-24 max|w| max|x|; four times that is allowed.
 
 from __future__ import annotations
 
+import functools
+
 import numpy as np
 import pytest
 
 from helpers import bits_to_f32
-from mote_amd import workloads as wl
+from mote_amd import ops, workloads as wl
 from mote_amd.device import DeviceBuffer, Stream
 from mote_amd.hip_runtime import HipRuntime
 from test_gpu_kquant import FORMATS, _blocks, _check, _fmt, _judge, _run
@@ -42,6 +44,16 @@ SHAPES = [
     # 96-row tiles
     (300, 14336, 256),
 ]
+# Every tile form on the same problems: 1, 2, 3, 5 and 9 super-blocks (an idle
+# second group, uneven groups, parts of one and short last parts), rows and columns one past
+# and short of a tile
+TILE_SHAPES = [(1, 1, 256), (33, 127, 512), (129, 128, 768), (257, 200, 1280), (95, 129, 2304)]
+# (format, (M, N, K), tile rows, K parts; 0: without scratch)
+TILES = [
+    (name, shape, rows, parts)
+    for name in ("q4_k", "q6_k") for shape in TILE_SHAPES for rows in (64, 96, 128) for parts in (0, 1, 2, 3, 5)
+    if parts <= shape[2] // 256 and (name, rows, parts) != ("q4_k", 128, 0)
+]
 
 
 @pytest.mark.parametrize("name", list(FORMATS))
@@ -57,6 +69,45 @@ def test_linear_many_tokens(stream, oracle, name, m, n, k):
     assert float(np.abs(y - y64).max()) <= bound, f"{name} {m}x{n}x{k}: past f32 summation of exact products"
     y16 = _run(stream, name, x, w, m, n, k, f16_out=True)
     _check(y16, y64, k, max_w, max_x, 2.0 ** -11, what=f"{name} {m}x{n}x{k} f16")
+
+
+@functools.lru_cache(maxsize=4)
+def _problem(name, m, n, k, special):
+    """Weights, activations and what the oracle says of them."""
+    import oracle
+
+    w = (wl.q4_k_weights if name == "q4_k" else wl.q6_k_weights)(860 + n, n, k)
+    x = wl.normal_f16(wl.seed_for(46, m + k), m * k).copy()
+    if special:
+        rng = np.random.default_rng(47 + k)
+        at = rng.choice(x.size, max(1, m // 4), replace=False)
+        x[at] = rng.choice(np.array([0x7C00, 0xFC00, 0x7E00], dtype=np.uint16), at.size)
+        blocks = w.reshape(n * k // 256, -1).copy()
+        bad = rng.random(len(blocks)) < 0.02
+        d = 0 if name == "q4_k" else 208
+        blocks[bad, d:d + 2] = np.array([0x00, 0x7C], dtype=np.uint8)  # infinite
+        w = blocks.reshape(-1)
+    x32, fmt = bits_to_f32(x), _fmt(oracle, name)
+    y64 = oracle.kquant_linear_f64(x32, w, fmt, m, n, k)
+    max_w = np.abs(oracle.dequantize_kquant_row(w, fmt, n * k))
+    return w, x, y64, float(max_w[np.isfinite(max_w)].max()), float(np.abs(x32)[np.isfinite(x32)].max())
+
+
+@pytest.mark.parametrize("special", [False, True])
+@pytest.mark.parametrize("name,shape,rows,parts", TILES)
+def test_every_tile(stream, name, shape, special, rows, parts):
+    m, n, k = shape
+    w, x, y64, max_w, max_x = _problem(name, m, n, k, special)
+    xb, wb, yb = DeviceBuffer.from_array(x), DeviceBuffer.from_array(w), DeviceBuffer(m * n * 4)
+    yb.upload(np.full(yb.nbytes, 0xA5, dtype=np.uint8))
+    ops.prompt_linear_tiles(name, xb.ptr, wb.ptr, yb.ptr, m, n, k, stream, rows, parts)
+    stream.synchronize()
+    y = yb.download(np.float32).reshape(y64.shape).astype(np.float64)
+    for cls in (np.isnan, np.isposinf, np.isneginf):
+        assert np.array_equal(cls(y), cls(y64)), f"{cls.__name__} positions differ"
+    ok = np.isfinite(y64)
+    bound = 4.0 * k * 2.0 ** -24 * max_w * max_x
+    assert float(np.abs(y[ok] - y64[ok]).max(initial=0.0)) <= bound, "past f32 summation of exact products"
 
 
 @pytest.mark.parametrize("name", list(FORMATS))

@@ -13,7 +13,9 @@ import pytest
 
 from helpers import bits_to_f32, wide_q4_0_weights
 from mote_amd import ops, workloads as wl
+from mote_amd._ffi import HipError
 from mote_amd.device import DeviceBuffer
+from test_gpu_q4_0 import check_against_oracle, run_linear, sample_columns
 
 pytestmark = pytest.mark.gpu
 
@@ -24,11 +26,11 @@ def _at(array, offset):
     return b, b.ptr + offset
 
 
-def _both(stream, call, x, weights, m, n, f16_out):
-    """The output with the weights on and off the 16-byte grid."""
+def _both(stream, call, x, weights, m, n, f16_out, other=None):
+    """The output with the weights on and off the 16-byte grid (there by `other`)."""
     out = []
     xb, xp = _at(x, 0)
-    for offset in (0, 4):
+    for offset, call in ((0, call), (4, other or call)):
         held = [_at(w, offset) for w in weights]
         yb = DeviceBuffer(m * n * (2 if f16_out else 4))
         yb.upload(np.full(yb.nbytes, 0xA5, dtype=np.uint8))
@@ -54,8 +56,9 @@ SHAPES = [
 @pytest.mark.parametrize("m,n,k", SHAPES)
 @pytest.mark.parametrize("scales", ["ordinary", "wide"])
 def test_ring_matches_staging_body(stream, variant, m, n, k, scales):
-    d = ops.Q4_0Dispatch()
-    d.force(variant)
+    d, staging = ops.Q4_0Dispatch(), ops.Q4_0Dispatch()
+    d.force(variant)  # its own tiles, or with "/P" the same over K parts
+    staging.force(variant.split("/")[0])
     x = wl.normal_f16(wl.seed_for(61, m + k), m * k)
     w = wl.q4_0_weights(wl.seed_for(61, n + k), n, k) if scales == "ordinary" else wide_q4_0_weights(62 + n, n, k, "full")
     max_d = float(np.abs(w.reshape(-1, 18)[:, 0:2].copy().view(np.float16).astype(np.float64)).max())
@@ -63,19 +66,52 @@ def test_ring_matches_staging_body(stream, variant, m, n, k, scales):
     for f16_out in (False, True):
         if f16_out and scales == "wide":
             continue  # past binary16's range
-        got, want = _both(stream, lambda xp, wp, yp: d.linear(xp, wp[0], yp, m, n, k, stream, f16_out=f16_out), x, [w],
-                          m, n, f16_out)
+        def call(dispatch):
+            return lambda xp, wp, yp: dispatch.linear(xp, wp[0], yp, m, n, k, stream, f16_out=f16_out)
+
+        got, want = _both(stream, call(d), x, [w], m, n, f16_out, call(staging))
         tol = bound + (2.0 ** -10 * np.abs(want) if f16_out else 0.0)
         assert np.all(np.abs(got - want) <= tol), f"{variant} {m}x{n}x{k}: {float(np.abs(got - want).max())} > {bound}"
 
 
-@pytest.mark.parametrize("variant", ["mfma_x32s_m64_n64_w2_k4", "mfma_x32s_m64_n128_w1_k4", "mfma_x32s_m128_n128_w1_k2"])
-@pytest.mark.parametrize("m,n,k", [(70, 96, 14336), (130, 129, 9472), (33, 257, 11008)])
+@pytest.mark.parametrize("variant", ["mfma_x32s_m128_n256_w1_k2", "mfma_x32s_m128_n128_w1_k2"])
+@pytest.mark.parametrize("parts", [2, 3, 8])
+@pytest.mark.parametrize("m,n,k", [(70, 96, 14336), (130, 257, 9472), (33, 300, 768), (128, 256, 256)])
 @pytest.mark.parametrize("scales", ["ordinary", "wide"])
-def test_k_parts_match_staging_body(stream, variant, m, n, k, scales):
-    """Few tiles and long K: 128-row ring tiles over K parts (a short last
-    part at K = 9472 and 11 008)."""
-    test_ring_matches_staging_body(stream, variant, m, n, k, scales)
+def test_k_parts_match_staging_body(stream, variant, parts, m, n, k, scales):
+    """K parts, with a short last part (K = 9472 over 3 and 8), parts of one
+    super-pair (the second half idle) and fewer parts than asked for."""
+    test_ring_matches_staging_body(stream, f"{variant}/{parts}", m, n, k, scales)
+
+
+@pytest.mark.parametrize("m,n,k", [(70, 96, 14336), (130, 129, 9472), (33, 257, 11008), (500, 14336, 512)])
+def test_dispatched_prompts(stream, oracle, m, n, k):
+    """The dispatcher's own choice, K parts among it, against the oracle."""
+    x, w = wl.normal_f16(wl.seed_for(64, m + k), m * k), wl.q4_0_weights(wl.seed_for(64, n + k), n, k)
+    y = run_linear(stream, x, w, m, n, k)
+    check_against_oracle(oracle, y, x, w, m, n, k, columns=sample_columns(n, 64), what=f"{m}x{n}x{k}")
+
+
+def test_forced_names():
+    d = ops.Q4_0Dispatch()
+    d.force("mfma_x32s_m128_n256_w1_k2/8")
+    assert d.select(512, 14336, 4096) == "mfma_x32s_m128_n256_w1_k2"
+    for name in ("mfma_x32s_m128_n256_w1_k2/1", "mfma_x32s_m128_n256_w1_k2/9", "mfma_x32s_m128_n256_w1_k2/",
+                 "mfma_x32s_m128_n256_w1_k2/22", "gateup_mfma_x32s_m128_n128_w1_k2/2", "/2", "q8_generic/2"):
+        with pytest.raises(HipError):
+            d.force(name)
+
+
+def test_parts_need_the_ring_tiles(stream):
+    """64-row tiles and weights off the 16-byte grid take no K parts."""
+    m, n, k = 70, 64, 1024
+    xb, wb = DeviceBuffer(m * k * 2), DeviceBuffer(n * k // 32 * 18 + 16)
+    yb = DeviceBuffer(m * n * 4)
+    d = ops.Q4_0Dispatch()
+    for name, offset in (("mfma_x32s_m64_n64_w2_k4/2", 0), ("mfma_x32s_m128_n128_w1_k2/2", 4)):
+        d.force(name)
+        with pytest.raises(HipError):
+            d.linear(xb.ptr, wb.ptr + offset, yb.ptr, m, n, k, stream)
 
 
 @pytest.mark.parametrize("m,n,k", [(128, 128, 256), (129, 127, 768), (200, 200, 1024)])

@@ -124,3 +124,31 @@ def test_not_finite_activations_cost_no_more(stream):
     for e in (begin, end):
         hip.destroy(e)
     assert max(times) <= 3.0 * times[0], f"finite, NaN, infinite: {times} ms"
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 1, 256), (33, 127, 512), (129, 128, 768), (257, 200, 1280), (95, 129, 2304)])
+@pytest.mark.parametrize("special", [False, True])
+def test_every_tile(stream, oracle, m, n, k, special):
+    """64-, 96- and 128-row tiles without scratch and over 1 to 5 K parts."""
+    w, x = weights(wl.seed_for(78, n), n, k), normal_x(wl.seed_for(78, k), m, k).copy()
+    if special:
+        rng = np.random.default_rng(79 + k)
+        at = rng.choice(x.size, max(1, m // 4), replace=False)
+        x[at] = rng.choice(np.array([0x7C00, 0xFC00, 0x7E00], dtype=np.uint16), at.size)
+        blocks = w.reshape(-1, 34).copy()
+        blocks[rng.random(len(blocks)) < 0.01, 0:2] = np.array([0x00, 0x7C], dtype=np.uint8)
+        w = blocks.reshape(-1)
+    y64 = linear_f64_full(oracle, x, w, m, n, k, oracle.Q8_0)
+    scale, max_x = np.abs(block_scales(w, n, k, 34)), np.abs(bits_to_f32(x))
+    bound = 4.0 * k * 2.0 ** -24 * 128.0 * float(scale[np.isfinite(scale)].max()) * float(max_x[np.isfinite(max_x)].max())
+    ok = np.isfinite(y64)
+    xb, wb, yb = DeviceBuffer.from_array(x), DeviceBuffer.from_array(w), DeviceBuffer(m * n * 4)
+    for rows in (64, 96, 128):
+        for parts in (p for p in (0, 1, 2, 3, 5) if p <= k // 256):
+            yb.upload(np.full(yb.nbytes, 0xA5, dtype=np.uint8))
+            ops.prompt_linear_tiles("q8_0", xb.ptr, wb.ptr, yb.ptr, m, n, k, stream, rows, parts)
+            stream.synchronize()
+            y = yb.download(np.float32).reshape(y64.shape).astype(np.float64)
+            for cls in (np.isnan, np.isposinf, np.isneginf):
+                assert np.array_equal(cls(y), cls(y64)), f"{rows} rows, {parts} parts: {cls.__name__} positions differ"
+            assert float(np.abs(y[ok] - y64[ok]).max(initial=0.0)) <= bound, f"{rows} rows, {parts} parts"
