@@ -816,19 +816,26 @@ Plan choose(uint32_t M, uint32_t N, uint32_t K, bool scratch = true) {
 }
 
 // Up to 64 tokens the few-token tiles of kquant.hip compete.  Their time is
-// about 4 us and 6.2 (Q4_K) or 13.3 ns (Q6_K) per item, (16 rows, 16 tokens, 16
-// super-blocks), twice that with three token tiles, and 3 us for a part sum
-// (64 x 4096 x 14 336 26 / 51 us, 48 x 4096 x 14 336 39 / 77, 64 x 4096 x 4096
-// 9.7 / 17.5, 64 x 14 336 x 4096 32 / 60, 32 x 14 336 x 4096 19 / 34); here the
-// same shapes take 23.4 / 30.3, 22.0 / 29.6, 17 / 19, 23.2 / 27.6, 22 / 26.5.
+// about 4 us, 1.2 + 0.33 s (Q4_K) or 2 + 0.73 s ns per item (16 rows, 16 tokens,
+// s super-blocks, at most 16), 1.9 times that with three token tiles and 1.6
+// times with three K parts (256 workgroups deal those out unevenly), and 3 us
+// for a part sum.  Of 1440 shapes (17 to 64 tokens, K 1024 to 16 384, N 1024 to
+// 32 768) the rule slows none by more than 1.1 % against the few-token tiles;
+// the largest gain it leaves is 28 %, and 64 x 14 336 x 32 768 goes from 221 (Q4_K)
+// and 455 us (Q6_K) to 100 and 168.  (With a time per item that left s out, K
+// below 4096 went up to 60 % slower: 32 x 1024 x 7168 Q6_K 12.9 us against 8.0, 32
+// x 2048 x 20 000 Q4_K 15.3 against 13.1.)
 bool worth(Fmt f, uint32_t M, uint32_t N, uint32_t K) {
     if (M > 64 || f == Fmt::Q8) return true;
     if (M <= 16) return false;
-    const uint32_t token_tiles = (M + 15) / 16, kparts = (K / kSuper + 15) / 16;
+    const uint32_t nb = K / kSuper, token_tiles = (M + 15) / 16, kparts = (nb + 15) / 16;
     const double items = static_cast<double>((N + 15) / 16) * token_tiles * kparts;
-    double few = 4.0 + items * (f == Fmt::Q4K ? 6.2e-3 : 13.3e-3) * (token_tiles == 3 ? 2.0 : 1.0);
+    const double s = nb < 16 ? nb : 16;
+    double few = 4.0 + items * (f == Fmt::Q4K ? 1.2 + 0.33 * s : 2.0 + 0.73 * s) * 1e-3 *
+                           (kparts == 3 ? 1.6 : token_tiles == 3 ? 1.9 : 1.0);
     if (kparts > 1) few += 3.0;
-    return (f == Fmt::Q4K ? choose<Fmt::Q4K>(M, N, K) : choose<Fmt::Q6K>(M, N, K)).us + 1.5 < 0.95 * few;
+    if (0.95 * few <= 2.5 + 5.0 + 1.45) return false;  // below every plan's time
+    return (f == Fmt::Q4K ? choose<Fmt::Q4K>(M, N, K) : choose<Fmt::Q6K>(M, N, K)).us + 2.5 < 0.95 * few;
 }
 
 // forced: this plan, parts 0 for one part without scratch; null: the rule's.

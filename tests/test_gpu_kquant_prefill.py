@@ -236,3 +236,30 @@ def test_many_tokens_not_finite_time(stream, name):
     for e in (begin, end):
         hip.destroy(e)
     assert max(times) <= 200.0 * times[0], f"{name}: finite, NaN, infinite {times} ms"
+
+
+@pytest.mark.parametrize("name,m,n,k,parts", [("q4_k", 24, 14336, 1024, 1), ("q6_k", 32, 7168, 1024, 2)])
+def test_short_k_keeps_the_few_token_tiles(stream, name, m, n, k, parts):
+    """Up to 64 tokens with short K the few-token tiles are the faster ones (7.3
+    against 10.7 us, 8.0 against 12.9): the linear does not take the many-token
+    form that fits best."""
+    hip, linear = HipRuntime(), FORMATS[name][2]
+    w = DeviceBuffer.from_array((wl.q4_k_weights if name == "q4_k" else wl.q6_k_weights)(890, n, k))
+    x, y = DeviceBuffer.from_array(wl.normal_f16(891, m * k)), DeviceBuffer(m * n * 4)
+    begin, end = hip.create(), hip.create()
+
+    def time(call):
+        best = 1e9
+        for _ in range(10):
+            hip.record(begin, stream)
+            for _ in range(50):
+                call()
+            hip.record(end, stream)
+            best = min(best, hip.elapsed_ms(begin, end))
+        return best
+
+    own = time(lambda: linear(x.ptr, w.ptr, y.ptr, m, n, k, stream))
+    many = time(lambda: ops.prompt_linear_tiles(name, x.ptr, w.ptr, y.ptr, m, n, k, stream, 64, parts))
+    for e in (begin, end):
+        hip.destroy(e)
+    assert own <= 0.9 * many, f"{name}: {own / 50 * 1e3:.2f} us, many-token tiles {many / 50 * 1e3:.2f}"
