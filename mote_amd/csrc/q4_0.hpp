@@ -73,6 +73,7 @@ bool prefill_supports(const Variant& v, const Problem& p);
 // (q4_0_prefill_ring.hip): the problems it takes, and a launch of its bm x bn
 // tiles (128 x 256, 128 x 128; gate/up 128 x 128).
 bool prefill_ring_supports(const Problem& p);
+bool prefill_ring_pays(const Problem& p, bool gate_up);  // against the staging-wave body of the same tiles
 hipError_t launch_prefill_ring(const Problem& p, int bm, int bn, bool gate_up, uint32_t parts = 1);
 // The linear on 128-row ring tiles over K parts where that is faster than bm x
 // bn tiles over all of K; hipErrorNotSupported, with nothing queued, where it is

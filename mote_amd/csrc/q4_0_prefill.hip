@@ -492,7 +492,9 @@ hipError_t launch_prefill(const Problem& p) {
                     if (e != hipErrorNotSupported) return e;
                 }
             }
-            if constexpr (BM == 128) return launch_prefill_ring(p, BM, BN, GATE_UP, p.ring_parts > 1 ? p.ring_parts : 1);
+            if constexpr (BM == 128)
+                if (p.ring_parts != 0 || prefill_ring_pays(p, GATE_UP))
+                    return launch_prefill_ring(p, BM, BN, GATE_UP, p.ring_parts > 1 ? p.ring_parts : 1);
         }
     }
     if (p.ring_parts > 1) return hipErrorInvalidValue;  // forced on tiles that take no parts

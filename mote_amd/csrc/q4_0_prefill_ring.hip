@@ -452,6 +452,17 @@ hipError_t launch_prefill_ring_parts(const Problem& p, int bm, int bn) {
     return tile == 256 ? launch_ring<4, 4, false>(p, parts) : launch_ring<4, 2, false>(p, parts);
 }
 
+// The rings fill and drain once per tile: with short K the staging-wave body of
+// the same tiles is the faster one.  Linear, this body against it in us: 65 x 256 x
+// 28 672 10.2 / 7.5, 100 x 1024 x 28 672 16.2 / 14.6, 256 x 1536 x 14 336 20.1 /
+// 19.5, 65 x 2048 x 28 672 23.7 / 22.9; from 2048 with more than one row of tiles it
+// gains (1 to 3 % on average there, 4 % at 4096).  Gate/up (less to hand over): 2048
+// x 768 x 28 672 287 / 260, 80 x 768 x 28 672 19.6 / 18.7; on average 1 % faster at
+// 1024, 2 to 4 % from 2048.
+bool prefill_ring_pays(const Problem& p, bool gate_up) {
+    return p.K >= (gate_up ? 1024u : p.M > 128 ? 2048u : 2304u);
+}
+
 hipError_t launch_prefill_ring(const Problem& p, int bm, int bn, bool gate_up, uint32_t parts) {
     if (bm != 128) return hipErrorInvalidValue;
     if (gate_up) return bn == 128 && parts == 1 ? launch_ring<4, 4, true>(p, 1) : hipErrorInvalidValue;

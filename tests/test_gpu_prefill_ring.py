@@ -130,3 +130,23 @@ def test_gate_up_ring_matches_staging_body(stream, m, n, k):
                       [wg.reshape(-1), wu.reshape(-1)], m, n, False)
     tol = 8.0 * 2.2 * e + 2.0 ** -20 * np.abs(want)  # factors below 8; the device exponential
     assert np.all(np.abs(got - want) <= tol), f"{float((np.abs(got - want) - tol).max())} past the tolerance"
+
+
+@pytest.mark.parametrize("m,n,k", [(100, 28672, 256), (100, 28672, 1024), (256, 14336, 512)])
+def test_short_k_keeps_the_staging_body(stream, m, n, k):
+    """With short K the staging-wave body of the 128-row tiles is the faster one
+    (65 x 256 x 28 672 7.5 us against 10.2): the linear runs it, so its outputs
+    are bit for bit those with weights off the 16-byte grid."""
+    x, w = wl.normal_f16(wl.seed_for(65, m + k), m * k), wl.q4_0_weights(wl.seed_for(65, n + k), n, k)
+    got, want = _both(stream, lambda xp, wp, yp: ops.quantized_linear_q4_0_f32(xp, wp[0], yp, m, n, k, stream), x, [w],
+                      m, n, False)
+    assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("m,n,k", [(65, 28672, 768), (300, 28672, 512)])
+def test_gate_up_short_k_keeps_the_staging_body(stream, m, n, k):
+    x = wl.normal_f16(wl.seed_for(66, m + k), m * k)
+    w = [wl.q4_0_weights(wl.seed_for(66, n + i), n, k) for i in (0, 1)]
+    got, want = _both(stream, lambda xp, wp, yp: ops.q4_0_gate_up_silu_f32(xp, wp[0], wp[1], yp, m, n, k, stream), x, w,
+                      m, n, False)
+    assert np.array_equal(got, want)
