@@ -411,7 +411,10 @@ bool prefill_ring_supports(const Problem& p) {
 
 // Where K is long and the tiles are few, K parts of 128-row tiles fill the chip:
 // the least of rounds of one workgroup per CU x (5 us + super-pairs of a part x
-// their time) + reduction, against a bm x bn tiling's own rounds.  Fits to
+// their time) + reduction, against 95 % of a bm x bn tiling's own rounds less 0.4
+// us per part (with 92 % and nothing per part, 65 x 4096 x 4096 took 20.0 us
+// instead of 17.0 and 64 x 3072 x 2048 15.3 instead of 13.7; of 303 shapes that took
+// parts then none is slower than its own tiles now).  Fits to
 // MI355X timings in us per super-pair: 3.6 (128 x 256), 2.2 (128 x 128), the
 // staging-wave tiles 1.25 (64 x 128), 0.85 (64 x 64); the reduction 3 us and the
 // planes written and read once at 4 TB/s, planes up to 48 MiB (inside a
@@ -435,12 +438,12 @@ hipError_t launch_prefill_ring_parts(const Problem& p, int bm, int bn) {
         return us;
     };
     const double own = cost(bm, bn, bm == 128 ? (bn == 256 ? 3.6 : 2.2) : (bn == 128 ? 1.25 : 0.85), 1);
-    double best = 0.92 * own;
+    double best = own;
     int tile = 0;
     uint32_t parts = 1;
     for (int tn = 256; tn >= 128; tn /= 2)
-        for (uint32_t k = 1; k <= 8 && k * 2 <= nsuper + 1; ++k) {
-            if (k > 1 && 4.0 * p.M * p.N * k > 48.0 * 1048576.0) break;
+        for (uint32_t k = 2; k <= 8 && k * 2 <= nsuper + 1; ++k) {
+            if (4.0 * p.M * p.N * k > 48.0 * 1048576.0) break;
             const double us = cost(128, tn, tn == 256 ? 3.6 : 2.2, k);
             if (us < best) {
                 best = us;
@@ -448,7 +451,7 @@ hipError_t launch_prefill_ring_parts(const Problem& p, int bm, int bn) {
                 parts = k;
             }
         }
-    if (tile == 0) return hipErrorNotSupported;
+    if (tile == 0 || best + 0.4 * parts >= 0.95 * own) return hipErrorNotSupported;
     return tile == 256 ? launch_ring<4, 4, false>(p, parts) : launch_ring<4, 2, false>(p, parts);
 }
 

@@ -150,3 +150,14 @@ def test_gate_up_short_k_keeps_the_staging_body(stream, m, n, k):
     got, want = _both(stream, lambda xp, wp, yp: ops.q4_0_gate_up_silu_f32(xp, wp[0], wp[1], yp, m, n, k, stream), x, w,
                       m, n, False)
     assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("m,n,k", [(65, 4096, 4096), (64, 2048, 3072), (256, 1024, 4096), (80, 4096, 5120)])
+def test_k_parts_only_where_they_pay(stream, m, n, k):
+    """Shapes whose 64-row tiles in one round are faster than 128-row ones over K
+    parts (65 x 4096 x 4096: 17.0 us against 20.0): no parts, so the outputs are
+    bit for bit those with weights off the 16-byte grid."""
+    x, w = wl.normal_f16(wl.seed_for(67, m + k), m * k), wl.q4_0_weights(wl.seed_for(67, n + k), n, k)
+    got, want = _both(stream, lambda xp, wp, yp: ops.quantized_linear_q4_0_f32(xp, wp[0], yp, m, n, k, stream), x, [w],
+                      m, n, False)
+    assert np.array_equal(got, want)
