@@ -67,6 +67,7 @@
 #include "q8_0_prefill_ring.hpp"
 #include "tile_ops.hpp"
 
+#include <algorithm>
 #include <cmath>
 #include <type_traits>
 
@@ -783,7 +784,10 @@ hipError_t launch_tile(const uint16_t* x, const uint8_t* w, OutT* y, uint32_t M,
 // 90 (128-row tiles), 101 / 109 (96-row), 99 / 113 (64-row), 100 x 4096 x 4096
 // 18 / 17 (64-row, four parts); Q6_K 256 x 14 336 x 4096 88 / 102, 63 / 61
 // (128-row, two, four parts); Q8_0 300 x 4096 x 14 336 80 / 93, 69 / 74, 79 / 85
-// (128-, 96-, 64-row), 256 x 14 336 x 4096 52 / 53 (64-row, two parts).
+// (128-, 96-, 64-row), 256 x 14 336 x 4096 52 / 53 (64-row, two parts).  Q8_0's
+// 64-row tiles wait for the weights where K is long, over all of it above all: 128 x
+// 8192 x 11 008 66 us, 128-row tiles over two parts 56; 512 x 11 008 x 11 008 256 and
+// 203.
 struct Plan {
     int tm;
     uint32_t parts;
@@ -801,12 +805,15 @@ Plan choose(uint32_t M, uint32_t N, uint32_t K, bool scratch = true) {
     Plan best{4, 1, 0.0};
     static constexpr double kBlockUs[3][3] = {{2.5, 1.95, 1.45}, {3.2, 2.7, 2.2}, {2.6, 2.0, 1.45}};
     for (int tm = F == Fmt::Q4K && !scratch ? 3 : 4; tm >= 2; --tm) {
-        const double block = kBlockUs[static_cast<int>(F)][4 - tm];
+        const double per_block = kBlockUs[static_cast<int>(F)][4 - tm];
         const double tiles = static_cast<double>((M + 32u * tm - 1) / (32u * tm)) * ((N + 127u) / 128u);
         for (uint32_t parts = 1; parts <= (scratch ? 8u : 1u) && parts * 2 <= nb + 1; ++parts) {
             const double plane_bytes = 4.0 * M * N * parts;
             if (parts > 1 && plane_bytes > static_cast<double>(kMaxPlaneBytes)) break;
             const double rounds = std::ceil(tiles * parts / cus);
+            double block = per_block;
+            if (F == Fmt::Q8 && tm == 2 && nb >= 32)
+                block = parts == 1 ? 1.9 : block + 0.2 * std::min(1.0, std::max(0.0, 2.0 * tiles * parts / cus - 1.0));
             double cost = rounds * (5.0 + block * ((nb + parts - 1) / parts));
             if (parts > 1) cost += 3.0 + 2.0 * plane_bytes / 4e6;
             if (best.us == 0.0 || cost < best.us) best = {tm, parts, cost};
@@ -825,6 +832,11 @@ Plan choose(uint32_t M, uint32_t N, uint32_t K, bool scratch = true) {
 // and 455 us (Q6_K) to 100 and 168.  (With a time per item that left s out, K
 // below 4096 went up to 60 % slower: 32 x 1024 x 7168 Q6_K 12.9 us against 8.0, 32
 // x 2048 x 20 000 Q4_K 15.3 against 13.1.)
+//
+// Q8_0's alternative, the tiles of q4_0_prefill.hip, is up to 12 % faster up to 64
+// tokens with long K and one part, where both wait for the weights (64 x 11 008 x
+// 28 672 103 us, here 115), and with K below 1024 and more than one round (512 x
+// 256 x 11 008 15.2, here 17.0), but has four times the error: these serve all.
 bool worth(Fmt f, uint32_t M, uint32_t N, uint32_t K) {
     if (M > 64 || f == Fmt::Q8) return true;
     if (M <= 16) return false;

@@ -152,3 +152,21 @@ def test_every_tile(stream, oracle, m, n, k, special):
             for cls in (np.isnan, np.isposinf, np.isneginf):
                 assert np.array_equal(cls(y), cls(y64)), f"{rows} rows, {parts} parts: {cls.__name__} positions differ"
             assert float(np.abs(y[ok] - y64[ok]).max(initial=0.0)) <= bound, f"{rows} rows, {parts} parts"
+
+
+def test_long_k_takes_128_row_tiles_over_two_parts(stream):
+    """128 x 8192 x 11 008: two rows of 64-row tiles over all of K wait for the
+    weights (66 us), one row of 128-row tiles over two parts does not (56)."""
+    m, n, k = 128, 11008, 8192
+    xb = DeviceBuffer.from_array(normal_x(wl.seed_for(80, k), m, k))
+    wb = DeviceBuffer.from_array(np.tile(weights(wl.seed_for(80, n), n // 43, k).reshape(-1), 43))
+    ys = []
+    for call in (
+        lambda y: ops.quantized_linear_q8_0_f32(xb.ptr, wb.ptr, y.ptr, m, n, k, stream),
+        lambda y: ops.prompt_linear_tiles("q8_0", xb.ptr, wb.ptr, y.ptr, m, n, k, stream, 128, 2),
+    ):
+        y = DeviceBuffer(m * n * 4)
+        call(y)
+        stream.synchronize()
+        ys.append(y.download(np.uint32))
+    assert np.array_equal(ys[0], ys[1])
