@@ -37,13 +37,15 @@
 // past 65504 recompute the token's outputs one by one, and the 128-row tile
 // spilled and waited for every load in flight once per super-block (512 x 4096
 // x 14 336 83.9 us against 81.7, 256 x 14 336 x 4096 47.6 against 46.9).
+//
 // The groups' partial tiles meet in LDS (fixed order); K parts, used where the
 // tiles are too few for the chip, meet in scratch planes that
 // parts_reduce_kernel adds in part order.  Planes and sums live in the stream's
 // prompt scratch (q4_0.hpp).  Without it there is one part, and Q4_K's sums are
 // added up from the operands in registers, 16 elements per lane, three MFMAs per
 // super-block (OWN): 32 dot products per tile and quarter in every wave, which 96-
-// and 64-row tiles have registers for.  512 x 4096 x 14 336 122 us against 85.
+// and 64-row tiles have registers for.  512 x 4096 x 14 336 121 us against 80, 256 x 14 336 x 4096 92
+// against 46.
 //
 // A result that is not finite is added up again with GGML's values, over the
 // activations and blocks that make it so (over all elements, as in the few-token
@@ -51,15 +53,15 @@
 // infinite activation in each token as long, now 0.16 and 2.2 ms).
 //
 // Measured on MI355X (weights of three calls rotated): 512 x 4096 x 14 336 Q4_K
-// 82 us (733 TFLOP/s), where the four-token passes of the LDS-ring GEMV, which
+// 80 us (750 TFLOP/s), where the four-token passes of the LDS-ring GEMV, which
 // read every weight M / 4 times, took 1723; 256 x 14 336 x 4096 Q6_K 62 us
-// against 1203.  Bound by the interval's instruction stream: MFMAs fill 37 % of
-// the cycles, vector instructions and the LDS (A operands read once per wave)
-// a third each, imperfectly overlapped at two waves per SIMD.  128 x 256 tiles
-// of four waves with 512 registers (half the A reads per MFMA) measured level
-// (84 us); 96- and 64-row tiles take 8 and 20 % longer per row and are for
-// token counts and grids that 128-row tiles fill badly (300 x 4096 x 14 336: 65
-// us on 96-row tiles).  The Q8_0 linear has a kernel of its own
+// against 1203.  Bound by the interval's instruction stream: counters have MFMAs
+// in 37 (Q4_K) and 44 % (Q6_K) of all SIMD cycles and 7.0 and 5.4 vector
+// instructions per MFMA, imperfectly overlapped at two waves per SIMD.  96- and
+// 64-row tiles take 8 and 20 % longer per row and are for token counts and grids
+// that 128-row tiles fill badly (300 x 4096 x 14 336: 65 us on 96-row tiles).
+// Activations off the 16-byte grid, and such Q4_K weights, keep the kernels of
+// few tokens in passes.  The Q8_0 linear has a kernel of its own
 // (q8_0_prefill_ring.hpp) and shares the launch.
 #include "export.hpp"
 #include "kquant_blocks.hpp"

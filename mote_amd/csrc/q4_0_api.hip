@@ -225,12 +225,17 @@ const Variant* cheapest_tiles(const Problem& p, const TileCost (&cand)[N]) {
     return best;
 }
 
-// The Q8_0 linear's prefill tiles and their wave times at K = 4096.
+// The Q8_0 linear's prefill tiles and their wave times at K = 4096, those of
+// q4_0_prefill.hip's body: it runs where K is no multiple of 256; else the name
+// picked only leads to the exact-integer tiles, which choose for themselves.
 const TileCost kQ8Tiles[] = {{"q8_mfma_x32s_m128_n256_w1", 2, 96.0f},
                              {"q8_mfma_x32s_m128_n128_w1", 2, 56.0f},
                              {"q8_mfma_x32s_m64_n128_w1", 4, 36.0f}};
 
-// The Q4_0 linear's prefill tiles and their wave times at K = 4096.
+// The Q4_0 linear's prefill tiles and their wave times at K = 4096, the staging
+// waves'.  (The ring body of the 128-row ones is some 5 % faster there, which
+// moves none of the crossovers by more than that; K parts are a second choice,
+// made at the launch, where the scratch is known.)
 const TileCost kTiles[] = {{"mfma_x32s_m128_n256_w1", 2, 60.0f},
                            {"mfma_x32s_m128_n128_w1", 2, 40.0f},
                            {"mfma_x32s_m64_n128_w1", 4, 25.0f},
@@ -861,7 +866,8 @@ const Variant* rules(const Problem& p, Op op, bool split_ok) {
 // and prefill linears and the fused gate/up at their benchmark shapes): every
 // candidate the autotuner would time for the shape, with its kernel time in
 // microseconds on MI355X (graph replays, weights rotated past the MALL), as
-// written by `bench.py --plan-table`.  A listed shape with operands on the
+// written by `bench.py --plan-table` (the prompt entries, of 65 tokens and more, on
+// the staging-wave bodies of the tiles).  A listed shape with operands on the
 // 16-byte grid (the class the table was measured in) runs its fastest entry
 // that supports the operands; every other shape runs the rules above.
 struct PlanEntry {

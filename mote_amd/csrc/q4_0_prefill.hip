@@ -43,10 +43,12 @@
 // tolerance for Q4_0's 4-bit values but measured too coarse for 8-bit ones.
 //
 // The 128-row multi-pair Q4_0 tiles (`_k2`) run the body of
-// q4_0_prefill_ring.hip where K is a multiple of 256 and the operands are
-// 16-byte aligned (5 - 16 % faster, measured there), the multi-pair Q8_0 tiles
-// those of q8_0_prefill_ring.hpp (7 - 48 % faster); this body serves them
-// otherwise.
+// q4_0_prefill_ring.hip where K is a multiple of 256, long enough
+// (prefill_ring_pays) and the operands are 16-byte aligned (5 - 16 % faster,
+// measured there), every multi-pair Q4_0 linear 128-row ring tiles over K parts
+// where those are faster, and all multi-pair Q8_0 names the one call of
+// q8_0_prefill_ring.hpp (7 - 48 % faster), which chooses its own tiles; this
+// body serves them otherwise.
 #include "common.hpp"
 #include "kquant_blocks.hpp"
 #include "q4_0.hpp"

@@ -7,7 +7,9 @@
 // 64 weight rows (tile j: rows 32 j ..; gate/up: 32 gate and the same 32 up
 // rows) over one half of K: TM x 2 tiles of v_mfma_f32_32x32x16_f16.  So every
 // weight is decoded by one wave, once per 32 TM tokens, two waves share each
-// SIMD, and the two halves' accumulators meet in LDS at the end.
+// SIMD (WN = 4; the 128-column tiles, WN = 2, have one wave per SIMD and 120 KB of
+// LDS, so they pay 2.2 us per super-pair where the 256-column ones pay 3.6), and
+// the two halves' accumulators meet in LDS at the end.
 //
 // An interval is 64 k (a block pair) of each half, with one barrier:
 //  * activations: 16-byte chunks in their natural order, three slots (two
@@ -24,10 +26,10 @@
 // The barrier stands before an interval's last slice, whose MFMAs cover the
 // next interval's first reads; its weights are read one slice earlier.
 //
-// Bound by power: at 512 x 4096 x 14 336 the loop takes 90 thousand cycles (65.5
-// thousand of MFMA) at 1.67 GHz; the same tile with pointer-addressed loads and
-// the weights read behind the barrier took 102 thousand at 1.84, 65.7 us against
-// 62.7: fewer cycles lower the clock.  Measured on MI355X (weights of three
+// Bound by the instruction stream, and the clock falls as it gets denser: counters
+// have MFMAs in 42 % of all SIMD cycles at 512 x 4096 x 14 336 (224 workgroups on 256
+// CUs) and 46 % in the 1024-token gate/up, and six vector instructions per MFMA.
+// Measured on MI355X (weights of three
 // calls rotated), the staging-wave body of q4_0_prefill.hip against this one:
 // 512 x 4096 x 14 336 66.2 -> 62.7 us, 2048 x 4096 x 4096 73.3 -> 69.7 (128 x
 // 256 tiles), 256 x 4096 x 14 336 40.9 -> 38.5, 1024 x 14 336 x 4096 143.7 ->

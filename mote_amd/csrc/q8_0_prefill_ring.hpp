@@ -33,7 +33,8 @@
 // 100 -> 52, 256 x 4096 x 4096 32 -> 22, 48 x 8192 x 28 672 80 -> 75; relative
 // error against 64 bits 5.7e-7 -> 1.5e-7 at K = 4096.  Bound by the vector
 // pipe: 16 fmas per tile and block beside two MFMAs, and 10 instructions per 8
-// weights.
+// weights; counters have 14 to 15 vector instructions per MFMA and MFMAs in 25 to
+// 27 % of all SIMD cycles.
 #pragma once
 
 #include "kquant_blocks.hpp"

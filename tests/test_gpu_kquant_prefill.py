@@ -25,10 +25,11 @@ from test_gpu_kquant import FORMATS, _blocks, _check, _fmt, _judge, _run
 pytestmark = pytest.mark.gpu
 
 SHAPES = [
-    # (M, N, K): one super-block (the second wave group idle), odd counts of
-    # blocks (uneven groups), one row past and short of a tile on both sides,
-    # a single column, several tiles of both heights, K parts (few tiles, long
-    # K) with a short last part
+    # (M, N, K), each on the tile that the linear picks (64 rows but for the
+    # last; test_every_tile runs the others): one super-block (the second wave
+    # group idle), odd counts of blocks (uneven groups), one row past and short of
+    # a tile on both sides, a single column, several tiles, K parts (few tiles,
+    # long K) with a short last part
     (65, 1, 256),
     (128, 128, 512),
     (129, 127, 768),
@@ -147,6 +148,14 @@ def test_q6_k_many_tokens_at_two_byte_offset(stream, oracle):
     x = wl.normal_f16(wl.seed_for(44, 1), m * k)
     y64, max_w, max_x = _judge(oracle, "q6_k", x, w, m, n, k)
     _check(_run(stream, "q6_k", x, w, m, n, k, w_offset=2), y64, k, max_w, max_x, what="q6_k at 2 mod 4")
+
+
+def test_q4_k_many_tokens_unaligned_weights(stream, oracle):
+    """Q4_K weights off the 16-byte grid keep the few-token kernels' route."""
+    m, n, k = 66, 20, 512
+    w, x = wl.q4_k_weights(851, n, k), wl.normal_f16(wl.seed_for(45, 2), m * k)
+    y64, max_w, max_x = _judge(oracle, "q4_k", x, w, m, n, k)
+    _check(_run(stream, "q4_k", x, w, m, n, k, w_offset=4), y64, k, max_w, max_x, what="q4_k w unaligned")
 
 
 @pytest.mark.parametrize("name", list(FORMATS))

@@ -4,7 +4,7 @@ Both decode every weight to the same binary16 value and sum exact products in
 f32, in another order: K additions that round a partial sum of about sqrt(K)
 max|w| max|x| by 2^-24 each, independently, in either body; twice their sum is
 allowed.  (Against the oracle both are judged by test_every_mfma_variant and
-the wide-scale tests.)"""
+the wide-scale tests; a forced variant runs its own tiles, here and there.)"""
 
 from __future__ import annotations
 
