@@ -170,9 +170,9 @@ __global__ __launch_bounds__(64 * kTileWaves * kTileGroups) void kq_prefill_kern
     const uint16_t* __restrict__ x, const uint8_t* __restrict__ w, const uint16_t* __restrict__ sums,
     OutT* __restrict__ y, float* __restrict__ partial, uint32_t M, uint32_t N, uint32_t K, uint32_t m_tiles,
     uint32_t n_tiles, uint32_t part_blocks, uint32_t total, uint32_t per_xcd) {
-    constexpr int KG = kTileGroups, TN = 1;  // TN: 32-row weight tiles per wave (two fill 512 registers)
+    constexpr int KG = kTileGroups;
     constexpr int BM = 32 * TM;
-    constexpr uint32_t BN = 32 * TN * kTileWaves;
+    constexpr uint32_t BN = 32 * kTileWaves;
     constexpr int kUnit = BM * 128;            // LDS bytes of one group's activations of an interval
     constexpr int kSlots = 4;                  // interval t, a quarter p = t % 4 of a super-block: slot p
     constexpr int NA = BM / (8 * kTileWaves);  // activation loads per wave and interval
@@ -194,7 +194,7 @@ __global__ __launch_bounds__(64 * kTileWaves * kTileGroups) void kq_prefill_kern
     constexpr bool SUMS = F == Fmt::Q4K && !OWN;
     constexpr int NS = SUMS ? (BM * 64 + kTileWaves * 1024 - 1) / (kTileWaves * 1024) : 0;  // loads per wave
     constexpr int kSumUnit = NS * kTileWaves * 1024;
-    constexpr int kReduce = kTileWaves * KG * ((TM + 1) / 2) * TN * 4096;
+    constexpr int kReduce = kTileWaves * KG * ((TM + 1) / 2) * 4096;
     static_assert(kRing >= kReduce && kRing + 2 * KG * kSumUnit <= 160 * 1024, "LDS");
     __shared__ __attribute__((aligned(1024))) uint8_t lds[kRing + 2 * KG * kSumUnit];
 
@@ -235,13 +235,10 @@ __global__ __launch_bounds__(64 * kTileWaves * kTileGroups) void kq_prefill_kern
         for (int i = 0; i < NA; ++i)
             load_lds16(xsrc, aoff[i], o, unit + slot * (KG * kUnit) + (wn * NA + i) * 1024);
     };
-    // Weights: row r of each of this wave's TN column tiles (clamped), from
-    // super-block b0 on.
-    const uint8_t* wrow[TN];
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-        wrow[j] = w + (static_cast<size_t>(min(n0 + (wn * TN + j) * 32 + lr, N - 1)) * nb + b0) * BB;
-    Raw<F> raw[TN];
+    // Weights: row r of this wave's 32 (clamped), from super-block b0 on.
+    const uint8_t* const wrow =
+        w + (static_cast<size_t>(min(n0 + wn * 32 + lr, N - 1)) * nb + b0) * BB;
+    Raw<F> raw;
     // After the second quarter of a half block, p = 1 or 3: that half's quants
     // of super-block s (clamped).  A quarter at a time, as it is freed, fetched
     // the lines of a row's half block twice.
@@ -249,141 +246,124 @@ __global__ __launch_bounds__(64 * kTileWaves * kTileGroups) void kq_prefill_kern
         constexpr int P = decltype(pc)::value, g = P / 2;
         if constexpr (P % 2 == 1) {
             const size_t at = static_cast<size_t>(min(s, ns - 1)) * BB;
+            const uint8_t* blk = wrow + at;
+            if constexpr (F == Fmt::Q4K) {
 #pragma unroll
-            for (int j = 0; j < TN; ++j) {
-                const uint8_t* blk = wrow[j] + at;
-                if constexpr (F == Fmt::Q4K) {
-#pragma unroll
-                    for (int p = 2 * g; p < 2 * g + 2; ++p)
-                        raw[j].qs[p] = *reinterpret_cast<const u32x4*>(blk + 16 + 32 * p + 16 * lc);
-                } else {
-                    raw[j].la[g] = *reinterpret_cast<const u32x4_a2*>(blk + 64 * g + 16 * lc);
-                    raw[j].lb[g] = *reinterpret_cast<const u32x4_a2*>(blk + 64 * g + 32 + 16 * lc);
-                    raw[j].qh[g] = *reinterpret_cast<const u32x4_a2*>(blk + 128 + 32 * g + 16 * lc);
-                }
+                for (int p = 2 * g; p < 2 * g + 2; ++p)
+                    raw.qs[p] = *reinterpret_cast<const u32x4*>(blk + 16 + 32 * p + 16 * lc);
+            } else {
+                raw.la[g] = *reinterpret_cast<const u32x4_a2*>(blk + 64 * g + 16 * lc);
+                raw.lb[g] = *reinterpret_cast<const u32x4_a2*>(blk + 64 * g + 32 + 16 * lc);
+                raw.qh[g] = *reinterpret_cast<const u32x4_a2*>(blk + 128 + 32 * g + 16 * lc);
             }
         }
     };
     auto load_head = [&](uint32_t s) {
         const size_t at = static_cast<size_t>(min(s, ns - 1)) * BB;
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            const uint8_t* blk = wrow[j] + at;
-            if constexpr (F == Fmt::Q4K) {
-                raw[j].head = *reinterpret_cast<const u32x4*>(blk);
-            } else {
-                raw[j].sc = *reinterpret_cast<const u32x4_a2*>(blk + 192);
-                raw[j].d = *reinterpret_cast<const uint16_t*>(blk + 208);
-            }
+        const uint8_t* blk = wrow + at;
+        if constexpr (F == Fmt::Q4K) {
+            raw.head = *reinterpret_cast<const u32x4*>(blk);
+        } else {
+            raw.sc = *reinterpret_cast<const u32x4_a2*>(blk + 192);
+            raw.d = *reinterpret_cast<const uint16_t*>(blk + 208);
         }
     };
-    Scales<F> sl[TN];
-    float d_fold[TN] = {};  // the scale of the block sums not yet folded
+    Scales<F> sl;
+    float d_fold = 0.0f;  // the scale of the block sums not yet folded
     auto unpack_head = [&]() {
+        if constexpr (F == Fmt::Q4K) {
+            const u32x4 head = raw.head;
+            sl.sc[0] = head.y & 0x3F3F3F3Fu;
+            sl.sc[1] = (head.w & 0x0F0F0F0Fu) | ((head.y >> 2) & 0x30303030u);
+            const uint32_t lo = head.z & 0x3F3F3F3Fu;
+            const uint32_t hi = ((head.w >> 4) & 0x0F0F0F0Fu) | ((head.z >> 2) & 0x30303030u);
+            sl.m[0] = bytes_bf16<0, 1>(lo);
+            sl.m[1] = bytes_bf16<2, 3>(lo);
+            sl.m[2] = bytes_bf16<0, 1>(hi);
+            sl.m[3] = bytes_bf16<2, 3>(hi);
+            sl.d = as_f32(half_lo_to_float(head.x));
+            sl.dmin = as_f32(half_hi_to_float(head.x));
+        } else {
+            const uint32_t s[4] = {raw.sc.x, raw.sc.y, raw.sc.z, raw.sc.w};
 #pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            if constexpr (F == Fmt::Q4K) {
-                const u32x4 head = raw[j].head;
-                sl[j].sc[0] = head.y & 0x3F3F3F3Fu;
-                sl[j].sc[1] = (head.w & 0x0F0F0F0Fu) | ((head.y >> 2) & 0x30303030u);
-                const uint32_t lo = head.z & 0x3F3F3F3Fu;
-                const uint32_t hi = ((head.w >> 4) & 0x0F0F0F0Fu) | ((head.z >> 2) & 0x30303030u);
-                sl[j].m[0] = bytes_bf16<0, 1>(lo);
-                sl[j].m[1] = bytes_bf16<2, 3>(lo);
-                sl[j].m[2] = bytes_bf16<0, 1>(hi);
-                sl[j].m[3] = bytes_bf16<2, 3>(hi);
-                sl[j].d = as_f32(half_lo_to_float(head.x));
-                sl[j].dmin = as_f32(half_hi_to_float(head.x));
-            } else {
-                const uint32_t s[4] = {raw[j].sc.x, raw[j].sc.y, raw[j].sc.z, raw[j].sc.w};
-#pragma unroll
-                for (int p = 0; p < 4; ++p) sl[j].sc[p] = s[p] >> (8 * lc);
-                sl[j].d = as_f32(8.0f * half_bits_to_float(raw[j].d));
-            }
+            for (int p = 0; p < 4; ++p) sl.sc[p] = s[p] >> (8 * lc);
+            sl.d = as_f32(8.0f * half_bits_to_float(raw.d));
         }
     };
     // The binary16 factors of a quarter's two sub-blocks (h = 0, 1).
-    f16x2 mul[TN][2][NB], add[TN][2][NB];
+    f16x2 mul[2][NB], add[2][NB];
     auto quarter_scales = [&](auto pc) {
         constexpr int P = decltype(pc)::value;
+        if constexpr (F == Fmt::Q4K) {
+            const uint32_t word = sl.sc[P / 2];
+            const f16x2 sc = as_h2(perm(0x64646464u, word, P % 2 ? 0x04030402u : 0x04010400u)) +
+                             both(static_cast<_Float16>(-1024.0f));
+            mul[0][0] = both(sc, false);
+            mul[1][0] = both(sc, true);
+            add[0][0] = mul[0][0] * both(static_cast<_Float16>(-1024.0f));
+            add[1][0] = mul[1][0] * both(static_cast<_Float16>(-64.0f));
+        } else {
 #pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            if constexpr (F == Fmt::Q4K) {
-                const uint32_t word = sl[j].sc[P / 2];
-                const f16x2 sc = as_h2(perm(0x64646464u, word, P % 2 ? 0x04030402u : 0x04010400u)) +
-                                 both(static_cast<_Float16>(-1024.0f));
-                mul[j][0][0] = both(sc, false);
-                mul[j][1][0] = both(sc, true);
-                add[j][0][0] = mul[j][0][0] * both(static_cast<_Float16>(-1024.0f));
-                add[j][1][0] = mul[j][1][0] * both(static_cast<_Float16>(-64.0f));
-            } else {
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const int sc = static_cast<int8_t>((sl[j].sc[P] >> (16 * h)) & 0xFFu);
-                    const _Float16 s = static_cast<_Float16>(static_cast<short>(sc >> 3));
-                    const _Float16 t =
-                        static_cast<_Float16>(static_cast<short>(sc & 7)) * static_cast<_Float16>(0.125f);
-                    mul[j][h][0] = both(s);
-                    mul[j][h][NB - 1] = both(t);
-                    add[j][h][0] = both(static_cast<_Float16>(s * static_cast<_Float16>(-1056.0f)));
-                    add[j][h][NB - 1] = both(static_cast<_Float16>(t * static_cast<_Float16>(-1056.0f)));
-                }
+            for (int h = 0; h < 2; ++h) {
+                const int sc = static_cast<int8_t>((sl.sc[P] >> (16 * h)) & 0xFFu);
+                const _Float16 s = static_cast<_Float16>(static_cast<short>(sc >> 3));
+                const _Float16 t =
+                    static_cast<_Float16>(static_cast<short>(sc & 7)) * static_cast<_Float16>(0.125f);
+                mul[h][0] = both(s);
+                mul[h][NB - 1] = both(t);
+                add[h][0] = both(static_cast<_Float16>(s * static_cast<_Float16>(-1056.0f)));
+                add[h][NB - 1] = both(static_cast<_Float16>(t * static_cast<_Float16>(-1056.0f)));
             }
         }
     };
     // The operands of slice (h, u) of quarter p.
-    f16x8 b[2][TN][NB];
-    auto decode = [&](auto pc, auto uc, f16x8 (&dst)[TN][NB]) {
+    f16x8 b[2][NB];
+    auto decode = [&](auto pc, auto uc, f16x8 (&dst)[NB]) {
         constexpr int P = decltype(pc)::value, U = decltype(uc)::value, h = U / 2, u = U % 2;
+        uint32_t q[2];
+        if constexpr (F == Fmt::Q4K) {
+            constexpr uint32_t mask = h ? 0xF0F0F0F0u : 0x0F0F0F0Fu, e = h ? 0x54545454u : 0x64646464u;
+            q[0] = (u ? raw.qs[P].z : raw.qs[P].x) & mask;
+            q[1] = (u ? raw.qs[P].w : raw.qs[P].y) & mask;
+            const f16x2 m = mul[h][0], a = add[h][0];
+            dst[0] = join(__builtin_elementwise_fma(as_h2(perm(e, q[0], 0x04010400u)), m, a),
+                          __builtin_elementwise_fma(as_h2(perm(e, q[0], 0x04030402u)), m, a),
+                          __builtin_elementwise_fma(as_h2(perm(e, q[1], 0x04010400u)), m, a),
+                          __builtin_elementwise_fma(as_h2(perm(e, q[1], 0x04030402u)), m, a));
+        } else {
+            // quarter c4 of half g: nibble c4 / 2 of run c4 % 2
+            constexpr int g = P / 2, c4 = 2 * (P % 2) + h;
+            const u32x4 l = c4 % 2 ? raw.lb[g] : raw.la[g];
+            const uint32_t lw[2] = {u ? l.z : l.x, u ? l.w : l.y};
+            const uint32_t hw[2] = {u ? raw.qh[g].z : raw.qh[g].x, u ? raw.qh[g].w : raw.qh[g].y};
+            f16x2 v[4];
 #pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            uint32_t q[2];
-            if constexpr (F == Fmt::Q4K) {
-                constexpr uint32_t mask = h ? 0xF0F0F0F0u : 0x0F0F0F0Fu, e = h ? 0x54545454u : 0x64646464u;
-                q[0] = (u ? raw[j].qs[P].z : raw[j].qs[P].x) & mask;
-                q[1] = (u ? raw[j].qs[P].w : raw[j].qs[P].y) & mask;
-                const f16x2 m = mul[j][h][0], a = add[j][h][0];
-                dst[j][0] = join(__builtin_elementwise_fma(as_h2(perm(e, q[0], 0x04010400u)), m, a),
-                                 __builtin_elementwise_fma(as_h2(perm(e, q[0], 0x04030402u)), m, a),
-                                 __builtin_elementwise_fma(as_h2(perm(e, q[1], 0x04010400u)), m, a),
-                                 __builtin_elementwise_fma(as_h2(perm(e, q[1], 0x04030402u)), m, a));
-            } else {
-                // quarter c4 of half g: nibble c4 / 2 of run c4 % 2
-                constexpr int g = P / 2, c4 = 2 * (P % 2) + h;
-                const u32x4 l = c4 % 2 ? raw[j].lb[g] : raw[j].la[g];
-                const uint32_t lw[2] = {u ? l.z : l.x, u ? l.w : l.y};
-                const uint32_t hw[2] = {u ? raw[j].qh[g].z : raw[j].qh[g].x, u ? raw[j].qh[g].w : raw[j].qh[g].y};
-                f16x2 v[4];
-#pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    const uint32_t low = (c4 < 2 ? lw[i] : lw[i] >> 4) & 0x0F0F0F0Fu;
-                    const uint32_t top = c4 == 0 ? hw[i] << 4 : c4 == 1 ? hw[i] << 2 : c4 == 2 ? hw[i] : hw[i] >> 2;
-                    q[i] = (top & 0x30303030u) | low;
-                    v[2 * i] = as_h2(perm(0x64646464u, q[i], 0x04010400u));
-                    v[2 * i + 1] = as_h2(perm(0x64646464u, q[i], 0x04030402u));
-                }
-#pragma unroll
-                for (int k = 0; k < NB; ++k)
-                    dst[j][k] = join(__builtin_elementwise_fma(v[0], mul[j][h][k], add[j][h][k]),
-                                     __builtin_elementwise_fma(v[1], mul[j][h][k], add[j][h][k]),
-                                     __builtin_elementwise_fma(v[2], mul[j][h][k], add[j][h][k]),
-                                     __builtin_elementwise_fma(v[3], mul[j][h][k], add[j][h][k]));
+            for (int i = 0; i < 2; ++i) {
+                const uint32_t low = (c4 < 2 ? lw[i] : lw[i] >> 4) & 0x0F0F0F0Fu;
+                const uint32_t top = c4 == 0 ? hw[i] << 4 : c4 == 1 ? hw[i] << 2 : c4 == 2 ? hw[i] : hw[i] >> 2;
+                q[i] = (top & 0x30303030u) | low;
+                v[2 * i] = as_h2(perm(0x64646464u, q[i], 0x04010400u));
+                v[2 * i + 1] = as_h2(perm(0x64646464u, q[i], 0x04030402u));
             }
+#pragma unroll
+            for (int k = 0; k < NB; ++k)
+                dst[k] = join(__builtin_elementwise_fma(v[0], mul[h][k], add[h][k]),
+                              __builtin_elementwise_fma(v[1], mul[h][k], add[h][k]),
+                              __builtin_elementwise_fma(v[2], mul[h][k], add[h][k]),
+                              __builtin_elementwise_fma(v[3], mul[h][k], add[h][k]));
         }
     };
 
-    f32x16 acc[TM][TN], blk[NC][TM][TN], runs[RUNS ? TM : 1][TN];
+    f32x16 acc[TM], blk[NC][TM], runs[RUNS ? TM : 1];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j)
+        for (int r = 0; r < 16; ++r) {
+            acc[i][r] = 0.0f;
+            if constexpr (RUNS) runs[i][r] = 0.0f;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                acc[i][j][r] = 0.0f;
-                if constexpr (RUNS) runs[i][j][r] = 0.0f;
-#pragma unroll
-                for (int c = 0; c < NC; ++c) blk[c][i][j][r] = 0.0f;
-            }
+            for (int c = 0; c < NC; ++c) blk[c][i][r] = 0.0f;
+        }
     const f32x16 zero = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
     f16x8 a[2][TM];
     const uint32_t a_row = lr * 128, a_x = (lr >> 1) & 7;
@@ -398,28 +378,25 @@ __global__ __launch_bounds__(64 * kTileWaves * kTileGroups) void kq_prefill_kern
         for (int k = 0; k < NB; ++k)
 #pragma unroll
             for (int i = 0; i < TM; ++i)
-#pragma unroll
-                for (int j = 0; j < TN; ++j) blk[k % NC][i][j] = mfma32(a[C][i], b[C][j][k], blk[k % NC][i][j]);
+                blk[k % NC][i] = mfma32(a[C][i], b[C][k], blk[k % NC][i]);
     };
     // The first slice of a super-block: the sums of the one before join the
     // result, tile by tile ahead of the tile's first product.
-    auto fold = [&](int i, int j) {
+    auto fold = [&](int i) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            const float sum = NC == 2 ? blk[0][i][j][r] + blk[NC - 1][i][j][r] : blk[0][i][j][r];
-            acc[i][j][r] = __builtin_fmaf(d_fold[j], sum, acc[i][j][r]);
+            const float sum = NC == 2 ? blk[0][i][r] + blk[NC - 1][i][r] : blk[0][i][r];
+            acc[i][r] = __builtin_fmaf(d_fold, sum, acc[i][r]);
         }
     };
     auto multiply_first = [&]() {
 #pragma unroll
         for (int k = 0; k < NB; ++k)
 #pragma unroll
-            for (int i = 0; i < TM; ++i)
-#pragma unroll
-                for (int j = 0; j < TN; ++j) {
-                    if (k == 0) fold(i, j);
-                    blk[k % NC][i][j] = mfma32(a[0][i], b[0][j][k], k < NC ? zero : blk[k % NC][i][j]);
-                }
+            for (int i = 0; i < TM; ++i) {
+                if (k == 0) fold(i);
+                blk[k % NC][i] = mfma32(a[0][i], b[0][k], k < NC ? zero : blk[k % NC][i]);
+            }
     };
     // Q4_K's minimum term of the super-block, one tile per slice of its second
     // half.  A row's sums are four 16-byte chunks: the three bfloat16 pieces of
@@ -446,23 +423,19 @@ __global__ __launch_bounds__(64 * kTileWaves * kTileGroups) void kq_prefill_kern
         for (int k = 0; k < 2; ++k)
             sx[i & 1][k] = *reinterpret_cast<const bf16x8*>(row + (((2 * k + lc) ^ ((lr >> 2) & 3)) * 16));
     };
-    auto mins = [&](int j) {
+    auto mins = [&]() {
         if constexpr (F == Fmt::Q4K)
-            return __builtin_bit_cast(bf16x8, u32x4{sl[j].m[0], sl[j].m[1], sl[j].m[2], sl[j].m[3]});
+            return __builtin_bit_cast(bf16x8, u32x4{sl.m[0], sl.m[1], sl.m[2], sl.m[3]});
     };
     auto minimum = [&](auto pc, auto ic, uint32_t s, auto slice) {
         constexpr int I = 4 * (decltype(pc)::value - 2) + decltype(ic)::value;
         if constexpr (SUMS) {
             if constexpr (I + 1 >= 0 && I + 1 < TM) read_sums(s, I + 1);
             if constexpr (I >= 0 && I < TM) {
-                f32x16 mn[TN];
-#pragma unroll
-                for (int j = 0; j < TN; ++j) mn[j] = mfma32(sx[I & 1][1], mins(j), mfma32(sx[I & 1][0], mins(j), zero));
+                const f32x16 mn = mfma32(sx[I & 1][1], mins(), mfma32(sx[I & 1][0], mins(), zero));
                 slice();
 #pragma unroll
-                for (int j = 0; j < TN; ++j)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) acc[I][j][r] = __builtin_fmaf(-sl[j].dmin, mn[j][r], acc[I][j][r]);
+                for (int r = 0; r < 16; ++r) acc[I][r] = __builtin_fmaf(-sl.dmin, mn[r], acc[I][r]);
             } else {
                 slice();
             }
@@ -496,25 +469,23 @@ __global__ __launch_bounds__(64 * kTileWaves * kTileGroups) void kq_prefill_kern
     auto own_minimum = [&]() {
         if constexpr (OWN) {
 #pragma unroll
-            for (int i = 0; i < TM; ++i)
+            for (int i = 0; i < TM; ++i) {
+                f32x16 mn = zero;
 #pragma unroll
-                for (int j = 0; j < TN; ++j) {
-                    f32x16 mn = zero;
-#pragma unroll
-                    for (int k = 0; k < 3; ++k) {
-                        const u32x4 v = {own[i][k][0], own[i][k][1], own[i][k][2], own[i][k][3]};
-                        mn = mfma32(__builtin_bit_cast(bf16x8, v), mins(j), mn);
-                    }
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) acc[i][j][r] = __builtin_fmaf(-sl[j].dmin, mn[r], acc[i][j][r]);
+                for (int k = 0; k < 3; ++k) {
+                    const u32x4 v = {own[i][k][0], own[i][k][1], own[i][k][2], own[i][k][3]};
+                    mn = mfma32(__builtin_bit_cast(bf16x8, v), mins(), mn);
                 }
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[i][r] = __builtin_fmaf(-sl.dmin, mn[r], acc[i][r]);
+            }
         }
     };
     // Loads a wave issues behind interval t's activations of four intervals on:
     // quants, the next super-block's sums (p = 0) and header (p = 2).
     constexpr bool kQ4 = F == Fmt::Q4K;
-    constexpr int kHalf = (kQ4 ? 2 : 3) * TN;  // a half block's quants
-    constexpr int kBehind[4] = {NS, kHalf, kQ4 ? TN : 2 * TN, kHalf};
+    constexpr int kHalf = kQ4 ? 2 : 3;  // a half block's quants
+    constexpr int kBehind[4] = {NS, kHalf, kQ4 ? 1 : 2, kHalf};
     using I0 = std::integral_constant<int, 0>;
     using I1 = std::integral_constant<int, 1>;
     using I2 = std::integral_constant<int, 2>;
@@ -537,7 +508,7 @@ __global__ __launch_bounds__(64 * kTileWaves * kTileGroups) void kq_prefill_kern
         order_fence();
         load_quants(I3{}, 0);
         order_fence();
-        wait_counts<vm_wait(3 * NA + (kQ4 ? 5 : 8) * TN)>();  // interval 0's activations
+        wait_counts<vm_wait(3 * NA + (kQ4 ? 5 : 8))>();  // interval 0's activations
     }
     group_barrier();
     order_fence();
@@ -590,8 +561,7 @@ __global__ __launch_bounds__(64 * kTileWaves * kTileGroups) void kq_prefill_kern
                 add_slice(pc, I3{});
                 if constexpr (P == 3) {
                     own_minimum();
-#pragma unroll
-                    for (int j = 0; j < TN; ++j) d_fold[j] = sl[j].d;
+                    d_fold = sl.d;
                     unpack_head();
                 }
                 quarter_scales(PN{});
@@ -607,22 +577,18 @@ __global__ __launch_bounds__(64 * kTileWaves * kTileGroups) void kq_prefill_kern
             if constexpr (RUNS) {
                 if (s % kRun == kRun - 1) {
 #pragma unroll
-                    for (int i = 0; i < TM; ++i)
-#pragma unroll
-                        for (int j = 0; j < TN; ++j) {
-                            runs[i][j] += acc[i][j];
-                            acc[i][j] = zero;
-                        }
+                    for (int i = 0; i < TM; ++i) {
+                        runs[i] += acc[i];
+                        acc[i] = zero;
+                    }
                 }
             }
         }
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int j = 0; j < TN; ++j) {
-                fold(i, j);
-                if constexpr (RUNS) acc[i][j] += runs[i][j];
-            }
+        for (int i = 0; i < TM; ++i) {
+            fold(i);
+            if constexpr (RUNS) acc[i] += runs[i];
+        }
     }
     for (uint32_t t = ns * 4; t < per * 4; ++t) group_barrier();
     wait_counts<vm_wait(0)>();
@@ -633,25 +599,23 @@ __global__ __launch_bounds__(64 * kTileWaves * kTileGroups) void kq_prefill_kern
     constexpr int H = (TM + 1) / 2;
     const int kept = kg == 0 ? H : TM - H, tile0 = kg == 0 ? 0 : H;
     float* red = reinterpret_cast<float*>(lds);
-    auto slot = [&](int wv, int i, int j, int r) { return red + (((wv * H + i) * TN + j) * 4 + r) * 256 + lane * 4; };
-    auto give = [&](const f32x16& v, int i, int j) {
+    auto slot = [&](int wv, int i, int r) { return red + ((wv * H + i) * 4 + r) * 256 + lane * 4; };
+    auto give = [&](const f32x16& v, int i) {
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-            *reinterpret_cast<f32x4*>(slot(wave, i, j, r)) = f32x4{v[4 * r], v[4 * r + 1], v[4 * r + 2], v[4 * r + 3]};
+            *reinterpret_cast<f32x4*>(slot(wave, i, r)) = f32x4{v[4 * r], v[4 * r + 1], v[4 * r + 2], v[4 * r + 3]};
     };
     if (kg == 0) {
 #pragma unroll
         for (int i = 0; i < TM - H; ++i)
-#pragma unroll
-            for (int j = 0; j < TN; ++j) give(acc[H + i][j], i, j);
+            give(acc[H + i], i);
     } else {
 #pragma unroll
-        for (int i = 0; i < H; ++i)
-#pragma unroll
-            for (int j = 0; j < TN; ++j) {
-                give(acc[i][j], i, j);
-                if (H + i < TM) acc[i][j] = acc[H + i][j];
-            }
+        for (int i = 0; i < H; ++i) {
+            give(acc[i], i);
+            if (H + i < TM) acc[i] = acc[H + i];
+        }
+        memory_fence();  // or the compiler merges both groups' writes behind selects
     }
     __syncthreads();
     const int other = wave ^ kTileWaves;
@@ -659,44 +623,39 @@ __global__ __launch_bounds__(64 * kTileWaves * kTileGroups) void kq_prefill_kern
     for (int i = 0; i < H; ++i) {
         if (i >= kept) break;  // uniform
 #pragma unroll
-        for (int j = 0; j < TN; ++j)
+        for (int r = 0; r < 4; ++r) {
+            const f32x4 v = *reinterpret_cast<const f32x4*>(slot(other, i, r));
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const f32x4 v = *reinterpret_cast<const f32x4*>(slot(other, i, j, r));
-#pragma unroll
-                for (int k = 0; k < 4; ++k) acc[i][j][4 * r + k] += v[k];
-            }
+            for (int k = 0; k < 4; ++k) acc[i][4 * r + k] += v[k];
+        }
     }
     // Lane (r, c) holds column r of each tile, rows 8 (k / 4) + 4 c + k % 4.
+    const uint32_t n = n0 + wn * 32 + lr;
+    if (n >= N) return;
+    auto token = [&](uint32_t at) { return m0 + tile0 * 32 + (at / 16) * 32 + 8 * (at / 4 % 4) + 4 * lc + at % 4; };
+    auto store = [&](uint32_t m, float v) {
+        if constexpr (SK)
+            partial[(static_cast<size_t>(part) * M + m) * N + n] = v;
+        else
+            y[static_cast<size_t>(m) * N + n] = to_out<OutT>(v);
+    };
+    uint32_t again = 0;
 #pragma unroll
-    for (int j = 0; j < TN; ++j) {
-        const uint32_t n = n0 + (wn * TN + j) * 32 + lr;
-        if (n >= N) continue;
-        auto token = [&](uint32_t at) { return m0 + tile0 * 32 + (at / 16) * 32 + 8 * (at / 4 % 4) + 4 * lc + at % 4; };
-        auto store = [&](uint32_t m, float v) {
-            if constexpr (SK)
-                partial[(static_cast<size_t>(part) * M + m) * N + n] = v;
-            else
-                y[static_cast<size_t>(m) * N + n] = to_out<OutT>(v);
-        };
-        uint32_t again = 0;
+    for (int i = 0; i < H; ++i) {
+        if (i >= kept) break;
 #pragma unroll
-        for (int i = 0; i < H; ++i) {
-            if (i >= kept) break;
-#pragma unroll
-            for (int k = 0; k < 16; ++k) {
-                const uint32_t m = token(16 * i + k);
-                if (m >= M) continue;
-                store(m, acc[i][j][k]);
-                again |= not_finite(acc[i][j][k]) ? 1u << (16 * i + k) : 0u;
-            }
+        for (int k = 0; k < 16; ++k) {
+            const uint32_t m = token(16 * i + k);
+            if (m >= M) continue;
+            store(m, acc[i][k]);
+            again |= not_finite(acc[i][k]) ? 1u << (16 * i + k) : 0u;
         }
-        for (; again != 0; again &= again - 1) {
-            const uint32_t m = token(__builtin_ctz(again));
-            store(m, kq_not_finite_thread<F>(w + (static_cast<size_t>(n) * nb + pb0) * BB,
-                                             x + static_cast<size_t>(m) * K + static_cast<size_t>(pb0) * kSuper,
-                                             pb1 - pb0));
-        }
+    }
+    for (; again != 0; again &= again - 1) {
+        const uint32_t m = token(__builtin_ctz(again));
+        store(m, kq_not_finite_thread<F>(w + (static_cast<size_t>(n) * nb + pb0) * BB,
+                                         x + static_cast<size_t>(m) * K + static_cast<size_t>(pb0) * kSuper,
+                                         pb1 - pb0));
     }
 }
 

@@ -38,6 +38,7 @@
 // waves (128 x 4096 x 14 336 25.1 against 24.8, 64 x 8192 x 28 672 60.9 against
 // 53.9; gate/up the same), so they keep those.
 #include "common.hpp"
+#include "kquant_blocks.hpp"
 #include "q4_0.hpp"
 #include "tile_ops.hpp"
 
@@ -425,13 +426,7 @@ bool prefill_ring_supports(const Problem& p) {
 // 336 x 5120 118 -> 82; 100 x 13 824 x 5120 49.4 -> 31.7; 65 x 28 672 x 8192 114
 // -> 73; 32 x 11 008 x 4096 39.4 -> 22.8.
 hipError_t launch_prefill_ring_parts(const Problem& p, int bm, int bn) {
-    static const int cus = [] {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-            n = 256;
-        return n;
-    }();
+    const double cus = kquant::device_cus();
     const uint32_t nsuper = p.K / 256u;
     auto cost = [&](int tm, int tn, double each, uint32_t parts) {
         const double tiles = static_cast<double>((p.M + tm - 1u) / tm) * ((p.N + tn - 1u) / tn) * parts;
